@@ -111,10 +111,15 @@ __host__ __device__ constexpr int ns_of(int s, int p)
 }
 
 // Twiddle rows of pass p >= 1 (stride Ns = ns_of(s, p), radix R): row k
-// (k < Ns) holds TW_ROW = 4 entries w^1, w^2, w^3, w^4 of
-// w = exp(-2*pi*i*k/(Ns*R)) (32 bytes, four rows per cache line); the other
-// powers are products of these (expand_twiddles).
+// (k < Ns) holds TW_ROW = 4 entries of w = exp(-2*pi*i*k/(Ns*R)) (32 bytes,
+// four rows per cache line): w, w^2, w^4, w^8 for a power-of-two radix (the
+// stage twiddles of dft_twiddled), w^1, w^2, w^3, w^4 for radix 12 (the other
+// powers are products of these, expand_twiddles).
 constexpr int TW_ROW = 4;
+__host__ __device__ constexpr int tw_exponent(int radix, int e)
+{
+    return (radix & (radix - 1)) == 0 ? (1 << e) : e + 1;
+}
 __host__ __device__ constexpr int64_t tw_pass_len(int s, int p)
 {
     return (p >= 1 && p < npass_of(s) ? int64_t(ns_of(s, p)) : 0) * TW_ROW;
@@ -280,35 +285,149 @@ __host__ __device__ constexpr int bitrev_small(int v, int bits)
     return r;
 }
 
-// one radix-2 DIF stage of span HALF over R points.  ZHI (first stage
-// only): u[R/2 + 1 ..] are known to be zero, so every pair but the first
-// is (a, 0) and becomes (a, twiddle * a) without additions.
-template <int R, int HALF, int BASE, int K, bool ZHI>
-__device__ __forceinline__ void dif_bfly(float2* u)
+// ---------------------------------------------------------------------------
+// Power-of-two radices: decimation in time with the pass's twiddles fused in.
+//
+// A pass multiplies input r by w^r and takes the R-point DFT.  Split even and
+// odd r: stage h (h = 1, 2, 4, .. R/2) combines a and b into a +- t*b with
+// t = w^(R/2h) * exp(-2*pi*i*k/2h), k < h.  The products never stand alone:
+// a + t*b is four fused multiply-adds, a - t*b = 2a - (a + t*b) two more, so a
+// twiddled radix-2 butterfly costs 6 instructions (8 for a product and two
+// sums), and only w^(R/2), .., w^2, w (loaded) and their constant rotations
+// (t at k >= h/2 is -i times the one at k - h/2, a swap of operands) are
+// needed: 8 twiddles for radix 16 instead of 15.  A radix-16 pass issues 208
+// VALU instructions, against 274 for 15 products, 11 derived twiddles and a
+// DIF butterfly; the kernels' VALU work is what bounds the long Bluestein
+// lines.
+// ---------------------------------------------------------------------------
+// a, b <- a + t*b, a - t*b with t rotated by -i when NEGI
+template <bool NEGI>
+__device__ __forceinline__ void bfly_tw(float2& a, float2& b, float2 t)
+{
+    float2 y;
+    if constexpr (NEGI) {
+        // (-i*t)*b = (t.x*b.y + t.y*b.x) - i*(t.x*b.x - t.y*b.y)
+        y.x = __builtin_fmaf(t.y, b.x, __builtin_fmaf(t.x, b.y, a.x));
+        y.y = __builtin_fmaf(t.y, b.y, __builtin_fmaf(-t.x, b.x, a.y));
+    } else {
+        y.x = __builtin_fmaf(-t.y, b.y, __builtin_fmaf(t.x, b.x, a.x));
+        y.y = __builtin_fmaf(t.y, b.x, __builtin_fmaf(t.x, b.y, a.y));
+    }
+    b = make_float2(__builtin_fmaf(2.0f, a.x, -y.x), __builtin_fmaf(2.0f, a.y, -y.y));
+    a = y;
+}
+
+// a, b <- a + t*b, a - t*b with t = exp(-2*pi*i*m/16), m < 8
+template <int m>
+__device__ __forceinline__ void bfly_const(float2& a, float2& b)
+{
+    if constexpr (m == 0) {
+        const float2 t = b;
+        b = csub(a, t);
+        a = cadd(a, t);
+    } else if constexpr (m == 4) {
+        const float2 t = make_float2(b.y, -b.x);
+        b = csub(a, t);
+        a = cadd(a, t);
+    } else if constexpr (m == 2 || m == 6) {
+        const float r = 0.70710678118654752440f;
+        // m = 2: r*(x + y) + i*r*(y - x); m = 6: r*(y - x) - i*r*(x + y)
+        const float p = b.x + b.y, q = b.y - b.x;
+        const float2 t = m == 2 ? make_float2(p, q) : make_float2(q, -p);
+        b = make_float2(__builtin_fmaf(-r, t.x, a.x), __builtin_fmaf(-r, t.y, a.y));
+        a = make_float2(__builtin_fmaf(r, t.x, a.x), __builtin_fmaf(r, t.y, a.y));
+    } else {
+        bfly_tw<false>(a, b, make_float2(kC16[m], -kS16[m]));
+    }
+}
+
+// stage H of the untwiddled DFT over bit-reversed u.  ZHI: inputs R/2 + 1 ..
+// are zero (bit-reversed: every odd slot but the first), so the pairs of stage
+// 1 after the first are copies.
+template <int R, int H, int BASE, int K, bool ZHI>
+__device__ __forceinline__ void dit_bfly(float2* u)
 {
     if constexpr (BASE < R) {
-        if constexpr (K < HALF) {
-            const float2 a = u[BASE + K];
-            if constexpr (ZHI && K > 0) {
-                u[BASE + K + HALF] = twc<K*(16 / (2 * HALF))>(a);
-            } else {
-                const float2 b = u[BASE + K + HALF];
-                u[BASE + K] = cadd(a, b);
-                u[BASE + K + HALF] = twc<K*(16 / (2 * HALF))>(csub(a, b));
-            }
-            dif_bfly<R, HALF, BASE, K + 1, ZHI>(u);
+        if constexpr (K < H) {
+            if constexpr (ZHI && H == 1 && BASE > 0)
+                u[BASE + 1] = u[BASE];
+            else
+                bfly_const<K*(16 / (2 * H))>(u[BASE + K], u[BASE + K + H]);
+            dit_bfly<R, H, BASE, K + 1, ZHI>(u);
         } else {
-            dif_bfly<R, HALF, BASE + 2 * HALF, 0, ZHI>(u);
+            dit_bfly<R, H, BASE + 2 * H, 0, ZHI>(u);
         }
     }
 }
 
-template <int R, int HALF, bool ZHI>
-__device__ __forceinline__ void dif_stages(float2* u)
+template <int R, int H, bool ZHI>
+__device__ __forceinline__ void dit_stages(float2* u)
 {
-    if constexpr (HALF >= 1) {
-        dif_bfly<R, HALF, 0, 0, ZHI>(u);
-        dif_stages<R, HALF / 2, false>(u);
+    if constexpr (H < R) {
+        dit_bfly<R, H, 0, 0, ZHI>(u);
+        dit_stages<R, 2 * H, ZHI>(u);
+    }
+}
+
+// stage H with the pass's twiddles; tw[k] = w^(R/2H) * exp(-2*pi*i*k/2H), k < max(H/2, 1)
+template <int R, int H, int BASE, int K>
+__device__ __forceinline__ void dit_tw_bfly(float2* u, const float2* tw)
+{
+    if constexpr (BASE < R) {
+        if constexpr (K < H) {
+            if constexpr (H > 1 && K >= H / 2)
+                bfly_tw<true>(u[BASE + K], u[BASE + K + H], tw[K - H / 2]);
+            else
+                bfly_tw<false>(u[BASE + K], u[BASE + K + H], tw[K]);
+            dit_tw_bfly<R, H, BASE, K + 1>(u, tw);
+        } else {
+            dit_tw_bfly<R, H, BASE + 2 * H, 0>(u, tw);
+        }
+    }
+}
+
+template <int R>
+__device__ __forceinline__ void bit_reverse(float2* u)
+{
+    constexpr int bits = (R == 2) ? 1 : (R == 4) ? 2 : (R == 8) ? 3 : 4;
+    float2 t[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) t[i] = u[bitrev_small(i, bits)];
+#pragma unroll
+    for (int i = 0; i < R; ++i) u[i] = t[i];
+}
+
+// R-point DFT of u[r] * w^r; q holds the pass's row (w, w^2), (w^4, w^8)
+template <int R>
+__device__ __forceinline__ void dft_twiddled(float2 (&u)[R], const float4* q)
+{
+    static_assert(R == 2 || R == 4 || R == 8 || R == 16, "radix");
+    bit_reverse<R>(u);
+    const float2 w1 = make_float2(q[0].x, q[0].y);
+    if constexpr (R == 2) {
+        dit_tw_bfly<R, 1, 0, 0>(u, &w1);
+    } else {
+        const float2 w2 = make_float2(q[0].z, q[0].w);
+        if constexpr (R == 4) {
+            dit_tw_bfly<R, 1, 0, 0>(u, &w2);
+            dit_tw_bfly<R, 2, 0, 0>(u, &w1);
+        } else {
+            const float2 w4 = make_float2(q[1].x, q[1].y);
+            if constexpr (R == 8) {
+                dit_tw_bfly<R, 1, 0, 0>(u, &w4);
+                dit_tw_bfly<R, 2, 0, 0>(u, &w2);
+                const float2 t4[2] = {w1, twc<2>(w1)};
+                dit_tw_bfly<R, 4, 0, 0>(u, t4);
+            } else {
+                const float2 w8 = make_float2(q[1].z, q[1].w);
+                dit_tw_bfly<R, 1, 0, 0>(u, &w8);
+                dit_tw_bfly<R, 2, 0, 0>(u, &w4);
+                const float2 t4[2] = {w2, twc<2>(w2)};
+                dit_tw_bfly<R, 4, 0, 0>(u, t4);
+                const float2 t8[4] = {w1, twc<1>(w1), twc<2>(w1), twc<3>(w1)};
+                dit_tw_bfly<R, 8, 0, 0>(u, t8);
+            }
+        }
     }
 }
 
@@ -350,13 +469,8 @@ __device__ __forceinline__ void dft_fwd(float2* u)
     } else {
         static_assert(R >= 1 && R <= 16 && (R & (R - 1)) == 0, "radix");
         if constexpr (R > 1) {
-            dif_stages<R, R / 2, ZHI>(u);
-            constexpr int bits = (R == 2) ? 1 : (R == 4) ? 2 : (R == 8) ? 3 : 4;
-            float2 t[R];
-#pragma unroll
-            for (int i = 0; i < R; ++i) t[i] = u[bitrev_small(i, bits)];
-#pragma unroll
-            for (int i = 0; i < R; ++i) u[i] = t[i];
+            bit_reverse<R>(u);
+            dit_stages<R, 1, ZHI>(u);
         }
     }
 }
@@ -450,11 +564,11 @@ __host__ __device__ constexpr bool tw_prefetch()
     return is_f3(S) || S <= 13;
 }
 
-// float4s of a row a radix-R butterfly reads: (w^1, w^2) and (w^3, w^4)
+// float4s of a row a radix-R butterfly reads
 template <int R>
 __host__ __device__ constexpr int tw_quads()
 {
-    return R <= 2 ? 1 : 2;
+    return R <= 4 ? 1 : 2;
 }
 
 template <int S, int THREADS, int P>
@@ -559,14 +673,20 @@ struct FftPass {
                 const float4* row = reinterpret_cast<const float4*>(tw + tw_pass_off(S, P) + int64_t(k) * TW_ROW);
 #pragma unroll
                 for (int r2 = 0; r2 < Q; ++r2) q[r2] = tw_prefetch<S>() ? w[b * Q + r2] : row[r2];
-                float2 wt[R];
-                expand_twiddles<R>(wt, q);
+                if constexpr ((R & (R - 1)) == 0) {
+                    dft_twiddled<R>(u, q);
+                } else {
+                    float2 wt[R];
+                    expand_twiddles<R>(wt, q);
 #pragma unroll
-                for (int r = 1; r < R; ++r) u[r] = cmul(u[r], wt[r]);
+                    for (int r = 1; r < R; ++r) u[r] = cmul(u[r], wt[r]);
+                    dft_fwd<R>(u);
+                }
+            } else {
+                // ZIN: slot b + NB*r holds a zero for r > R/2 (b + NB*(R/2 + 1) >= EPT/2 + 1)
+                dft_fwd<R, ZIN>(u);
             }
-            // ZIN: slot b + NB*r holds a zero for r > R/2 (b + NB*(R/2 + 1) >= EPT/2 + 1)
             static_assert(!ZIN || P == 0, "zero inputs only in the first pass");
-            dft_fwd<R, ZIN>(u);
 #pragma unroll
             for (int r = 0; r < R; ++r) v[b + NB * r] = u[r];
         }

@@ -4,7 +4,7 @@
 //   * dtab[q]    = (1/M) * sum_l h2[l] exp(-2*pi*i*(l*q mod M)/M), the FFT of the
 //                  circulant embedding h2 of conj(chirp)  (function.cpp:75-92,
 //                  dft.cpp:77-111), with the 1/M of the inverse FFT folded in
-//   * twiddles   = per-pass Stockham rows: w^1..w^4 of w = exp(-2*pi*i*k/L), exponents k*e mod L
+//   * twiddles   = per-pass Stockham rows: four powers of w = exp(-2*pi*i*k/L), exponents k*e mod L
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -20,13 +20,13 @@ __device__ __forceinline__ double2 unit_root(int64_t q, int64_t den)
     return make_double2(c, -s);
 }
 
-// row k of a pass: w^1..w^TW_ROW of w = exp(-2*pi*i*k/(ns*radix))
+// row k of a pass: TW_ROW powers (tw_exponent) of w = exp(-2*pi*i*k/(ns*radix))
 __global__ void k_gen_twiddle_block(float2* out, int ns, int radix)
 {
     const int64_t idx = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     const int64_t len = int64_t(ns) * radix;
     if (idx >= int64_t(ns) * TW_ROW) return;
-    const int64_t k = idx / TW_ROW, e = idx % TW_ROW + 1;
+    const int64_t k = idx / TW_ROW, e = tw_exponent(radix, (int)(idx % TW_ROW));
     const double2 w = unit_root((k * e) % len, len);
     out[idx] = make_float2((float)w.x, (float)w.y);
 }
