@@ -25,7 +25,12 @@ COMMON = [
     f"-I{os.path.join(ROOT, 'include')}",
 ]
 
+# a source, or (source, object name, defines) for one compiled several times;
+# the longest compilations first
 SOURCES = [
+    ("kernels/batch_kernels.hip", f"batch_{kind}_{t}", [f"-DMDFT_BATCH_T={t}", f"-DMDFT_BATCH_PERSISTENT_TU={p}"])
+    for p, kind in ((0, "grid"), (1, "persistent")) for t in (256, 512, 1024)
+] + [
     "kernels/axis.hip",
     "kernels/batch.hip",
     "kernels/tables.hip",
@@ -43,10 +48,11 @@ SOURCES = [
 ]
 
 
-def _compile(src):
-    out = os.path.join(BUILD, src.replace("/", "_") + ".o")
+def _compile(entry):
+    src, name, defines = entry if isinstance(entry, tuple) else (entry, entry.replace("/", "_"), [])
+    out = os.path.join(BUILD, name + ".o")
     lang = ["-x", "hip"] if src.endswith(".hip") else ["-x", "hip"]
-    cmd = [HIPCC] + COMMON + lang + ["-c", os.path.join(CSRC, src), "-o", out]
+    cmd = [HIPCC] + COMMON + defines + lang + ["-c", os.path.join(CSRC, src), "-o", out]
     r = subprocess.run(cmd, capture_output=True, text=True)
     msgs = "\n".join(l for l in (r.stdout + r.stderr).splitlines() if "packed-fp32-ops" not in l)
     if r.returncode != 0:

@@ -24,7 +24,7 @@ void arrange_for_xcds(const std::vector<uint2>& items, const std::vector<double>
 
 int batch_threads_for(const uint32_t* widths, const uint32_t* heights, size_t count)
 {
-    const int limit = batch_max_logm(1024);
+    const int limit = batch_max_logm();
     int tpl = 1;
     for (size_t i = 0; i < count; ++i) {
         compute_m(widths[i]);  // validates the sides
@@ -35,7 +35,7 @@ int batch_threads_for(const uint32_t* widths, const uint32_t* heights, size_t co
             throw Error(MDFT_ERR_SIZE, "batch transform " + std::to_string(i) + " (" + std::to_string(widths[i]) + "x" +
                                            std::to_string(heights[i]) + ") exceeds the batch padded-length limit " +
                                            std::to_string(1 << limit));
-        tpl = std::max({tpl, m_of(sr) / ept_of(sr), m_of(sc) / ept_of(sc)});
+        tpl = std::max({tpl, tpl_of(sr), tpl_of(sc)});
     }
     // the smallest tile that holds a whole line of every length
     return tpl <= 256 ? 256 : tpl <= 512 ? 512 : 1024;

@@ -597,7 +597,7 @@ bool Context::wide_tiles(int shape, bool blue, bool cols, int count) const
 {
     if (variant(shape, blue, cols) == 0) return false;
     // wide tiles hold 4x the lines of narrow ones; keep at least one tile per CU
-    const int tpl = m_of(shape) / ept_of(shape);
+    const int tpl = tpl_of(shape);
     const int lines_wide = tpl >= 1024 ? 1 : 1024 / tpl;
     const int64_t tiles = (int64_t(count) + lines_wide - 1) / lines_wide;
     return tiles >= int64_t(cu_count_);
@@ -609,7 +609,7 @@ int Context::tile_threads(int shape, bool blue, bool cols, int count) const
     // passes with few lines: smaller tiles (one wave for lines of up to 1024
     // points) so every CU gets work; rows aim at four tiles per CU, columns at
     // one, since narrower column tiles read shorter runs of each row
-    const int tpl = m_of(shape) / ept_of(shape);
+    const int tpl = tpl_of(shape);
     const int64_t want = int64_t(cols ? 1 : 4) * cu_count_;
     int t = tpl > 256 ? tpl : 256;
     while (t > 64 && t / 2 >= tpl && (int64_t(count) + t / tpl - 1) / (t / tpl) < want) t /= 2;

@@ -38,7 +38,7 @@ float time_launches(hipStream_t s, F&& fn, int reps)
 
 int tile_threads(int shape, bool wide)
 {
-    const int tpl = mdft::m_of(shape) / mdft::ept_of(shape);
+    const int tpl = mdft::tpl_of(shape);
     const int base = wide ? 1024 : 256;
     return tpl > base ? tpl : base;
 }

@@ -16,7 +16,7 @@ namespace mdft {
 // which widens the contiguous run a column tile reads from each row.
 __host__ __device__ constexpr int axis_threads(int shape, bool wide)
 {
-    const int tpl = m_of(shape) / ept_of(shape);
+    const int tpl = tpl_of(shape);
     const int base = wide ? 1024 : 256;
     return tpl > base ? tpl : base;
 }
@@ -62,7 +62,7 @@ static hipError_t launch_axis_tt(const AxisJob& job, bool blue, bool cols, hipSt
 template <int S>
 static hipError_t launch_axis_t(const AxisJob& job, bool blue, bool cols, int threads, hipStream_t stream)
 {
-    constexpr int TPL = m_of(S) / ept_of(S);
+    constexpr int TPL = tpl_of(S);
     constexpr int TN = axis_threads(S, false), TW = axis_threads(S, true);
     if (threads >= 1024 && TW != TN) return launch_axis_tt<S, TW>(job, blue, cols, stream);
     if constexpr (TPL <= 64) {

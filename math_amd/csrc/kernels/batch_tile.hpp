@@ -1,0 +1,175 @@
+// Batched 2-D DFTs of mixed sizes.
+//
+// A batch is a list of work items over a table of axis jobs (one row job
+// and one column job per image).  An item is one tile of one job, or a whole
+// small image: a workgroup runs the row tile, makes its stores visible to its
+// own waves, then runs the column tile, with no cross-workgroup
+// synchronisation at all.  Three launch shapes share the item code:
+//
+//  * k_batch_grid: one workgroup per item, items laid out by the host so
+//    each job runs on one XCD; a batch is two launches, whole images + row
+//    tiles (256-thread tiles), then column tiles (512-thread tiles, 2-8
+//    columns each for padded lengths 1024-4096, so each row of a tile is a
+//    longer contiguous run, with two workgroups per CU).
+//  * k_batch_persistent: a grid sized to the device's residency takes items
+//    from a ticket counter, one launch per phase.
+//  * k_batch_persistent with dependencies: one launch for everything; a
+//    column tile waits on a per-image counter of finished row tiles (a
+//    device-scope release/acquire pair per tile, which costs an L2
+//    write-back per row tile).
+//
+// Every line runs the same per-line arithmetic as the single-image kernels
+// (same radix schedule, explicit fmas), so a result is bitwise the same alone
+// and in any mix.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "fft_device.hpp"
+#include "launch.hpp"
+
+namespace mdft {
+
+template <int S, int T>
+constexpr int lds_need()
+{
+    if constexpr (tpl_of(S) > T) {
+        return 0;
+    } else {
+        constexpr int a = LineCfg<S, T>::template lds_floats<false>();
+        constexpr int b = LineCfg<S, T>::template lds_floats<true>();
+        return a > b ? a : b;
+    }
+}
+
+constexpr int cmax(int a, int b) { return a > b ? a : b; }
+
+template <int T>
+constexpr int batch_lds()
+{
+    return cmax(cmax(cmax(cmax(lds_need<5, T>(), lds_need<6, T>()), cmax(lds_need<7, T>(), lds_need<8, T>())),
+                     cmax(cmax(cmax(lds_need<9, T>(), lds_need<10, T>()), cmax(lds_need<11, T>(), lds_need<12, T>())),
+                          lds_need<13, T>())),
+                cmax(cmax(cmax(lds_need<F3_BASE + 6, T>(), lds_need<F3_BASE + 7, T>()),
+                          cmax(lds_need<F3_BASE + 8, T>(), lds_need<F3_BASE + 9, T>())),
+                     cmax(lds_need<F3_BASE + 10, T>(), lds_need<F3_BASE + 11, T>())));
+}
+
+// One variant.  The thread and tile indices go through an empty asm of its own in every
+// variant: otherwise the index arithmetic the variants share is hoisted above
+// the dispatch and held there in registers that the variants then spill.
+template <int S, int T, bool BLUE, bool COLS>
+__device__ __forceinline__ void run_variant(const AxisJob& job, int tile, float* lds)
+{
+    int tid = threadIdx.x;
+    asm volatile("; tile variant %2" : "+v"(tid), "+s"(tile) : "n"(S * 4 + (BLUE ? 2 : 0) + (COLS ? 1 : 0)));
+    line_tile<S, T, BLUE, COLS>(job, tile, lds, tid);
+}
+
+template <int S, int T>
+__device__ __forceinline__ void run_tile_body(const AxisJob& job, int blue, int cols, int tile, float* lds)
+{
+    if constexpr (tpl_of(S) <= T) {
+        if constexpr (S >= 2) {
+            if (blue) {
+                if (cols)
+                    run_variant<S, T, true, true>(job, tile, lds);
+                else
+                    run_variant<S, T, true, false>(job, tile, lds);
+                return;
+            }
+        }
+        if (cols)
+            run_variant<S, T, false, true>(job, tile, lds);
+        else
+            run_variant<S, T, false, false>(job, tile, lds);
+    }
+}
+
+template <int S, int T>
+__device__ __noinline__ void run_tile_call(const BatchJob* jobs, uint32_t job, int tile, float* lds);
+
+// Grid kernels inline every variant (register allocation per region,
+// occupancy-constrained); the persistent kernels call them out of line, since
+// inlining into the ticket loop keeps too much alive across it.
+template <int S, int T, bool INL>
+__device__ __forceinline__ void run_tile(const BatchJob* jobs, uint32_t job, const BatchJob& bj, int tile, float* lds)
+{
+    if constexpr (INL)
+        run_tile_body<S, T>(bj.job, bj.blue, bj.cols, tile, lds);
+    else
+        run_tile_call<S, T>(jobs, job, tile, lds);
+}
+
+// Arguments of a call arrive in vector registers: the job is read again here,
+// at a uniform address, so its fields are scalars in the tile code.
+template <int S, int T>
+__device__ __noinline__ void run_tile_call(const BatchJob* jobs, uint32_t job, int tile, float* lds)
+{
+    static_assert(sizeof(BatchJob) % 4 == 0, "copied by words");
+    const uint64_t p = reinterpret_cast<uint64_t>(jobs + job);
+    const uint64_t u = (uint64_t(__builtin_amdgcn_readfirstlane(uint32_t(p >> 32))) << 32) |
+                       __builtin_amdgcn_readfirstlane(uint32_t(p));
+    auto words = reinterpret_cast<const __attribute__((address_space(4))) uint32_t*>(u);
+    union Copy {
+        uint32_t w[sizeof(BatchJob) / 4];
+        BatchJob job;
+        __device__ Copy() {}
+    } copy;
+#pragma unroll
+    for (size_t i = 0; i < sizeof(BatchJob) / 4; ++i) copy.w[i] = words[i];
+    const BatchJob& bj = copy.job;
+    run_tile_body<S, T>(bj.job, bj.blue, bj.cols, __builtin_amdgcn_readfirstlane(tile), lds);
+}
+
+template <int T, bool INL>
+__device__ __forceinline__ void run_job_tile(const BatchJob* jobs, uint32_t job, int tile, float* lds)
+{
+    const BatchJob bj = jobs[job];
+    switch (bj.shape) {
+    case 1: run_tile<1, T, INL>(jobs, job, bj, tile, lds); break;
+    case 2: run_tile<2, T, INL>(jobs, job, bj, tile, lds); break;
+    case 3: run_tile<3, T, INL>(jobs, job, bj, tile, lds); break;
+    case 4: run_tile<4, T, INL>(jobs, job, bj, tile, lds); break;
+    case 5: run_tile<5, T, INL>(jobs, job, bj, tile, lds); break;
+    case 6: run_tile<6, T, INL>(jobs, job, bj, tile, lds); break;
+    case 7: run_tile<7, T, INL>(jobs, job, bj, tile, lds); break;
+    case 8: run_tile<8, T, INL>(jobs, job, bj, tile, lds); break;
+    case 9: run_tile<9, T, INL>(jobs, job, bj, tile, lds); break;
+    case 10: run_tile<10, T, INL>(jobs, job, bj, tile, lds); break;
+    case 11: run_tile<11, T, INL>(jobs, job, bj, tile, lds); break;
+    case 12: run_tile<12, T, INL>(jobs, job, bj, tile, lds); break;
+    case 13: run_tile<13, T, INL>(jobs, job, bj, tile, lds); break;
+    case F3_BASE + 6: run_tile<F3_BASE + 6, T, INL>(jobs, job, bj, tile, lds); break;
+    case F3_BASE + 7: run_tile<F3_BASE + 7, T, INL>(jobs, job, bj, tile, lds); break;
+    case F3_BASE + 8: run_tile<F3_BASE + 8, T, INL>(jobs, job, bj, tile, lds); break;
+    case F3_BASE + 9: run_tile<F3_BASE + 9, T, INL>(jobs, job, bj, tile, lds); break;
+    case F3_BASE + 10: run_tile<F3_BASE + 10, T, INL>(jobs, job, bj, tile, lds); break;
+    case F3_BASE + 11: run_tile<F3_BASE + 11, T, INL>(jobs, job, bj, tile, lds); break;
+    default: break;
+    }
+}
+
+// One item; every branch is on a wave-uniform value.
+template <int T, bool INL>
+__device__ __forceinline__ void run_item(const BatchJob* __restrict__ jobs, uint2 item, float* lds)
+{
+    const uint32_t x = __builtin_amdgcn_readfirstlane(item.x);
+    const uint32_t y = __builtin_amdgcn_readfirstlane(item.y);
+    // one copy of the tile code: a whole image takes two turns (rows, columns)
+    const bool whole = (y & BATCH_WHOLE) != 0;
+    uint32_t job = x;
+    int tile = whole ? 0 : (int)y;
+    for (int turn = 0;; ++turn) {
+        run_job_tile<T, INL>(jobs, job, tile, lds);
+        if (!whole || turn == 1) break;
+        // the column tile reads what this workgroup's waves just stored
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __syncthreads();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        job = y & ~BATCH_WHOLE;
+    }
+}
+
+}  // namespace mdft

@@ -64,8 +64,13 @@ __device__ __forceinline__ float2 cscale(float2 a, float s) { return make_float2
 // compile-time line geometry
 // ---------------------------------------------------------------------------
 // A line's FFT has a "shape" S:
-//  * S in [1, MAX_LOGM]: M = 2^S, radix-16 passes (16 points per thread) and
-//    one remainder pass;
+//  * S in [1, 12]: M = 2^S, radix-16 passes (16 points per thread) and one
+//    remainder pass;
+//  * S = 13, 14: 32 points per thread, passes 32 x 16 x 16 and 32 x 32 x 16, and
+//    the LDS exchange one component at a time, so a line takes half the threads
+//    and half the LDS of 16 points per thread (8192 points: 256 threads and
+//    33 KB, 16384: 512 threads and 66 KB), a CU holds twice the lines, and
+//    there is one exchange less than with radix 16;
 //  * S = F3_BASE + k: M = 3 * 2^k (Bluestein convolutions, and lines of
 //    exactly 3 * 2^k points transformed directly), 12 points per
 //    thread: radix-4 passes, one radix-2 pass when k is odd, and a final
@@ -80,16 +85,19 @@ constexpr int F3_MIN_K = 6;   // M = 192: the radix-12 pass follows at least two
 constexpr int F3_MAX_K = 11;  // M = 6144: 512 threads per line
 __host__ __device__ constexpr bool is_f3(int s) { return s >= F3_BASE; }
 __host__ __device__ constexpr int f3_k(int s) { return s - F3_BASE; }
-// bits per pass of the full-radix passes
-__host__ __device__ constexpr int fft_bits(int s) { return is_f3(s) ? 2 : 4; }
+// 8192 and 16384 points: 32 per thread
+__host__ __device__ constexpr bool is_wide(int s) { return s == 13 || s == 14; }
 __host__ __device__ constexpr int m_of(int s) { return is_f3(s) ? (3 << f3_k(s)) : (1 << s); }
+// points per thread
 __host__ __device__ constexpr int ept_of(int s)
 {
-    return is_f3(s) ? 12 : s < fft_bits(s) ? (1 << s) : (1 << fft_bits(s));
+    return is_f3(s) ? 12 : is_wide(s) ? 32 : s < 4 ? (1 << s) : 16;
 }
+// threads per line
+__host__ __device__ constexpr int tpl_of(int s) { return m_of(s) / ept_of(s); }
 __host__ __device__ constexpr int npass_of(int s)
 {
-    return is_f3(s) ? (f3_k(s) - 2) / 2 + (f3_k(s) - 2) % 2 + 1 : (s + fft_bits(s) - 1) / fft_bits(s);
+    return is_f3(s) ? (f3_k(s) - 2) / 2 + (f3_k(s) - 2) % 2 + 1 : is_wide(s) ? 3 : (s + 3) / 4;
 }
 // radix of pass p (1 when p is past the last pass)
 __host__ __device__ constexpr int radix_of(int s, int p)
@@ -99,8 +107,8 @@ __host__ __device__ constexpr int radix_of(int s, int p)
         const int a = f3_k(s) - 2;
         return p < a / 2 ? 4 : (p == npass_of(s) - 1 ? 12 : 2);
     }
-    const int b = fft_bits(s);
-    return 1 << ((s - b * p) >= b ? b : (s - b * p));
+    if (is_wide(s)) return p == 0 || (s == 14 && p == 1) ? 32 : 16;
+    return 1 << ((s - 4 * p) >= 4 ? 4 : (s - 4 * p));
 }
 // Stockham stride before pass p: the product of the earlier radices
 __host__ __device__ constexpr int ns_of(int s, int p)
@@ -111,18 +119,19 @@ __host__ __device__ constexpr int ns_of(int s, int p)
 }
 
 // Twiddle rows of pass p >= 1 (stride Ns = ns_of(s, p), radix R): row k
-// (k < Ns) holds TW_ROW = 4 entries of w = exp(-2*pi*i*k/(Ns*R)) (32 bytes,
-// four rows per cache line): w, w^2, w^4, w^8 for a power-of-two radix (the
-// stage twiddles of dft_twiddled), w^1, w^2, w^3, w^4 for radix 12 (the other
-// powers are products of these, expand_twiddles).
-constexpr int TW_ROW = 4;
+// (k < Ns) holds 4 entries of w = exp(-2*pi*i*k/(Ns*R)) (32 bytes, four rows
+// per cache line): w, w^2, w^4, w^8 for a power-of-two radix (the stage
+// twiddles of dft_twiddled), w^1, w^2, w^3, w^4 for radix 12 (the other powers
+// are products of these, expand_twiddles).  Radix 32 also needs w^16: rows of
+// 6 entries, the last unused.
+__host__ __device__ constexpr int tw_row(int radix) { return radix == 32 ? 6 : 4; }
 __host__ __device__ constexpr int tw_exponent(int radix, int e)
 {
     return (radix & (radix - 1)) == 0 ? (1 << e) : e + 1;
 }
 __host__ __device__ constexpr int64_t tw_pass_len(int s, int p)
 {
-    return (p >= 1 && p < npass_of(s) ? int64_t(ns_of(s, p)) : 0) * TW_ROW;
+    return p >= 1 && p < npass_of(s) ? int64_t(ns_of(s, p)) * tw_row(radix_of(s, p)) : 0;
 }
 __host__ __device__ constexpr int64_t tw_pass_off(int s, int p)
 {
@@ -180,9 +189,11 @@ template <int S, int THREADS>
 struct LineCfg {
     static constexpr int M = m_of(S);
     static constexpr int EPT = ept_of(S);
-    static constexpr int TPL = M / EPT;          // threads per line
+    static constexpr int TPL = tpl_of(S);        // threads per line
     static constexpr int LPW = THREADS / TPL;    // lines per tile
     static constexpr int NPASS = npass_of(S);
+    // exchange the real parts, then the imaginary parts, through one plane
+    static constexpr bool SPLIT = EPT > 16;
     static_assert(TPL <= THREADS, "line does not fit the workgroup");
     static_assert(LPW * TPL == THREADS, "workgroup must hold whole lines");
     // words of one line's slice: the largest padded position over the exchanges
@@ -214,63 +225,43 @@ struct LineCfg {
     template <bool COLS>
     static constexpr int lds_floats()
     {
-        return NPASS > 1 ? 2 * LPW * lstride<COLS>() : 0;
+        return NPASS > 1 ? (SPLIT ? 1 : 2) * LPW * lstride<COLS>() : 0;
     }
 };
 
 // ---------------------------------------------------------------------------
-// radix-R forward DFT in registers (R <= 16), natural order in and out
+// radix-R forward DFT in registers (R <= 32), natural order in and out
 // ---------------------------------------------------------------------------
-// cos(2*pi*m/16), sin(2*pi*m/16)
-__device__ constexpr float kC16[16] = {1.0f,
-                                       0.92387953251128675613f,
-                                       0.70710678118654752440f,
-                                       0.38268343236508977173f,
-                                       0.0f,
-                                       -0.38268343236508977173f,
-                                       -0.70710678118654752440f,
-                                       -0.92387953251128675613f,
-                                       -1.0f,
-                                       -0.92387953251128675613f,
-                                       -0.70710678118654752440f,
-                                       -0.38268343236508977173f,
-                                       0.0f,
-                                       0.38268343236508977173f,
-                                       0.70710678118654752440f,
-                                       0.92387953251128675613f};
-__device__ constexpr float kS16[16] = {0.0f,
-                                       0.38268343236508977173f,
-                                       0.70710678118654752440f,
-                                       0.92387953251128675613f,
-                                       1.0f,
-                                       0.92387953251128675613f,
-                                       0.70710678118654752440f,
-                                       0.38268343236508977173f,
-                                       0.0f,
-                                       -0.38268343236508977173f,
-                                       -0.70710678118654752440f,
-                                       -0.92387953251128675613f,
-                                       -1.0f,
-                                       -0.92387953251128675613f,
-                                       -0.70710678118654752440f,
-                                       -0.38268343236508977173f};
+// cos(2*pi*m/32), sin(2*pi*m/32), m < 16
+__device__ constexpr float kC32[16] = {
+    1.0f, 0.98078528040323043f, 0.92387953251128674f, 0.83146961230254524f,
+    0.70710678118654757f, 0.55557023301960229f, 0.38268343236508984f, 0.19509032201612833f,
+    0.0f, -0.19509032201612819f, -0.38268343236508973f, -0.55557023301960196f,
+    -0.70710678118654746f, -0.83146961230254535f, -0.92387953251128674f, -0.98078528040323043f
+};
+__device__ constexpr float kS32[16] = {
+    0.0f, 0.19509032201612825f, 0.38268343236508978f, 0.55557023301960218f,
+    0.70710678118654746f, 0.83146961230254524f, 0.92387953251128674f, 0.98078528040323043f,
+    1.0f, 0.98078528040323043f, 0.92387953251128674f, 0.83146961230254546f,
+    0.70710678118654757f, 0.55557023301960218f, 0.38268343236508989f, 0.19509032201612861f
+};
 
-// d * exp(-2*pi*i*m/16) for a compile-time m
+// d * exp(-2*pi*i*m/32) for a compile-time m < 16
 template <int m>
 __device__ __forceinline__ float2 twc(float2 d)
 {
     if constexpr (m == 0) {
         return d;
-    } else if constexpr (m == 4) {
+    } else if constexpr (m == 8) {
         return make_float2(d.y, -d.x);
-    } else if constexpr (m == 2) {
+    } else if constexpr (m == 4) {
         const float r = 0.70710678118654752440f;
         return make_float2(r * (d.x + d.y), r * (d.y - d.x));
-    } else if constexpr (m == 6) {
+    } else if constexpr (m == 12) {
         const float r = 0.70710678118654752440f;
         return make_float2(r * (d.y - d.x), -r * (d.x + d.y));
     } else {
-        const float c = kC16[m], s = kS16[m];
+        const float c = kC32[m], s = kS32[m];
         return make_float2(__builtin_fmaf(d.x, c, d.y * s), __builtin_fmaf(d.y, c, -(d.x * s)));
     }
 }
@@ -317,7 +308,7 @@ __device__ __forceinline__ void bfly_tw(float2& a, float2& b, float2 t)
     a = y;
 }
 
-// a, b <- a + t*b, a - t*b with t = exp(-2*pi*i*m/16), m < 8
+// a, b <- a + t*b, a - t*b with t = exp(-2*pi*i*m/32), m < 16
 template <int m>
 __device__ __forceinline__ void bfly_const(float2& a, float2& b)
 {
@@ -325,19 +316,19 @@ __device__ __forceinline__ void bfly_const(float2& a, float2& b)
         const float2 t = b;
         b = csub(a, t);
         a = cadd(a, t);
-    } else if constexpr (m == 4) {
+    } else if constexpr (m == 8) {
         const float2 t = make_float2(b.y, -b.x);
         b = csub(a, t);
         a = cadd(a, t);
-    } else if constexpr (m == 2 || m == 6) {
+    } else if constexpr (m == 4 || m == 12) {
         const float r = 0.70710678118654752440f;
-        // m = 2: r*(x + y) + i*r*(y - x); m = 6: r*(y - x) - i*r*(x + y)
+        // m = 4: r*(x + y) + i*r*(y - x); m = 12: r*(y - x) - i*r*(x + y)
         const float p = b.x + b.y, q = b.y - b.x;
-        const float2 t = m == 2 ? make_float2(p, q) : make_float2(q, -p);
+        const float2 t = m == 4 ? make_float2(p, q) : make_float2(q, -p);
         b = make_float2(__builtin_fmaf(-r, t.x, a.x), __builtin_fmaf(-r, t.y, a.y));
         a = make_float2(__builtin_fmaf(r, t.x, a.x), __builtin_fmaf(r, t.y, a.y));
     } else {
-        bfly_tw<false>(a, b, make_float2(kC16[m], -kS16[m]));
+        bfly_tw<false>(a, b, make_float2(kC32[m], -kS32[m]));
     }
 }
 
@@ -352,7 +343,7 @@ __device__ __forceinline__ void dit_bfly(float2* u)
             if constexpr (ZHI && H == 1 && BASE > 0)
                 u[BASE + 1] = u[BASE];
             else
-                bfly_const<K*(16 / (2 * H))>(u[BASE + K], u[BASE + K + H]);
+                bfly_const<K*(32 / (2 * H))>(u[BASE + K], u[BASE + K + H]);
             dit_bfly<R, H, BASE, K + 1, ZHI>(u);
         } else {
             dit_bfly<R, H, BASE + 2 * H, 0, ZHI>(u);
@@ -389,7 +380,7 @@ __device__ __forceinline__ void dit_tw_bfly(float2* u, const float2* tw)
 template <int R>
 __device__ __forceinline__ void bit_reverse(float2* u)
 {
-    constexpr int bits = (R == 2) ? 1 : (R == 4) ? 2 : (R == 8) ? 3 : 4;
+    constexpr int bits = (R == 2) ? 1 : (R == 4) ? 2 : (R == 8) ? 3 : (R == 16) ? 4 : 5;
     float2 t[R];
 #pragma unroll
     for (int i = 0; i < R; ++i) t[i] = u[bitrev_small(i, bits)];
@@ -397,11 +388,11 @@ __device__ __forceinline__ void bit_reverse(float2* u)
     for (int i = 0; i < R; ++i) u[i] = t[i];
 }
 
-// R-point DFT of u[r] * w^r; q holds the pass's row (w, w^2), (w^4, w^8)
+// R-point DFT of u[r] * w^r; q holds the pass's row (w, w^2), (w^4, w^8), (w^16, -)
 template <int R>
 __device__ __forceinline__ void dft_twiddled(float2 (&u)[R], const float4* q)
 {
-    static_assert(R == 2 || R == 4 || R == 8 || R == 16, "radix");
+    static_assert(R == 2 || R == 4 || R == 8 || R == 16 || R == 32, "radix");
     bit_reverse<R>(u);
     const float2 w1 = make_float2(q[0].x, q[0].y);
     if constexpr (R == 2) {
@@ -416,16 +407,29 @@ __device__ __forceinline__ void dft_twiddled(float2 (&u)[R], const float4* q)
             if constexpr (R == 8) {
                 dit_tw_bfly<R, 1, 0, 0>(u, &w4);
                 dit_tw_bfly<R, 2, 0, 0>(u, &w2);
-                const float2 t4[2] = {w1, twc<2>(w1)};
+                const float2 t4[2] = {w1, twc<4>(w1)};
                 dit_tw_bfly<R, 4, 0, 0>(u, t4);
             } else {
                 const float2 w8 = make_float2(q[1].z, q[1].w);
-                dit_tw_bfly<R, 1, 0, 0>(u, &w8);
-                dit_tw_bfly<R, 2, 0, 0>(u, &w4);
-                const float2 t4[2] = {w2, twc<2>(w2)};
-                dit_tw_bfly<R, 4, 0, 0>(u, t4);
-                const float2 t8[4] = {w1, twc<1>(w1), twc<2>(w1), twc<3>(w1)};
-                dit_tw_bfly<R, 8, 0, 0>(u, t8);
+                if constexpr (R == 16) {
+                    dit_tw_bfly<R, 1, 0, 0>(u, &w8);
+                    dit_tw_bfly<R, 2, 0, 0>(u, &w4);
+                    const float2 t4[2] = {w2, twc<4>(w2)};
+                    dit_tw_bfly<R, 4, 0, 0>(u, t4);
+                    const float2 t8[4] = {w1, twc<2>(w1), twc<4>(w1), twc<6>(w1)};
+                    dit_tw_bfly<R, 8, 0, 0>(u, t8);
+                } else {
+                    const float2 w16 = make_float2(q[2].x, q[2].y);
+                    dit_tw_bfly<R, 1, 0, 0>(u, &w16);
+                    dit_tw_bfly<R, 2, 0, 0>(u, &w8);
+                    const float2 t4[2] = {w4, twc<4>(w4)};
+                    dit_tw_bfly<R, 4, 0, 0>(u, t4);
+                    const float2 t8[4] = {w2, twc<2>(w2), twc<4>(w2), twc<6>(w2)};
+                    dit_tw_bfly<R, 8, 0, 0>(u, t8);
+                    const float2 t16[8] = {w1,          twc<1>(w1), twc<2>(w1), twc<3>(w1),
+                                           twc<4>(w1), twc<5>(w1), twc<6>(w1), twc<7>(w1)};
+                    dit_tw_bfly<R, 16, 0, 0>(u, t16);
+                }
             }
         }
     }
@@ -467,7 +471,7 @@ __device__ __forceinline__ void dft_fwd(float2* u)
             u[(8 + 9 * k2) % 12] = a2[k2];
         }
     } else {
-        static_assert(R >= 1 && R <= 16 && (R & (R - 1)) == 0, "radix");
+        static_assert(R >= 1 && R <= 32 && (R & (R - 1)) == 0, "radix");
         if constexpr (R > 1) {
             bit_reverse<R>(u);
             dit_stages<R, 1, ZHI>(u);
@@ -534,6 +538,52 @@ __device__ __forceinline__ float cabs_scaled(float2 y, float s)
     return __builtin_sqrtf(__builtin_fmaf(y.x, y.x, y.y * y.y)) * s;
 }
 
+// Global accesses.  The pointers of a batch job come from memory, where the
+// compiler cannot tell global from LDS addresses and would use flat
+// instructions, whose loads and stores also count as LDS traffic and are
+// waited for at every exchange: the address space is stated.
+typedef float vec2 __attribute__((ext_vector_type(2)));
+typedef float vec4 __attribute__((ext_vector_type(4)));
+#define MDFT_GLOBAL __attribute__((address_space(1)))
+__device__ __forceinline__ float2 load_global(const float2* p)
+{
+    const vec2 x = *(const MDFT_GLOBAL vec2*)p;
+    return make_float2(x.x, x.y);
+}
+__device__ __forceinline__ void store_global(float2* p, float2 x) { *(MDFT_GLOBAL vec2*)p = vec2{x.x, x.y}; }
+// At a uniform address (p must not depend on the lane) plus a 32-bit element
+// index: the address is kept in scalar registers, so every slot's access takes
+// its offset from one vector register; left to itself the compiler adds each
+// slot's offset to a 64-bit vector address, two or three VALU instructions and
+// two registers a slot.
+__device__ __forceinline__ float2 load_at(const float2* p, uint32_t i)
+{
+    auto g = (const MDFT_GLOBAL char*)p;
+    asm("" : "+s"(g));
+    const vec2 x = *(const MDFT_GLOBAL vec2*)(g + i * 8u);
+    return make_float2(x.x, x.y);
+}
+__device__ __forceinline__ float4 load4_at(const float2* p, uint32_t bytes)
+{
+    auto g = (const MDFT_GLOBAL char*)p;
+    asm("" : "+s"(g));
+    const vec4 x = *(const MDFT_GLOBAL vec4*)(g + bytes);
+    return make_float4(x.x, x.y, x.z, x.w);
+}
+__device__ __forceinline__ void store_at(float2* p, uint32_t i, float2 x)
+{
+    auto g = (MDFT_GLOBAL char*)p;
+    asm("" : "+s"(g));
+    *(MDFT_GLOBAL vec2*)(g + i * 8u) = vec2{x.x, x.y};
+}
+// a value the compiler knows nothing about
+template <class V>
+__device__ __forceinline__ V opaque(V x)
+{
+    asm("" : "+v"(x));
+    return x;
+}
+
 // ---------------------------------------------------------------------------
 // FFT of the tile held in registers
 // ---------------------------------------------------------------------------
@@ -556,19 +606,12 @@ __device__ __forceinline__ void exchange_sync()
 
 // Twiddle rows of pass P for the thread's butterflies are loaded one pass
 // ahead (pass 1's with the tile's input), so the table latency overlaps the
-// LDS exchange instead of following it.  Off for 16384 points, where the
-// extra registers spill.
-template <int S>
-__host__ __device__ constexpr bool tw_prefetch()
-{
-    return is_f3(S) || S <= 13;
-}
-
+// LDS exchange instead of following it.
 // float4s of a row a radix-R butterfly reads
 template <int R>
 __host__ __device__ constexpr int tw_quads()
 {
-    return R <= 4 ? 1 : 2;
+    return R <= 4 ? 1 : R <= 16 ? 2 : 3;
 }
 
 template <int S, int THREADS, int P>
@@ -584,9 +627,10 @@ struct TwLoad {
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
             const int k = (t + b * C::TPL) & (NS - 1);
-            const float4* row = reinterpret_cast<const float4*>(tw + tw_pass_off(S, P) + int64_t(k) * TW_ROW);
+            // the second float4 of a row is an immediate offset away
 #pragma unroll
-            for (int r2 = 0; r2 < Q; ++r2) w[b * Q + r2] = row[r2];
+            for (int r2 = 0; r2 < Q; ++r2)
+                w[b * Q + r2] = load4_at(tw + tw_pass_off(S, P), uint32_t(k) * uint32_t(8 * tw_row(R)) + 16u * r2);
         }
     }
 };
@@ -625,7 +669,7 @@ __device__ __forceinline__ void expand_twiddles(float2 (&wt)[R], const float4* q
 // loaded into pf one pass before the last, so their latency overlaps the
 // last exchange and butterflies; slots PF .. PFL-1 at the start of the last
 // pass, after its exchange (with one pass, all PFL at its start).
-template <int S, int THREADS, bool COLS, int P, bool ZIN = false, int PF = 0, int PFL = 0>
+template <int S, int THREADS, bool COLS, int P, bool ZIN = false, int PF = 0, int PFL = 0, int EL = 0>
 struct FftPass {
     using C = LineCfg<S, THREADS>;
     static constexpr bool WAVE = !COLS && C::TPL <= 64;
@@ -636,43 +680,90 @@ struct FftPass {
     static constexpr int LST = C::template lstride<COLS>();
     static_assert(NB * R == C::EPT, "the radix divides the points per thread");
 
-    __device__ __forceinline__ static void run(float2 (&v)[C::EPT], int t, float* re, float* im, const float2* tw,
-                                               float4 (&w)[C::EPT / 2], const float2* pfs, float2 (&pf)[C::EPT])
+    // Stockham positions of this pass's outputs, component c
+    template <int c>
+    __device__ __forceinline__ static void scatter(const float2 (&v)[C::EPT], int t, float* plane)
     {
-        static_assert(PF <= C::EPT && PFL <= C::EPT, "prefetch slots");
-        if constexpr (PF > 0 && C::NPASS == 1) {
-#pragma unroll
-            for (int i = 0; i < (PFL > PF ? PFL : PF); ++i) pf[i] = pfs[t + i * C::TPL];
-        }
-        if constexpr (P > 0) {
-            exchange_sync<WAVE>();
-            // layout written by the previous pass; the offset of slot i is a
-            // compile-time constant (an LDS immediate)
-            const int q0 = lds_pos<S, THREADS, COLS, P - 1>(t);
-#pragma unroll
-            for (int i = 0; i < C::EPT; ++i) {
-                const int q = q0 + lds_pos<S, THREADS, COLS, P - 1>(i * C::TPL);
-                v[i] = make_float2(re[q], im[q]);
-            }
-            if constexpr (LAST && PFL > PF) {
-#pragma unroll
-                for (int i = PF; i < PFL; ++i) pf[i] = pfs[t + i * C::TPL];
-            }
-        }
-        // butterfly b reads and writes only the slots b + NB*r: update in place
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
             const int j = t + b * C::TPL;
             const int k = j & (NS - 1);
+            const int base = (j - k) * R + k;
+            // the layout keeps the R outputs' offsets linear: each step adds f(NS)
+            constexpr int step = lds_pos<S, THREADS, COLS, P>(NS);
+            const int q0 = lds_pos<S, THREADS, COLS, P>(base);
+#pragma unroll
+            for (int r = 0; r < R; ++r) plane[q0 + r * step] = c == 0 ? v[b + NB * r].x : v[b + NB * r].y;
+        }
+    }
+
+    // the next pass's operands: the thread's fixed positions t + i*TPL (the
+    // offset of slot i is a compile-time constant, an LDS immediate)
+    template <int c>
+    __device__ __forceinline__ static void gather(float2 (&v)[C::EPT], int t, const float* plane)
+    {
+        const int q0 = lds_pos<S, THREADS, COLS, P>(t);
+#pragma unroll
+        for (int i = 0; i < C::EPT; ++i) {
+            const float x = plane[q0 + lds_pos<S, THREADS, COLS, P>(i * C::TPL)];
+            if constexpr (c == 0)
+                v[i].x = x;
+            else
+                v[i].y = x;
+        }
+    }
+
+    __device__ __forceinline__ static void exchange(float2 (&v)[C::EPT], int t, float* re, float* im)
+    {
+        exchange_sync<WAVE>();  // the previous exchange's reads are done
+        if constexpr (C::SPLIT) {
+            scatter<0>(v, t, re);
+            exchange_sync<WAVE>();
+            gather<0>(v, t, re);
+            exchange_sync<WAVE>();
+            scatter<1>(v, t, re);
+            exchange_sync<WAVE>();
+            gather<1>(v, t, re);
+        } else {
+            scatter<0>(v, t, re);
+            scatter<1>(v, t, im);
+            exchange_sync<WAVE>();
+            gather<0>(v, t, re);
+            gather<1>(v, t, im);
+        }
+    }
+
+    template <class Epi>
+    __device__ __forceinline__ static void run(float2 (&v)[C::EPT], int t, float* re, float* im, const float2* tw,
+                                               float4 (&w)[C::EPT / 2], const float2* pfs, float2 (&pf)[C::EPT],
+                                               const Epi& epi)
+    {
+        static_assert(PF <= C::EPT && PFL <= C::EPT, "prefetch slots");
+        if constexpr (PF > 0 && C::NPASS == 1) {
+#pragma unroll
+            for (int i = 0; i < (PFL > PF ? PFL : PF); ++i) pf[i] = load_at(pfs + i * C::TPL, uint32_t(t));
+        }
+        if constexpr (LAST && P > 0 && PFL > PF) {
+#pragma unroll
+            for (int i = PF; i < PFL; ++i) pf[i] = load_at(pfs + i * C::TPL, uint32_t(t));
+        }
+        // butterfly b reads and writes only the slots b + NB*r: update in place
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
             float2 u[R];
+            float2 tab[R];
+            if constexpr (LAST && C::SPLIT && EL > 0) {
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    if (b + NB * r < EL) tab[r] = load_at(pfs + (b + NB * r) * C::TPL, uint32_t(t));
+            }
 #pragma unroll
             for (int r = 0; r < R; ++r) u[r] = v[b + NB * r];
             if constexpr (P > 0) {
                 constexpr int Q = tw_quads<R>();
-                float4 q[2];
-                const float4* row = reinterpret_cast<const float4*>(tw + tw_pass_off(S, P) + int64_t(k) * TW_ROW);
+                float4 q[Q];
 #pragma unroll
-                for (int r2 = 0; r2 < Q; ++r2) q[r2] = tw_prefetch<S>() ? w[b * Q + r2] : row[r2];
+                for (int r2 = 0; r2 < Q; ++r2) q[r2] = w[b * Q + r2];
                 if constexpr ((R & (R - 1)) == 0) {
                     dft_twiddled<R>(u, q);
                 } else {
@@ -689,30 +780,22 @@ struct FftPass {
             static_assert(!ZIN || P == 0, "zero inputs only in the first pass");
 #pragma unroll
             for (int r = 0; r < R; ++r) v[b + NB * r] = u[r];
+            if constexpr (LAST && C::SPLIT) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) epi(b + NB * r, v[b + NB * r], tab[r]);
+            }
+            // one butterfly's operands at a time: without it the scheduler
+            // starts the next one's loads early and spills
+            if constexpr (C::SPLIT && NB > 1) __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (!LAST) {
-            if constexpr (tw_prefetch<S>()) TwLoad<S, THREADS, P + 1>::run(w, t, tw);
+            TwLoad<S, THREADS, P + 1>::run(w, t, tw);
             if constexpr (PF > 0 && P + 2 == C::NPASS) {
 #pragma unroll
-                for (int i = 0; i < PF; ++i) pf[i] = pfs[t + i * C::TPL];
+                for (int i = 0; i < PF; ++i) pf[i] = load_at(pfs + i * C::TPL, uint32_t(t));
             }
-            exchange_sync<WAVE>();
-#pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                const int j = t + b * C::TPL;
-                const int k = j & (NS - 1);
-                const int base = (j - k) * R + k;
-                // the layout keeps the R outputs' offsets linear: each step adds f(NS)
-                constexpr int step = lds_pos<S, THREADS, COLS, P>(NS);
-                const int q0 = lds_pos<S, THREADS, COLS, P>(base);
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const int q = q0 + r * step;
-                    re[q] = v[b + NB * r].x;
-                    im[q] = v[b + NB * r].y;
-                }
-            }
-            FftPass<S, THREADS, COLS, P + 1, false, PF, PFL>::run(v, t, re, im, tw, w, pfs, pf);
+            exchange(v, t, re, im);
+            FftPass<S, THREADS, COLS, P + 1, false, PF, PFL, EL>::run(v, t, re, im, tw, w, pfs, pf, epi);
         }
     }
 };
@@ -722,6 +805,14 @@ struct FftPass {
 // constant zero).  PF > 0: pf[i] = pfs[t + i*TPL] for i < max(PF, PFL) on
 // return, loaded during the FFT (pfs must be readable at every such
 // position).
+//
+// Shapes with the split exchange have no registers for that: run_epi calls
+// epi(i, v[i], pfs[t + i*TPL]) for every slot as the last pass finishes it,
+// with the table entries of one butterfly loaded before its arithmetic (the
+// entries of slots EL .. are not loaded).
+struct NoEpilogue {
+    __device__ __forceinline__ void operator()(int, float2&, float2) const {}
+};
 template <int S, int THREADS, bool COLS, bool ZIN = false, int PF = 0, int PFL = 0>
 struct FftTile {
     using C = LineCfg<S, THREADS>;
@@ -729,17 +820,33 @@ struct FftTile {
     {
         static_assert(PF == 0 && PFL == 0, "prefetch needs a destination");
         float2 pf[C::EPT];
-        run(v, t, ll, lds, tw, nullptr, pf);
+        run_all<0>(v, t, ll, lds, tw, nullptr, pf, NoEpilogue{});
     }
     __device__ __forceinline__ static void run(float2 (&v)[C::EPT], int t, int ll, float* lds, const float2* tw,
                                                const float2* pfs, float2 (&pf)[C::EPT])
     {
+        run_all<0>(v, t, ll, lds, tw, pfs, pf, NoEpilogue{});
+    }
+    template <int EL, class Epi>
+    __device__ __forceinline__ static void run_epi(float2 (&v)[C::EPT], int t, int ll, float* lds, const float2* tw,
+                                                   const float2* pfs, const Epi& epi)
+    {
+        static_assert(C::SPLIT && PF == 0 && PFL == 0, "split exchange only");
+        float2 pf[C::EPT];
+        run_all<EL>(v, t, ll, lds, tw, pfs, pf, epi);
+    }
+
+private:
+    template <int EL, class Epi>
+    __device__ __forceinline__ static void run_all(float2 (&v)[C::EPT], int t, int ll, float* lds, const float2* tw,
+                                                   const float2* pfs, float2 (&pf)[C::EPT], const Epi& epi)
+    {
         constexpr int LST = C::template lstride<COLS>();
         float* re = lds + ll * LST;
-        float* im = lds + C::LPW * LST + ll * LST;
+        float* im = C::SPLIT ? re : re + C::LPW * LST;
         float4 w[C::EPT / 2];
-        if constexpr (tw_prefetch<S>() && C::NPASS > 1) TwLoad<S, THREADS, 1>::run(w, t, tw);
-        FftPass<S, THREADS, COLS, 0, ZIN, PF, PFL>::run(v, t, re, im, tw, w, pfs, pf);
+        if constexpr (!C::SPLIT && C::NPASS > 1) TwLoad<S, THREADS, 1>::run(w, t, tw);
+        FftPass<S, THREADS, COLS, 0, ZIN, PF, PFL, EL>::run(v, t, re, im, tw, w, pfs, pf, epi);
     }
 };
 
@@ -758,10 +865,16 @@ __device__ __forceinline__ void line_tile(const AxisJob& job, int tile, float* l
     const int line = tile * C::LPW + ll;
     const bool valid = line < job.count;
     const int n = job.n;
-    // rows are contiguous (stride 1, known at compile time); a column steps by
-    // the image width.  Consecutive slots of a thread are TPL elements apart.
-    const int64_t es = COLS ? job.es : 1;
-    const int64_t step = int64_t(C::TPL) * es;
+    // Consecutive slots of a thread are TPL elements apart.  A column steps by
+    // the image width: 64-bit addresses.  Rows are contiguous, and like the
+    // tables they are addressed as a uniform base (of the tile's first line and
+    // the slot) plus a 32-bit offset: a tile's rows span less than 2^25
+    // elements, and one register serves every slot.
+    const int64_t step = COLS ? int64_t(C::TPL) * job.es : int64_t(C::TPL);
+    // (a line past the last one reads the tile's first line and stores nothing)
+    const int64_t base = COLS ? int64_t(valid ? line : tile * C::LPW) * job.ls + int64_t(t) * job.es
+                              : int64_t(tile) * C::LPW * job.ls;
+    const uint32_t off = COLS ? 0u : valid ? uint32_t(ll) * uint32_t(job.ls) + uint32_t(t) : uint32_t(t);
     // direction enters as a sign mask: conjugation is one xor, and the
     // inverse's 1/n is a multiply by job.scale (exactly 1 for the forward)
     const uint32_t sgn = job.inverse ? 0x80000000u : 0u;
@@ -775,66 +888,104 @@ __device__ __forceinline__ void line_tile(const AxisJob& job, int tile, float* l
     // the first FFT skips the zero half in the butterflies of its first pass
     constexpr bool ZIN = BLUE;
 
+    // Every load is issued before the first wait: no load sits under a branch,
+    // where the compiler waits for it before it goes on (nine latencies in a
+    // row per Bluestein tile).  A slot past the end of its line reads the
+    // thread's first slot and becomes zero afterwards; the chirp is readable at
+    // every live slot (dir_tables_len).  The line fills more than a quarter (a
+    // third for 3 * 2^k) of the FFT, so the first slots need no check.
+    constexpr int SURE = BLUE ? (is_f3(S) ? C::EPT / 3 : C::EPT / 4) : C::EPT;
     float2 v[C::EPT];
     {
-        const float2* s = job.src + int64_t(valid ? line : 0) * job.ls + int64_t(t) * es;
-#pragma unroll
-        for (int i = 0; i < C::EPT; ++i) {
-            const uint32_t pos = uint32_t(t + i * C::TPL);
-            float2 x = make_float2(0.0f, 0.0f);
-            if (i < LIVE && valid && in_line((int)pos)) {
-                if constexpr ((IO & IO_LUM) != 0)
-                    x = make_float2(image_luminance(io, int64_t(line) * io.ils + int64_t(pos) * io.iel), 0.0f);
-                else
-                    x = s[i * step];
-                // forward x*c, inverse x*conj(c) (direction tables); direct lines: conj for the inverse
-                x = BLUE ? cmul(x, job.chirp[pos]) : cxor(x, sgn);
-            }
-            v[i] = x;
-        }
-    }
-
-    // Bluestein: D arrives during the first FFT, its first half one pass
-    // before the end and the rest at the start of the last pass (up to 4096
-    // points; earlier loads of all of D, or D of 8192 points, spill at the
-    // 128-VGPR cap), and the live slots of the output chirp during the second
-    constexpr int PFD = (BLUE && C::NPASS <= 3) ? C::EPT / 2 : 0;
-    constexpr int PFDL = PFD > 0 ? C::EPT : 0;
-    float2 pf[C::EPT];
-    FftTile<S, THREADS, COLS, ZIN, PFD, PFDL>::run(v, t, ll, lds, job.tw, job.dtab, pf);
-
-    if constexpr (BLUE) {
-        // forward conj(v*D), inverse conj(v)*D = conj(v*conj(D)); the outer
-        // conjugation turns the next forward FFT into the inverse one
-#pragma unroll
-        for (int i = 0; i < C::EPT; ++i) {
-            const uint32_t pos = uint32_t(t + i * C::TPL);
-            v[i] = cmul_conj(v[i], i < PFDL ? pf[i] : job.dtab[pos]);
-        }
-        // the output chirp block is followed by readable entries up to
-        // position M/2 + M/16 (dir_tables_len), so every live slot can be loaded
-        FftTile<S, THREADS, COLS, false, LIVE>::run(v, t, ll, lds, job.tw, job.chirp_out, pf);
-    }
-
-    if (valid) {
-        float2* o = job.dst + int64_t(line) * job.ls + int64_t(t) * es;
-        const float sc = job.scale;
+        const float2* s = job.src + base;
+        float2 c[LIVE];
 #pragma unroll
         for (int i = 0; i < LIVE; ++i) {
-            const uint32_t pos = uint32_t(t + i * C::TPL);
-            if (in_line((int)pos)) {
-                float2 y;
-                if constexpr (BLUE) {
-                    // forward conj(v)*c = conj(v*conj(c)), inverse conj(v*c)/n = conj(v*(c/n))
-                    y = cmul_conj(v[i], pf[i]);
-                } else {
-                    y = cscale(cxor(v[i], sgn), sc);
-                }
-                if constexpr ((IO & IO_MAG) != 0)
-                    io.mag[int64_t(line) * io.mls + int64_t(pos) * io.mel] = cabs_scaled(y, io.mscale);
+            const bool in = i < SURE || t + i * C::TPL < n;
+            if constexpr ((IO & IO_LUM) != 0) {
+                const int64_t pos = in ? t + i * C::TPL : t;
+                v[i] = make_float2(image_luminance(io, int64_t(valid ? line : tile * C::LPW) * io.ils + pos * io.iel),
+                                   0.0f);
+            } else {
+                // opaque: else the select becomes a branch around the load
+                if constexpr (COLS)
+                    v[i] = load_global(i < SURE ? s + i * step : s + opaque(in ? i * step : 0));
                 else
-                    o[i * step] = y;
+                    v[i] = i < SURE ? load_at(s + i * step, off)
+                                    : load_at(s, opaque(in ? off + uint32_t(i * C::TPL) : off));
             }
+            if constexpr (BLUE) c[i] = load_at(job.chirp + i * C::TPL, uint32_t(t));
+        }
+#pragma unroll
+        for (int i = 0; i < C::EPT; ++i) {
+            if (i >= LIVE) {
+                v[i] = make_float2(0.0f, 0.0f);
+            } else if constexpr (BLUE) {
+                // forward x*c, inverse x*conj(c) (direction tables)
+                const bool in = i < SURE || t + i * C::TPL < n;
+                const float2 x = cmul(v[i], c[i]);
+                v[i] = in ? x : make_float2(0.0f, 0.0f);
+            } else {
+                v[i] = cxor(v[i], sgn);  // conj for the inverse
+            }
+        }
+    }
+
+    float2* o = job.dst + base;
+    const float sc = job.scale;
+    // finished slot i into the output
+    auto put = [&](int i, float2 y) {
+        const uint32_t pos = uint32_t(t + i * C::TPL);
+        if (!valid || !in_line((int)pos)) return;
+        if constexpr ((IO & IO_MAG) != 0)
+            io.mag[int64_t(line) * io.mls + int64_t(pos) * io.mel] = cabs_scaled(y, io.mscale);
+        else if constexpr (COLS)
+            store_global(o + i * step, y);
+        else
+            store_at(o + i * step, off, y);
+    };
+
+    if constexpr (C::SPLIT) {
+        if constexpr (BLUE) {
+            // the products of the branch below, slot by slot in the last passes
+            FftTile<S, THREADS, COLS, ZIN>::template run_epi<C::EPT>(
+                v, t, ll, lds, job.tw, job.dtab, [&](int, float2& x, float2 d) { x = cmul_conj(x, d); });
+            FftTile<S, THREADS, COLS>::template run_epi<LIVE>(v, t, ll, lds, job.tw, job.chirp_out,
+                                                               [&](int i, float2& x, float2 c) {
+                                                                   if (i < LIVE) put(i, cmul_conj(x, c));
+                                                               });
+        } else {
+            FftTile<S, THREADS, COLS>::template run_epi<0>(
+                v, t, ll, lds, job.tw, nullptr, [&](int i, float2& x, float2) { put(i, cscale(cxor(x, sgn), sc)); });
+        }
+    } else {
+        // Bluestein: D arrives during the first FFT, its first half one pass
+        // before the end and the rest at the start of the last pass (earlier
+        // loads of all of D spill at the 128-VGPR cap), and the live slots of
+        // the output chirp during the second
+        constexpr int PFD = (BLUE && C::NPASS <= 3) ? C::EPT / 2 : 0;
+        constexpr int PFDL = PFD > 0 ? C::EPT : 0;
+        float2 pf[C::EPT];
+        FftTile<S, THREADS, COLS, ZIN, PFD, PFDL>::run(v, t, ll, lds, job.tw, job.dtab, pf);
+
+        if constexpr (BLUE) {
+            // forward conj(v*D), inverse conj(v)*D = conj(v*conj(D)); the outer
+            // conjugation turns the next forward FFT into the inverse one
+#pragma unroll
+            for (int i = 0; i < C::EPT; ++i) {
+                v[i] = cmul_conj(v[i], i < PFDL ? pf[i] : load_at(job.dtab + i * C::TPL, uint32_t(t)));
+            }
+            // the output chirp block is followed by readable entries up to
+            // position M/2 + M/16 (dir_tables_len), so every live slot can be loaded
+            FftTile<S, THREADS, COLS, false, LIVE>::run(v, t, ll, lds, job.tw, job.chirp_out, pf);
+        }
+#pragma unroll
+        for (int i = 0; i < LIVE; ++i) {
+            // forward conj(v)*c = conj(v*conj(c)), inverse conj(v*c)/n = conj(v*(c/n))
+            if constexpr (BLUE)
+                put(i, cmul_conj(v[i], pf[i]));
+            else
+                put(i, cscale(cxor(v[i], sgn), sc));
         }
     }
 }

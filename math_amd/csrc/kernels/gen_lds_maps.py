@@ -26,15 +26,15 @@ CANDIDATES = [(0, 2)] + [(c, s) for c in (1, 2, 4, 8, 16) for s in range(2, 10)]
 
 def is_f3(s): return s >= F3_BASE
 def m_of(s): return (3 << (s - F3_BASE)) if is_f3(s) else (1 << s)
-def fft_bits(s): return 2 if is_f3(s) else 4
-def ept_of(s): return 12 if is_f3(s) else (1 << s if s < 4 else 16)
+def is_wide(s): return s in (13, 14)
+def ept_of(s): return 12 if is_f3(s) else 32 if is_wide(s) else (1 << s if s < 4 else 16)
 
 
 def npass_of(s):
     if is_f3(s):
         a = s - F3_BASE - 2
         return a // 2 + a % 2 + 1
-    return (s + 3) // 4
+    return 3 if is_wide(s) else (s + 3) // 4
 
 
 def radix_of(s, p):
@@ -43,6 +43,8 @@ def radix_of(s, p):
     if is_f3(s):
         a = s - F3_BASE - 2
         return 4 if p < a // 2 else (12 if p == npass_of(s) - 1 else 2)
+    if is_wide(s):
+        return 32 if p == 0 or (s == 14 and p == 1) else 16
     return 1 << min(4, s - 4 * p)
 
 

@@ -15,7 +15,7 @@ namespace mdft {
 
 __host__ __device__ constexpr int image_threads(int shape, bool wide)
 {
-    const int tpl = m_of(shape) / ept_of(shape);
+    const int tpl = tpl_of(shape);
     const int base = wide ? 1024 : 256;
     return tpl > base ? tpl : base;
 }

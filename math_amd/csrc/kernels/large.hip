@@ -185,7 +185,7 @@ static hipError_t launch_large_tt(const LargeJob& job0, hipStream_t stream)
 template <int LOGM>
 static hipError_t launch_large_t(const LargeJob& job, int min_blocks, hipStream_t stream)
 {
-    constexpr int TPL = m_of(LOGM) / ept_of(LOGM);
+    constexpr int TPL = tpl_of(LOGM);
     auto blocks = [&](int t) { return (job.count + t / TPL - 1) / (t / TPL); };
     if constexpr (TPL <= 256) {
         if (blocks(1024) < min_blocks) {

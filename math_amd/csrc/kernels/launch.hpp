@@ -108,14 +108,26 @@ hipError_t launch_image_magnitude(const ImageIO& io, const float2* src, int w, i
 // lengths 1024-4096 (wider contiguous runs per row), two workgroups per CU.
 constexpr int BATCH_COL_THREADS = 512;
 
-// batch kernels: threads is 256 (padded lengths up to 4096), 512 or 1024 (up to 8192)
+// batch kernels: threads is 256, 512 or 1024 (padded lengths up to 8192; 6144 from 512 threads)
 hipError_t launch_batch_grid(int threads, const BatchJob* jobs, const uint2* items, uint32_t nitems,
                              hipStream_t stream);
 hipError_t launch_batch_persistent(int threads, const BatchJob* jobs, const uint2* items, uint32_t nitems,
                                    uint32_t* ctl, uint32_t nctl, int grid, uint32_t spin_limit, hipStream_t stream);
+// their kernels of one workgroup size (batch_kernels.hip, compiled per size and launch shape)
+template <int T>
+hipError_t launch_batch_grid_t(const BatchJob* jobs, const uint2* items, uint32_t nitems, hipStream_t stream);
+template <int T>
+hipError_t launch_batch_persistent_t(const BatchJob* jobs, const uint2* items, uint32_t nitems, uint32_t* ctl,
+                                     int grid, uint32_t spin_limit, hipStream_t stream);
+template <int T>
+hipError_t batch_occupancy_t(int* blocks_per_cu);
+template <int T>
+hipError_t warm_batch_grid(uint32_t* word, hipStream_t stream);
+template <int T>
+hipError_t warm_batch_persistent(uint32_t* word, hipStream_t stream);
 // lines of a shape one tile of `threads` threads holds (0: the shape does not fit)
 int batch_lines_per_tile(int threads, int shape);
 hipError_t batch_occupancy(int threads, int* blocks_per_cu);
-int batch_max_logm(int threads);
+int batch_max_logm();
 
 }  // namespace mdft

@@ -20,13 +20,14 @@ __device__ __forceinline__ double2 unit_root(int64_t q, int64_t den)
     return make_double2(c, -s);
 }
 
-// row k of a pass: TW_ROW powers (tw_exponent) of w = exp(-2*pi*i*k/(ns*radix))
+// row k of a pass: tw_row powers (tw_exponent) of w = exp(-2*pi*i*k/(ns*radix))
 __global__ void k_gen_twiddle_block(float2* out, int ns, int radix)
 {
     const int64_t idx = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     const int64_t len = int64_t(ns) * radix;
-    if (idx >= int64_t(ns) * TW_ROW) return;
-    const int64_t k = idx / TW_ROW, e = tw_exponent(radix, (int)(idx % TW_ROW));
+    const int row = tw_row(radix);
+    if (idx >= int64_t(ns) * row) return;
+    const int64_t k = idx / row, e = tw_exponent(radix, (int)(idx % row));
     const double2 w = unit_root((k * e) % len, len);
     out[idx] = make_float2((float)w.x, (float)w.y);
 }
@@ -137,7 +138,7 @@ hipError_t gen_twiddles(float2* table, hipStream_t stream)
         for (int p = 1; p < npass_of(shape); ++p) {
             const int ns = ns_of(shape, p);
             const int radix = radix_of(shape, p);
-            const int64_t len = int64_t(ns) * TW_ROW;
+            const int64_t len = tw_pass_len(shape, p);
             float2* out = table + tw_off(shape) + tw_pass_off(shape, p);
             const int blocks = (int)((len + 255) / 256);
             hipLaunchKernelGGL(k_gen_twiddle_block, dim3(blocks), dim3(256), 0, stream, out, ns, radix);
