@@ -109,8 +109,9 @@ __device__ __noinline__ void run_tile_call(const BatchJob* jobs, uint32_t job, i
 {
     static_assert(sizeof(BatchJob) % 4 == 0, "copied by words");
     const uint64_t p = reinterpret_cast<uint64_t>(jobs + job);
-    const uint64_t u = (uint64_t(__builtin_amdgcn_readfirstlane(uint32_t(p >> 32))) << 32) |
-                       __builtin_amdgcn_readfirstlane(uint32_t(p));
+    // the builtin returns a signed int: without the casts the low word's sign fills the high one
+    const uint64_t u = (uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(p >> 32)))) << 32) |
+                       uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(p)));
     auto words = reinterpret_cast<const __attribute__((address_space(4))) uint32_t*>(u);
     union Copy {
         uint32_t w[sizeof(BatchJob) / 4];

@@ -119,15 +119,22 @@ __host__ __device__ constexpr int ns_of(int s, int p)
 }
 
 // Twiddle rows of pass p >= 1 (stride Ns = ns_of(s, p), radix R): row k
-// (k < Ns) holds 4 entries of w = exp(-2*pi*i*k/(Ns*R)) (32 bytes, four rows
-// per cache line): w, w^2, w^4, w^8 for a power-of-two radix (the stage
-// twiddles of dft_twiddled), w^1, w^2, w^3, w^4 for radix 12 (the other powers
-// are products of these, expand_twiddles).  Radix 32 also needs w^16: rows of
-// 6 entries, the last unused.
-__host__ __device__ constexpr int tw_row(int radix) { return radix == 32 ? 6 : 4; }
-__host__ __device__ constexpr int tw_exponent(int radix, int e)
+// (k < Ns) holds powers of w = exp(-2*pi*i*k/(Ns*R)):
+//  * radix 16: w, w^2, w^4, w^8, the base twiddles of dft_twiddled (32 bytes,
+//    four rows per cache line; the other stage twiddles are rotations);
+//  * radix 32 (a pass of few rows): all 16 stage twiddles of dft_twiddled,
+//    w^16, w^8, w^4 * {1, W8}, w^2 * {1, W16, W16^2, W16^3}, w * {1, W32, .. W32^7};
+//  * other radices: w^1, w^2, w^3, w^4; the other powers are products of these
+//    (expand_twiddles).
+__host__ __device__ constexpr int tw_row(int radix) { return radix == 32 ? 16 : 4; }
+// entry e of row k: exp(-2*pi*i*q/(Ns*R)) with q = power * k + rotation * Ns*R/32
+__host__ __device__ constexpr int tw_power(int radix, int e)
 {
-    return (radix & (radix - 1)) == 0 ? (1 << e) : e + 1;
+    return radix == 16 ? (1 << e) : radix == 32 ? (e == 0 ? 16 : e == 1 ? 8 : e < 4 ? 4 : e < 8 ? 2 : 1) : e + 1;
+}
+__host__ __device__ constexpr int tw_rotation(int radix, int e)
+{
+    return radix != 32 || e < 2 ? 0 : e < 4 ? (e - 2) * 4 : e < 8 ? (e - 4) * 2 : e - 8;
 }
 __host__ __device__ constexpr int64_t tw_pass_len(int s, int p)
 {
@@ -277,34 +284,44 @@ __host__ __device__ constexpr int bitrev_small(int v, int bits)
 }
 
 // ---------------------------------------------------------------------------
-// Power-of-two radices: decimation in time with the pass's twiddles fused in.
+// Radix 16 and 32: decimation in time with the pass's twiddles fused in.
 //
 // A pass multiplies input r by w^r and takes the R-point DFT.  Split even and
 // odd r: stage h (h = 1, 2, 4, .. R/2) combines a and b into a +- t*b with
 // t = w^(R/2h) * exp(-2*pi*i*k/2h), k < h.  The products never stand alone:
 // a + t*b is four fused multiply-adds, a - t*b = 2a - (a + t*b) two more, so a
 // twiddled radix-2 butterfly costs 6 instructions (8 for a product and two
-// sums), and only w^(R/2), .., w^2, w (loaded) and their constant rotations
-// (t at k >= h/2 is -i times the one at k - h/2, a swap of operands) are
-// needed: 8 twiddles for radix 16 instead of 15.  A radix-16 pass issues 208
-// VALU instructions, against 274 for 15 products, 11 derived twiddles and a
-// DIF butterfly; the kernels' VALU work is what bounds the long Bluestein
-// lines.
+// sums, or where a - t*b is formed by itself), and only w^(R/2), .., w^2, w
+// and their constant rotations (t at k >= h/2 is -i times the one at k - h/2,
+// a swap of operands) are needed: 8 twiddles for radix 16 instead of 15.  A
+// radix-16 pass issues 224 VALU instructions, against 274 for 15 products, 11
+// derived twiddles and a DIF butterfly.  Radices 2, 4 and 8 keep separate
+// products: there the fused form saves nothing.
 // ---------------------------------------------------------------------------
-// a, b <- a + t*b, a - t*b with t rotated by -i when NEGI
-template <bool NEGI>
+// a, b <- a + t*b, a - t*b with t rotated by -i when NEGI.  FULL: a - t*b by
+// four fused multiply-adds of its own (8 instructions), which leaves out the
+// rounding of a + t*b that 2a - (a + t*b) carries along.
+template <bool NEGI, bool FULL>
 __device__ __forceinline__ void bfly_tw(float2& a, float2& b, float2 t)
 {
+    // (-i*t)*b = (t.x*b.y + t.y*b.x) - i*(t.x*b.x - t.y*b.y)
     float2 y;
     if constexpr (NEGI) {
-        // (-i*t)*b = (t.x*b.y + t.y*b.x) - i*(t.x*b.x - t.y*b.y)
         y.x = __builtin_fmaf(t.y, b.x, __builtin_fmaf(t.x, b.y, a.x));
         y.y = __builtin_fmaf(t.y, b.y, __builtin_fmaf(-t.x, b.x, a.y));
     } else {
         y.x = __builtin_fmaf(-t.y, b.y, __builtin_fmaf(t.x, b.x, a.x));
         y.y = __builtin_fmaf(t.y, b.x, __builtin_fmaf(t.x, b.y, a.y));
     }
-    b = make_float2(__builtin_fmaf(2.0f, a.x, -y.x), __builtin_fmaf(2.0f, a.y, -y.y));
+    if constexpr (!FULL) {
+        b = make_float2(__builtin_fmaf(2.0f, a.x, -y.x), __builtin_fmaf(2.0f, a.y, -y.y));
+    } else if constexpr (NEGI) {
+        b = make_float2(__builtin_fmaf(-t.y, b.x, __builtin_fmaf(-t.x, b.y, a.x)),
+                        __builtin_fmaf(-t.y, b.y, __builtin_fmaf(t.x, b.x, a.y)));
+    } else {
+        b = make_float2(__builtin_fmaf(t.y, b.y, __builtin_fmaf(-t.x, b.x, a.x)),
+                        __builtin_fmaf(-t.y, b.x, __builtin_fmaf(-t.x, b.y, a.y)));
+    }
     a = y;
 }
 
@@ -328,7 +345,7 @@ __device__ __forceinline__ void bfly_const(float2& a, float2& b)
         b = make_float2(__builtin_fmaf(-r, t.x, a.x), __builtin_fmaf(-r, t.y, a.y));
         a = make_float2(__builtin_fmaf(r, t.x, a.x), __builtin_fmaf(r, t.y, a.y));
     } else {
-        bfly_tw<false>(a, b, make_float2(kC32[m], -kS32[m]));
+        bfly_tw<false, false>(a, b, make_float2(kC32[m], -kS32[m]));
     }
 }
 
@@ -360,16 +377,22 @@ __device__ __forceinline__ void dit_stages(float2* u)
     }
 }
 
+// Stages whose butterflies take the 8-instruction form: with the 6-instruction
+// form in every stage the error against FP64 was 1-3 % above that of separate
+// products and sums at 512-4096 points, 5 % at 16384; so it is 0.5-1 % below.
+__host__ __device__ constexpr bool full_stage(int radix, int h) { return radix == 32 || h >= 8; }
+
 // stage H with the pass's twiddles; tw[k] = w^(R/2H) * exp(-2*pi*i*k/2H), k < max(H/2, 1)
 template <int R, int H, int BASE, int K>
 __device__ __forceinline__ void dit_tw_bfly(float2* u, const float2* tw)
 {
     if constexpr (BASE < R) {
         if constexpr (K < H) {
+            constexpr bool FULL = full_stage(R, H);
             if constexpr (H > 1 && K >= H / 2)
-                bfly_tw<true>(u[BASE + K], u[BASE + K + H], tw[K - H / 2]);
+                bfly_tw<true, FULL>(u[BASE + K], u[BASE + K + H], tw[K - H / 2]);
             else
-                bfly_tw<false>(u[BASE + K], u[BASE + K + H], tw[K]);
+                bfly_tw<false, FULL>(u[BASE + K], u[BASE + K + H], tw[K]);
             dit_tw_bfly<R, H, BASE, K + 1>(u, tw);
         } else {
             dit_tw_bfly<R, H, BASE + 2 * H, 0>(u, tw);
@@ -388,50 +411,32 @@ __device__ __forceinline__ void bit_reverse(float2* u)
     for (int i = 0; i < R; ++i) u[i] = t[i];
 }
 
-// R-point DFT of u[r] * w^r; q holds the pass's row (w, w^2), (w^4, w^8), (w^16, -)
+// R-point DFT of u[r] * w^r from the pass's row q (tw_row), R = 16 or 32
 template <int R>
 __device__ __forceinline__ void dft_twiddled(float2 (&u)[R], const float4* q)
 {
-    static_assert(R == 2 || R == 4 || R == 8 || R == 16 || R == 32, "radix");
+    static_assert(R == 16 || R == 32, "radix");
     bit_reverse<R>(u);
-    const float2 w1 = make_float2(q[0].x, q[0].y);
-    if constexpr (R == 2) {
-        dit_tw_bfly<R, 1, 0, 0>(u, &w1);
+    auto entry = [&](int e) { return e % 2 ? make_float2(q[e / 2].z, q[e / 2].w) : make_float2(q[e / 2].x, q[e / 2].y); };
+    if constexpr (R == 16) {
+        const float2 w1 = entry(0), w2 = entry(1), w4 = entry(2), w8 = entry(3);
+        dit_tw_bfly<R, 1, 0, 0>(u, &w8);
+        dit_tw_bfly<R, 2, 0, 0>(u, &w4);
+        const float2 t4[2] = {w2, twc<4>(w2)};
+        dit_tw_bfly<R, 4, 0, 0>(u, t4);
+        const float2 t8[4] = {w1, twc<2>(w1), twc<4>(w1), twc<6>(w1)};
+        dit_tw_bfly<R, 8, 0, 0>(u, t8);
     } else {
-        const float2 w2 = make_float2(q[0].z, q[0].w);
-        if constexpr (R == 4) {
-            dit_tw_bfly<R, 1, 0, 0>(u, &w2);
-            dit_tw_bfly<R, 2, 0, 0>(u, &w1);
-        } else {
-            const float2 w4 = make_float2(q[1].x, q[1].y);
-            if constexpr (R == 8) {
-                dit_tw_bfly<R, 1, 0, 0>(u, &w4);
-                dit_tw_bfly<R, 2, 0, 0>(u, &w2);
-                const float2 t4[2] = {w1, twc<4>(w1)};
-                dit_tw_bfly<R, 4, 0, 0>(u, t4);
-            } else {
-                const float2 w8 = make_float2(q[1].z, q[1].w);
-                if constexpr (R == 16) {
-                    dit_tw_bfly<R, 1, 0, 0>(u, &w8);
-                    dit_tw_bfly<R, 2, 0, 0>(u, &w4);
-                    const float2 t4[2] = {w2, twc<4>(w2)};
-                    dit_tw_bfly<R, 4, 0, 0>(u, t4);
-                    const float2 t8[4] = {w1, twc<2>(w1), twc<4>(w1), twc<6>(w1)};
-                    dit_tw_bfly<R, 8, 0, 0>(u, t8);
-                } else {
-                    const float2 w16 = make_float2(q[2].x, q[2].y);
-                    dit_tw_bfly<R, 1, 0, 0>(u, &w16);
-                    dit_tw_bfly<R, 2, 0, 0>(u, &w8);
-                    const float2 t4[2] = {w4, twc<4>(w4)};
-                    dit_tw_bfly<R, 4, 0, 0>(u, t4);
-                    const float2 t8[4] = {w2, twc<2>(w2), twc<4>(w2), twc<6>(w2)};
-                    dit_tw_bfly<R, 8, 0, 0>(u, t8);
-                    const float2 t16[8] = {w1,          twc<1>(w1), twc<2>(w1), twc<3>(w1),
-                                           twc<4>(w1), twc<5>(w1), twc<6>(w1), twc<7>(w1)};
-                    dit_tw_bfly<R, 16, 0, 0>(u, t16);
-                }
-            }
-        }
+        const float2 t1 = entry(0), t2 = entry(1);
+        dit_tw_bfly<R, 1, 0, 0>(u, &t1);
+        dit_tw_bfly<R, 2, 0, 0>(u, &t2);
+        const float2 t4[2] = {entry(2), entry(3)};
+        dit_tw_bfly<R, 4, 0, 0>(u, t4);
+        const float2 t8[4] = {entry(4), entry(5), entry(6), entry(7)};
+        dit_tw_bfly<R, 8, 0, 0>(u, t8);
+        const float2 t16[8] = {entry(8),  entry(9),  entry(10), entry(11),
+                               entry(12), entry(13), entry(14), entry(15)};
+        dit_tw_bfly<R, 16, 0, 0>(u, t16);
     }
 }
 
@@ -611,7 +616,7 @@ __device__ __forceinline__ void exchange_sync()
 template <int R>
 __host__ __device__ constexpr int tw_quads()
 {
-    return R <= 4 ? 1 : R <= 16 ? 2 : 3;
+    return R <= 2 ? 1 : R == 32 ? 8 : 2;
 }
 
 template <int S, int THREADS, int P>
@@ -764,7 +769,7 @@ struct FftPass {
                 float4 q[Q];
 #pragma unroll
                 for (int r2 = 0; r2 < Q; ++r2) q[r2] = w[b * Q + r2];
-                if constexpr ((R & (R - 1)) == 0) {
+                if constexpr (R == 16 || R == 32) {
                     dft_twiddled<R>(u, q);
                 } else {
                     float2 wt[R];

@@ -20,15 +20,16 @@ __device__ __forceinline__ double2 unit_root(int64_t q, int64_t den)
     return make_double2(c, -s);
 }
 
-// row k of a pass: tw_row powers (tw_exponent) of w = exp(-2*pi*i*k/(ns*radix))
+// row k of a pass: tw_row entries (tw_power, tw_rotation) of w = exp(-2*pi*i*k/(ns*radix))
 __global__ void k_gen_twiddle_block(float2* out, int ns, int radix)
 {
     const int64_t idx = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     const int64_t len = int64_t(ns) * radix;
     const int row = tw_row(radix);
     if (idx >= int64_t(ns) * row) return;
-    const int64_t k = idx / row, e = tw_exponent(radix, (int)(idx % row));
-    const double2 w = unit_root((k * e) % len, len);
+    const int64_t k = idx / row;
+    const int e = (int)(idx % row);
+    const double2 w = unit_root((k * tw_power(radix, e) + tw_rotation(radix, e) * (len / 32)) % len, len);
     out[idx] = make_float2((float)w.x, (float)w.y);
 }
 
