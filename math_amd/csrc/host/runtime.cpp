@@ -5,6 +5,7 @@
 
 #include "../../../include/mdft.h"
 
+#include <algorithm>
 #include <cstdlib>
 #include <string>
 #include <vector>
@@ -521,46 +522,49 @@ void Context::enqueue_large_axis(const LinePlan& lp, const float2* src, float2* 
         enqueue_large_blue3(lp, src, dst, es, ls, count, inverse, scratch, stream);
         return;
     }
+    // The scratch holds a line's M elements together; where the lines are an
+    // image's columns (adjacent in memory) it keeps the lines adjacent too, and
+    // the steps take them fastest: every access of a step is then one run over
+    // the lines, instead of one element per image row.
+    const bool inter = es > 1 && ls == 1 && count > 1 && count * std::max(M1, M2) <= 0x7fffffff;
+    const int64_t sl = inter ? 1 : M, se = inter ? count : 1, lines = inter ? count : 0;
     float2* S = scratch;  // step A output, count * M (later steps in place or out of it)
-    auto step_a = [&](const float2* from, int64_t fls, int64_t fes, int load_mode) {
+    auto step_a = [&](int load_mode) {
         LargeJob a = large_job(lp.tw_lo, lp.tw_hi, inverse, lp.n);
-        a.src = from;
+        a.src = src;
         a.dst = S;
-        a.sub_in = M1, a.ls_in = fls, a.ls2_in = fes, a.es_in = M1 * fes;
-        a.sub_out = M1, a.ls_out = M, a.ls2_out = M2, a.es_out = 1;
-        a.count = count * M1;
+        a.sub_in = M1, a.ls_in = ls, a.ls2_in = es, a.es_in = M1 * es;
+        a.sub_out = M1, a.ls_out = sl, a.ls2_out = M2 * se, a.es_out = se;
+        a.count = count * M1, a.lines = lines;
         a.load_mode = load_mode, a.store_mode = LARGE_STORE_TWIDDLE;
         a.tmod = M1;  // w_M^(n1*k2)
         a.m1 = M1, a.m2 = M2;
         a.chirp = lp.chirp;
         large_step(lp.logm2, twiddles(lp.logm2), a, cu_count_, stream);
     };
-    auto step_c = [&](float2* to, int64_t tls, int64_t tes, int store_mode, float sc) {
+    if (!lp.blue) {
+        step_a(LARGE_LOAD_CONJ);  // conj(x) for the inverse
+        // C: conj(v)/n for the inverse
         LargeJob c = large_job(lp.tw_lo, lp.tw_hi, inverse, lp.n);
         c.src = S;
-        c.dst = to;
-        c.sub_in = M2, c.ls_in = M, c.ls2_in = 1, c.es_in = M2;
-        c.sub_out = M2, c.ls_out = tls, c.ls2_out = tes, c.es_out = M2 * tes;
-        c.count = count * M2;
-        c.load_mode = LARGE_LOAD_PLAIN, c.store_mode = store_mode;
-        c.m1 = M1, c.m2 = M2, c.kmul = M2, c.scale = sc;
-        c.chirp = lp.chirp, c.dtab = lp.dtab;
+        c.dst = dst;
+        c.sub_in = M2, c.ls_in = sl, c.ls2_in = se, c.es_in = M2 * se;
+        c.sub_out = M2, c.ls_out = ls, c.ls2_out = es, c.es_out = M2 * es;
+        c.count = count * M2, c.lines = lines;
+        c.load_mode = LARGE_LOAD_PLAIN, c.store_mode = LARGE_STORE_CONJ;
+        c.m1 = M1, c.m2 = M2, c.kmul = M2, c.scale = scale;
         large_step(lp.logm1, twiddles(lp.logm1), c, cu_count_, stream);
-    };
-    if (!lp.blue) {
-        step_a(src, ls, es, LARGE_LOAD_CONJ);         // conj(x) for the inverse
-        step_c(dst, ls, es, LARGE_STORE_CONJ, scale);  // conj(v)/n for the inverse
         return;
     }
-    step_a(src, ls, es, LARGE_LOAD_CHIRP);  // x * c, zero past n
+    step_a(LARGE_LOAD_CHIRP);  // x * c, zero past n
     // B, in place: per (line, k2) the M1-point FFT over n1, conj(v * D), the
     // M1-point FFT over k1 and the twiddle w_M^(k2*j1), at j1*M2 + k2
     LargeJob b = large_job(lp.tw_lo, lp.tw_hi, inverse, lp.n);
     b.src = S;
     b.dst = S;
-    b.sub_in = M2, b.ls_in = M, b.ls2_in = 1, b.es_in = M2;
-    b.sub_out = M2, b.ls_out = M, b.ls2_out = 1, b.es_out = M2;
-    b.count = count * M2;
+    b.sub_in = M2, b.ls_in = sl, b.ls2_in = se, b.es_in = M2 * se;
+    b.sub_out = M2, b.ls_out = sl, b.ls2_out = se, b.es_out = M2 * se;
+    b.count = count * M2, b.lines = lines;
     b.load_mode = LARGE_LOAD_PLAIN, b.store_mode = LARGE_STORE_DIAG_FFT;
     b.tmod = M2;  // w_M^(k2*j1)
     b.m1 = M1, b.m2 = M2, b.kmul = M2;
@@ -571,9 +575,9 @@ void Context::enqueue_large_axis(const LinePlan& lp, const float2* src, float2* 
     LargeJob c = large_job(lp.tw_lo, lp.tw_hi, inverse, lp.n);
     c.src = S;
     c.dst = dst;
-    c.sub_in = M1, c.ls_in = M, c.ls2_in = M2, c.es_in = 1;
+    c.sub_in = M1, c.ls_in = sl, c.ls2_in = M2 * se, c.es_in = se;
     c.sub_out = M1, c.ls_out = ls, c.ls2_out = es, c.es_out = M1 * es;
-    c.count = count * M1;
+    c.count = count * M1, c.lines = lines;
     c.load_mode = LARGE_LOAD_PLAIN, c.store_mode = LARGE_STORE_CHIRP;
     c.m1 = M1, c.m2 = M2, c.kmul = M1, c.scale = scale;
     c.chirp = lp.chirp;

@@ -41,22 +41,38 @@ namespace mdft {
 
 __device__ __forceinline__ int64_t low_bits(int64_t v, int lg) { return v & ((int64_t(1) << lg) - 1); }
 
-// line L of a step maps to (L / sub) * ls + r * ls2 with r = L % sub, element
-// p to p * es; r may split once more (sub2 > 0): (r % sub2) * ls2 + (r / sub2) * ls3.
-// sub and sub2 are powers of two (lg: their log2, lg2 = -1 without the split).
-__device__ __forceinline__ int64_t line_base3(int64_t L, int lg, int64_t ls, int64_t ls2, int lg2, int64_t ls3)
+// sub-line r of a line maps to line * ls + r * ls2, element p to p * es; r may
+// split once more (lg2 >= 0): (r % 2^lg2) * ls2 + (r / 2^lg2) * ls3
+__device__ __forceinline__ int64_t line_base3(int64_t line, int64_t r, int64_t ls, int64_t ls2, int lg2, int64_t ls3)
 {
-    const int64_t r = low_bits(L, lg);
     const int64_t off = lg2 >= 0 ? low_bits(r, lg2) * ls2 + (r >> lg2) * ls3 : r * ls2;
-    return (L >> lg) * ls + off;
+    return line * ls + off;
 }
 
-// w_M^e, e < M, from the two-level table
-__device__ __forceinline__ float2 large_twiddle(const LargeJob& job, int64_t e)
+// v[i] *= w_M^(tq * (t + i*TPL)) from the two-level table: the exponent is
+// below M <= 2^30, so 32 bits hold it, and every entry is on its way before the
+// first product waits (half the slots at a time where a thread has 32).
+template <class C>
+__device__ __forceinline__ void apply_twiddles(float2 (&v)[C::EPT], const LargeJob& job, uint32_t tq, uint32_t t)
 {
-    return cmul(job.tw_lo[e & (LARGE_LO - 1)], job.tw_hi[e >> LARGE_LO_BITS]);
+    constexpr int G = C::EPT > 16 ? 8 : C::EPT;
+#pragma unroll
+    for (int g = 0; g < C::EPT; g += G) {
+        float2 lo[G], hi[G];
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+            const uint32_t e = tq * (t + uint32_t((g + i) * C::TPL));
+            lo[i] = load_at(job.tw_lo, e & uint32_t(LARGE_LO - 1));
+            hi[i] = load_at(job.tw_hi, e >> LARGE_LO_BITS);
+        }
+#pragma unroll
+        for (int i = 0; i < G; ++i) v[g + i] = cmul(v[g + i], cmul(lo[i], hi[i]));
+    }
 }
 
+// The load and store modes are uniform: each is a branch around whole loops
+// over the slots, so a slot's loads never wait for the one before (a branch
+// per slot made every load a latency of its own).
 template <int LOGM, int T, bool FUSED>
 __global__ __launch_bounds__(T) void k_large_step(LargeJob job)
 {
@@ -66,75 +82,122 @@ __global__ __launch_bounds__(T) void k_large_step(LargeJob job)
     const int tid = threadIdx.x;
     const int ll = tid % C::LPW;
     const int t = tid / C::LPW;
-    const int64_t line = int64_t(xcd_remap(blockIdx.x, gridDim.x)) * C::LPW + ll;
-    const bool valid = line < job.count;
+    // a sub-line past the last one repeats the tile's first and stores nothing
+    const int64_t line0 = int64_t(xcd_remap(blockIdx.x, gridDim.x)) * C::LPW;
+    const bool valid = line0 + ll < job.count;
+    const int64_t L = valid ? line0 + ll : line0;
+    // (line, sub-line) of the load and of the store: sub-lines fastest, or lines
+    // fastest when the lines of an image are its columns
+    int64_t line_in, r_in, line_out, r_out;
+    if (job.lines > 0) {
+        line_in = line_out = uint32_t(L) % uint32_t(job.lines);
+        r_in = r_out = uint32_t(L) / uint32_t(job.lines);
+    } else {
+        line_in = L >> job.lg_sub_in, r_in = low_bits(L, job.lg_sub_in);
+        line_out = L >> job.lg_sub_out, r_out = low_bits(L, job.lg_sub_out);
+    }
     const uint32_t sgn = job.inverse ? 0x80000000u : 0u;
-    // sub-line coordinate inside the long line (the chirp load's element offset)
-    const int64_t sub_idx = low_bits(line, job.lg_sub_in);
-    // twiddle exponent per element of this sub-line
-    const int64_t tq = (low_bits(line, job.lg_tmod) >> job.lg_tdiv) * job.tmul;
+    // twiddle exponent per element of this sub-line (tmod divides both sub-line counts)
+    const uint32_t tq = uint32_t((low_bits(r_in, job.lg_tmod) >> job.lg_tdiv) * job.tmul);
 
     float2 v[C::EPT];
     {
-        const float2* s =
-            job.src + (valid ? line_base3(line, job.lg_sub_in, job.ls_in, job.ls2_in, job.lg_sub2_in, job.ls3_in) : 0);
+        const int64_t step = int64_t(C::TPL) * job.es_in;
+        const float2* s = job.src +
+                          line_base3(line_in, r_in, job.ls_in, job.ls2_in, job.lg_sub2_in, job.ls3_in) +
+                          int64_t(t) * job.es_in;
+        if (job.load_mode == LARGE_LOAD_CHIRP) {
+            // element j = sub + m1*pos of the Bluestein input: chirped, zero past
+            // n <= M/2 + 1, so slots past the middle hold nothing and the middle
+            // one only element M/2 of such a line; a slot that ends earlier reads
+            // the thread's first one, which is inside: sub + m1*t < M/16 < n
+            const int64_t j0 = r_in + job.m1 * t, jstep = job.m1 * C::TPL;
+            constexpr int HALF = C::EPT / 2;
+            float2 c[HALF + 1];
 #pragma unroll
-        for (int i = 0; i < C::EPT; ++i) {
-            const int64_t pos = t + i * C::TPL;
-            float2 x = make_float2(0.0f, 0.0f);
-            if (valid) {
-                if (job.load_mode == LARGE_LOAD_CHIRP) {
-                    // element n1 + M1*n2 of the Bluestein input: chirped, zero past n
-                    const int64_t j = sub_idx + job.m1 * pos;
-                    if (j < job.n) x = cmul(s[pos * job.es_in], cxor(job.chirp[j], sgn));
-                } else if (job.load_mode == LARGE_LOAD_CONJ) {
-                    x = cxor(s[pos * job.es_in], sgn);
-                } else if (job.load_mode == LARGE_LOAD_TWIDDLE) {
-                    x = cmul(s[pos * job.es_in], large_twiddle(job, tq * pos));
+            for (int i = 0; i < HALF; ++i) {
+                const bool in = j0 + i * jstep < job.n;
+                v[i] = load_global(s + opaque(in ? i * step : 0));
+                c[i] = load_global(job.chirp + opaque(in ? j0 + i * jstep : j0));
+            }
+            v[HALF] = c[HALF] = make_float2(0.0f, 0.0f);
+            if (j0 + HALF * jstep < job.n) {
+                v[HALF] = load_global(s + HALF * step);
+                c[HALF] = load_global(job.chirp + (j0 + HALF * jstep));
+            }
+#pragma unroll
+            for (int i = 0; i < C::EPT; ++i) {
+                if (i > HALF) {
+                    v[i] = make_float2(0.0f, 0.0f);
                 } else {
-                    x = s[pos * job.es_in];
+                    const float2 x = cmul(v[i], cxor(c[i], sgn));
+                    v[i] = j0 + i * jstep < job.n ? x : make_float2(0.0f, 0.0f);
                 }
             }
-            v[i] = x;
+        } else {
+#pragma unroll
+            for (int i = 0; i < C::EPT; ++i) v[i] = load_global(s + i * step);
+            if (job.load_mode == LARGE_LOAD_CONJ) {
+#pragma unroll
+                for (int i = 0; i < C::EPT; ++i) v[i] = cxor(v[i], sgn);
+            } else if (job.load_mode == LARGE_LOAD_TWIDDLE) {
+                apply_twiddles<C>(v, job, tq, t);
+            }
         }
     }
 
     FftTile<LOGM, T, true>::run(v, t, ll, lds, job.tw);
-    const int64_t q_line = low_bits(line, job.lg_sub_out);
-    if constexpr (FUSED) {
-        // conj(v * D) at k = k2 + M2*k1 (q_line = k2 < M2, pos = k1 < M1; three factors: kr + Mr*k1;
-        // in bounds on every line), then the next length-M1 FFT over k1; its outputs j1 take the twiddle below
+    // natural index of slot i: kq + i * kstep (q < M2, pos < M1: q + M2*pos; three factors: kr + Mr*k1)
+    const int64_t kq = r_out + job.kmul * t, kstep = job.kmul * C::TPL;
+    // conj(v * D), forward; conj(v * conj(D)), inverse
+    auto times_d = [&]() {
+        constexpr int G = C::EPT > 16 ? 16 : C::EPT;
 #pragma unroll
-        for (int i = 0; i < C::EPT; ++i) {
-            const int64_t k = q_line + job.kmul * (t + i * C::TPL);
-            v[i] = cmul_conj(v[i], cxor(job.dtab[k], sgn));
+        for (int g = 0; g < C::EPT; g += G) {
+            float2 d[G];
+#pragma unroll
+            for (int i = 0; i < G; ++i) d[i] = load_global(job.dtab + kq + (g + i) * kstep);
+#pragma unroll
+            for (int i = 0; i < G; ++i) v[g + i] = cmul_conj(v[g + i], cxor(d[i], sgn));
         }
+    };
+    if constexpr (FUSED) {
+        // then the next length-M1 FFT over k1; its outputs j1 take the twiddle below
+        times_d();
         FftTile<LOGM, T, true>::run(v, t, ll, lds, job.tw);
     }
 
-    if (!valid) return;
-    float2* o = job.dst + line_base3(line, job.lg_sub_out, job.ls_out, job.ls2_out, job.lg_sub2_out, job.ls3_out);
+    const int64_t ostep = int64_t(C::TPL) * job.es_out;
+    float2* o = job.dst + line_base3(line_out, r_out, job.ls_out, job.ls2_out, job.lg_sub2_out, job.ls3_out) +
+                int64_t(t) * job.es_out;
+    if (job.store_mode == LARGE_STORE_CHIRP) {
+        // outputs past n <= M/2 + 1 are not kept: only the slots up to the middle
+        constexpr int LIVE = C::EPT / 2 + 1;
+        float2 c[LIVE];
 #pragma unroll
-    for (int i = 0; i < C::EPT; ++i) {
-        const int64_t pos = t + i * C::TPL;
-        float2 y = v[i];
-        if (job.store_mode == LARGE_STORE_TWIDDLE || job.store_mode == LARGE_STORE_DIAG_FFT) {
-            // the step's twiddle w_M^(tq*pos), tq*pos < M: n1*k2 (A), k2*j1 (B), M1*n2*k3 (A1),
-            // kr*j1 (fused C), M1*k3*jr2 (X1)
-            y = cmul(y, large_twiddle(job, tq * pos));
-        } else if (job.store_mode == LARGE_STORE_DIAG) {
-            // natural index k = k2 + M2*k1; forward conj(v*D), inverse conj(v*conj(D))
-            const int64_t k = q_line + job.kmul * pos;
-            y = cmul_conj(y, cxor(job.dtab[k], sgn));
-        } else if (job.store_mode == LARGE_STORE_CHIRP) {
-            const int64_t k = q_line + job.kmul * pos;
-            if (k >= job.n) continue;
-            y = cscale(cmul_conj(y, cxor(job.chirp[k], sgn ^ 0x80000000u)), job.scale);
-        } else if (job.store_mode == LARGE_STORE_CONJ) {
-            y = cscale(cxor(y, sgn), job.scale);
+        for (int i = 0; i < LIVE; ++i) {
+            const int64_t k = kq + i * kstep;
+            c[i] = load_global(job.chirp + opaque(k < job.n ? k : int64_t(0)));
         }
-        o[pos * job.es_out] = y;
+#pragma unroll
+        for (int i = 0; i < LIVE; ++i)
+            if (valid && kq + i * kstep < job.n)
+                store_global(o + i * ostep, cscale(cmul_conj(v[i], cxor(c[i], sgn ^ 0x80000000u)), job.scale));
+        return;
     }
+    if (job.store_mode == LARGE_STORE_TWIDDLE || job.store_mode == LARGE_STORE_DIAG_FFT) {
+        // the step's twiddle w_M^(tq*pos), tq*pos < M: n1*k2 (A), k2*j1 (B), M1*n2*k3 (A1),
+        // kr*j1 (fused C), M1*k3*jr2 (X1)
+        apply_twiddles<C>(v, job, tq, t);
+    } else if (job.store_mode == LARGE_STORE_DIAG) {
+        times_d();
+    } else if (job.store_mode == LARGE_STORE_CONJ) {
+#pragma unroll
+        for (int i = 0; i < C::EPT; ++i) v[i] = cscale(cxor(v[i], sgn), job.scale);
+    }
+    if (!valid) return;
+#pragma unroll
+    for (int i = 0; i < C::EPT; ++i) store_global(o + i * ostep, v[i]);
 }
 
 // log2 of a power of two, -1 for anything else
@@ -161,6 +224,9 @@ static hipError_t launch_large_tt(const LargeJob& job0, hipStream_t stream)
     job.lg_sub2_out = job.sub2_out > 0 ? lg_of(job.sub2_out) : -1;
     if (job.lg_sub_in < 0 || job.lg_sub_out < 0 || job.sub2_in < 0 || job.sub2_out < 0 ||
         (job.sub2_in > 0 && job.lg_sub2_in < 0) || (job.sub2_out > 0 && job.lg_sub2_out < 0))
+        return hipErrorInvalidValue;
+    // lines fastest: one sub-line count, indices in 32 bits
+    if (job.lines < 0 || (job.lines > 0 && (job.sub_in != job.sub_out || job.count > 0x7fffffff)))
         return hipErrorInvalidValue;
     const bool twiddled = job.load_mode == LARGE_LOAD_TWIDDLE || job.store_mode == LARGE_STORE_TWIDDLE ||
                           job.store_mode == LARGE_STORE_DIAG_FFT;

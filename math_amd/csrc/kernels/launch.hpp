@@ -46,7 +46,8 @@ enum LargeStore { LARGE_STORE_PLAIN = 0, LARGE_STORE_TWIDDLE = 1, LARGE_STORE_DI
 // ls3_in in place of r * ls2_in), and writes likewise with the *_out fields.
 // The twiddle of LARGE_LOAD_TWIDDLE, LARGE_STORE_TWIDDLE and
 // LARGE_STORE_DIAG_FFT is w_M^e of element pos, e = ((L % tmod) / tdiv) * tmul * pos.
-// sub_*, sub2_*, tmod and tdiv are powers of two.
+// sub_*, sub2_*, tmod and tdiv are powers of two.  lines > 0: sub-line r of line
+// l is L = r * lines + l instead (adjacent lanes take adjacent lines).
 struct LargeJob {
     const float2* src;
     float2* dst;
@@ -55,7 +56,7 @@ struct LargeJob {
     int64_t ls_out, ls2_out, es_out, sub_out;
     int64_t sub2_out, ls3_out;
     int64_t tmod, tdiv, tmul;
-    int64_t count;
+    int64_t count, lines;
     int load_mode, store_mode, inverse, pad;
     int64_t n, m1, m2;
     int64_t kmul;  // natural index of the store modes DIAG, DIAG_FFT, CHIRP: q + kmul * pos
