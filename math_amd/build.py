@@ -29,7 +29,7 @@ COMMON = [
 # the longest compilations first
 SOURCES = [
     ("kernels/batch_kernels.hip", f"batch_{kind}_{t}", [f"-DMDFT_BATCH_T={t}", f"-DMDFT_BATCH_PERSISTENT_TU={p}"])
-    for p, kind in ((0, "grid"), (1, "persistent")) for t in (256, 512, 1024)
+    for p, kind, t in ((0, "grid", 256), (1, "persistent", 256), (0, "grid", 512), (0, "grid", 1024))
 ] + [
     "kernels/axis.hip",
     "kernels/batch.hip",

@@ -63,14 +63,14 @@ void enqueue_batch(mdft_batch_s* b, hipStream_t stream)
 {
     const int T = b->threads;
     if (b->flags & MDFT_BATCH_DEPENDENT) {
-        mdft::hip_check(mdft::launch_batch_persistent(T, b->jobs_dev, b->items_dev, b->nitems, b->ctl_dev, b->nctl,
+        mdft::hip_check(mdft::launch_batch_persistent(b->jobs_dev, b->items_dev, b->nitems, b->ctl_dev, b->nctl,
                                                       b->grid, b->spin_limit, stream),
                         "batch launch");
     } else if (b->flags & MDFT_BATCH_PERSISTENT) {
-        mdft::hip_check(mdft::launch_batch_persistent(T, b->jobs_dev, b->items_dev, b->nphase1, b->ctl_dev, b->nctl,
+        mdft::hip_check(mdft::launch_batch_persistent(b->jobs_dev, b->items_dev, b->nphase1, b->ctl_dev, b->nctl,
                                                       b->grid, b->spin_limit, stream),
                         "batch launch (phase 1)");
-        mdft::hip_check(mdft::launch_batch_persistent(T, b->jobs_dev, b->items_dev + b->nphase1,
+        mdft::hip_check(mdft::launch_batch_persistent(b->jobs_dev, b->items_dev + b->nphase1,
                                                       b->nitems - b->nphase1, b->ctl_dev + b->nctl, b->nctl, b->grid,
                                                       b->spin_limit, stream),
                         "batch launch (phase 2)");
@@ -197,7 +197,7 @@ int mdft_batch_create(mdft_batch* batch, const mdft_desc* descs, uint32_t count,
     count_phase_bytes(b.get());
 
     int per_cu = 0;
-    mdft::hip_check(mdft::batch_occupancy(T, &per_cu), "occupancy");
+    mdft::hip_check(mdft::batch_occupancy(&per_cu), "occupancy");
     b->grid = std::max(1, ctx.cu_count() * std::max(per_cu, 1));
 
     const size_t njobs = b->build.jobs.size();

@@ -74,13 +74,13 @@ void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int T, i
         auto cp = ctx.line_plan(h, true);
         out.keep.push_back(rp);
         out.keep.push_back(cp);
-        const int lpw_r = w > 1 ? batch_lines_per_tile(T, rp->shape) : 0;
+        const int lpw_r = w > 1 ? batch_lines_per_tile(T, rp->shape, false) : 0;
         // a whole image runs both passes in one row-phase workgroup
-        const int lpw_cw = h > 1 ? batch_lines_per_tile(T, cp->shape) : 0;
+        const int lpw_cw = h > 1 ? batch_lines_per_tile(T, cp->shape, true) : 0;
         const bool whole = (w > 1 && h > 1 && h <= lpw_r && w <= lpw_cw);
         // column tiles of images with a row pass run in the column phase (TC
         // threads); a single-column-pass image (w == 1) runs with the rows
-        const int lpw_c = h > 1 ? batch_lines_per_tile((w > 1 && !whole) ? TC : T, cp->shape) : 0;
+        const int lpw_c = h > 1 ? batch_lines_per_tile((w > 1 && !whole) ? TC : T, cp->shape, true) : 0;
         const int ntr = w > 1 ? (h + lpw_r - 1) / lpw_r : 0;
         const int ntc = h > 1 ? (w + lpw_c - 1) / lpw_c : 0;
         const int sig = (dependent && w > 1 && h > 1 && !whole) ? (int)counter++ : -1;
@@ -152,7 +152,7 @@ void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int T, i
         std::vector<double> c1, c2;
         for (const Item& it : items) {
             // cost of a tile ~ points x passes (x2 for Bluestein's two FFTs)
-            const int lpw = batch_lines_per_tile(it.kind == 2 && it.phase == 2 ? TC : T, it.shape);
+            const int lpw = batch_lines_per_tile(it.kind == 2 && it.phase == 2 ? TC : T, it.shape, it.kind == 2);
             const double cost = double(lpw) * double(it.m) * (std::log2(double(it.m)) + 2) * (it.blue ? 2.0 : 1.0) *
                                 (it.kind == 0 ? 2.0 : 1.0);
             (it.phase == 1 ? p1 : p2).push_back(it.v);

@@ -157,9 +157,9 @@ int mdft_cache_set_limit(uint64_t bytes)
 
 static void check_tune_args(int shape, int blue, int cols)
 {
-    const bool ok_shape = (shape >= 1 && shape <= mdft::MAX_LOGM) ||
-                          (mdft::is_f3(shape) && mdft::f3_k(shape) >= mdft::F3_MIN_K &&
-                           mdft::f3_k(shape) <= mdft::F3_MAX_K);
+    const bool ok_shape =
+        (shape >= 1 && shape <= mdft::MAX_LOGM) ||
+        (shape >= mdft::F3_BASE + mdft::F3_MIN_K && shape <= mdft::F3_BASE + mdft::F3_MAX_K);
     if (!ok_shape || (blue != 0 && blue != 1) || (cols != 0 && cols != 1))
         throw Error(MDFT_ERR_INVALID, "tune: shape must be in [1, 14] or [38, 43], blue and cols 0 or 1");
 }

@@ -76,8 +76,8 @@ int line_shape(long long n, bool cols)
         return F3_BASE + ilog2((uint64_t)(n / 3));
     long long m3 = 3LL << F3_MIN_K;
     while (m3 < 2 * n - 1) m3 <<= 1;
-    const long long min3 = cols ? (3LL << F3_MIN_K) : (3LL << F3_ROW_MIN_K);
-    if (m3 < m && m3 >= min3 && m3 <= (3LL << F3_MAX_K)) return F3_BASE + ilog2((uint64_t)(m3 / 3));
+    const int k3 = ilog2((uint64_t)(m3 / 3));
+    if (m3 < m && k3 >= (cols ? F3_MIN_K : F3_ROW_MIN_K) && k3 <= F3_MAX_K) return F3_BASE + k3;
     return ilog2((uint64_t)m);
 }
 
@@ -183,10 +183,13 @@ Context::Context(int device) : device_(device)
     hip_check(warm_batch(word, gen_stream_), "kernel load");
     hip_check(hipStreamSynchronize(gen_stream_), "kernel load");
     noalloc_setup(device);
-    // default tile shapes: wide tiles for columns of 1024 points and more
+    // default tile shapes: wide tiles for columns of 1024 points and more, and for rows with an X2 form
     for (int i = 0; i < NSHAPES; ++i) {
         const int shape = i <= MAX_LOGM ? i : F3_BASE + F3_MIN_K + (i - MAX_LOGM - 1);
-        for (int b = 0; b < 2; ++b) variant_[i][b][1] = (m_of(shape) >= 1024) ? 1 : 0;
+        for (int b = 0; b < 2; ++b) {
+            variant_[i][b][0] = has_x2(shape) ? 1 : 0;
+            variant_[i][b][1] = (m_of(shape) >= 1024) ? 1 : 0;
+        }
     }
 }
 
@@ -593,18 +596,17 @@ void Context::enqueue_axis(const LinePlan& lp, const float2* src, float2* dst, i
         return;
     }
     const AxisJob j = make_job(lp, src, dst, es, ls, count, inverse);
-    hip_check(launch_axis(lp.shape, j, lp.blue, cols, tile_threads(lp.shape, lp.blue, cols, count), stream),
-              "axis pass launch");
+    const int threads = tile_threads(lp.shape, lp.blue, cols, count);
+    hip_check(launch_axis(lp.shape, j, lp.blue, cols, threads, stream), "axis pass launch");
 }
 
 bool Context::wide_tiles(int shape, bool blue, bool cols, int count) const
 {
     if (variant(shape, blue, cols) == 0) return false;
-    // wide tiles hold 4x the lines of narrow ones; keep at least one tile per CU
-    const int tpl = tpl_of(shape);
-    const int lines_wide = tpl >= 1024 ? 1 : 1024 / tpl;
+    // keep at least one tile per CU (rows: the four that run at a time)
+    const int lines_wide = wide_threads(shape, cols) / tpl_of(shape) * lines_per_thread(wide_shape(shape));
     const int64_t tiles = (int64_t(count) + lines_wide - 1) / lines_wide;
-    return tiles >= int64_t(cu_count_);
+    return tiles >= int64_t(cols ? 1 : 4) * cu_count_;
 }
 
 int Context::tile_threads(int shape, bool blue, bool cols, int count) const

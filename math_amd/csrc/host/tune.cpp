@@ -36,13 +36,6 @@ float time_launches(hipStream_t s, F&& fn, int reps)
     return ms / reps;
 }
 
-int tile_threads(int shape, bool wide)
-{
-    const int tpl = mdft::tpl_of(shape);
-    const int base = wide ? 1024 : 256;
-    return tpl > base ? tpl : base;
-}
-
 // every FFT shape of the tile kernels: powers of two, then 3 * 2^k
 std::vector<int> all_shapes()
 {
@@ -55,7 +48,7 @@ std::vector<int> all_shapes()
 bool valid_shape(int shape)
 {
     return (shape >= 1 && shape <= mdft::MAX_LOGM) ||
-           (mdft::is_f3(shape) && mdft::f3_k(shape) >= mdft::F3_MIN_K && mdft::f3_k(shape) <= mdft::F3_MAX_K);
+           (shape >= mdft::F3_BASE + mdft::F3_MIN_K && shape <= mdft::F3_BASE + mdft::F3_MAX_K);
 }
 
 }  // namespace
@@ -76,7 +69,6 @@ int mdft_tune_auto(double* seconds)
     mdft::hip_check(hipMemsetAsync(buf, 0, sizeof(float2) * BUF_ELEMS, s), "hipMemsetAsync");
     try {
         for (int shape : all_shapes()) {
-            if (tile_threads(shape, false) == tile_threads(shape, true)) continue;  // one tile size only
             const int m = mdft::m_of(shape);
             for (int blue = 0; blue < 2; ++blue) {
                 if (blue && shape < 2) continue;
@@ -84,9 +76,7 @@ int mdft_tune_auto(double* seconds)
                 // power-of-two Bluestein convolution, m/2 - 1 for a 3 * 2^k one
                 // (m/2 = 3 * 2^(k-1) may itself be a direct length)
                 const int n = !blue ? m : mdft::is_f3(shape) ? m / 2 - 1 : m / 2 + 1;
-                // 3 * 2^k convolutions are only chosen for columns; the tile
-                // kernels of a shape are tuned along both axes all the same
-                auto lp = ctx.line_plan(n, mdft::is_f3(shape));
+                auto lp = ctx.line_plan(n, true);
                 if (lp->shape != shape) throw Error(MDFT_ERR_STATE, "tune: length " + std::to_string(n) +
                                                                         " does not have the shape being tuned");
                 const int count = (int)(BUF_ELEMS / (size_t)n);

@@ -33,37 +33,28 @@ hipError_t warm_batch(uint32_t* word, hipStream_t stream)
     if (e == hipSuccess) e = warm_batch_grid<512>(word, stream);
     if (e == hipSuccess) e = warm_batch_grid<1024>(word, stream);
     if (e == hipSuccess) e = warm_batch_persistent<256>(word, stream);
-    if (e == hipSuccess) e = warm_batch_persistent<512>(word, stream);
-    if (e == hipSuccess) e = warm_batch_persistent<1024>(word, stream);
     return e;
 }
 
-hipError_t launch_batch_persistent(int threads, const BatchJob* jobs, const uint2* items, uint32_t nitems,
-                                   uint32_t* ctl, uint32_t nctl, int grid, uint32_t spin_limit, hipStream_t stream)
+hipError_t launch_batch_persistent(const BatchJob* jobs, const uint2* items, uint32_t nitems, uint32_t* ctl,
+                                   uint32_t nctl, int grid, uint32_t spin_limit, hipStream_t stream)
 {
     if (nitems == 0) return hipSuccess;
     // clear ticket, error flag and counters with a kernel (graph-capture safe)
     hipLaunchKernelGGL(k_fill_u32, dim3((nctl + 255) / 256), dim3(256), 0, stream, ctl, nctl, 0u);
-    if (threads == 256) return launch_batch_persistent_t<256>(jobs, items, nitems, ctl, grid, spin_limit, stream);
-    if (threads == 512) return launch_batch_persistent_t<512>(jobs, items, nitems, ctl, grid, spin_limit, stream);
-    return launch_batch_persistent_t<1024>(jobs, items, nitems, ctl, grid, spin_limit, stream);
+    return launch_batch_persistent_t<256>(jobs, items, nitems, ctl, grid, spin_limit, stream);
 }
 
-int batch_lines_per_tile(int threads, int shape)
+int batch_lines_per_tile(int threads, int shape, bool cols)
 {
     if (shape < 1 || (!is_f3(shape) && shape > BATCH_MAXLOGM) ||
         (is_f3(shape) && (f3_k(shape) < F3_MIN_K || f3_k(shape) > F3_MAX_K)))
         return 0;
     const int tpl = tpl_of(shape);
-    return tpl <= threads ? threads / tpl : 0;
+    return tpl <= threads ? threads / tpl * lines_per_thread(batch_shape(shape, threads, cols)) : 0;
 }
 
-hipError_t batch_occupancy(int threads, int* blocks_per_cu)
-{
-    if (threads == 256) return batch_occupancy_t<256>(blocks_per_cu);
-    if (threads == 512) return batch_occupancy_t<512>(blocks_per_cu);
-    return batch_occupancy_t<1024>(blocks_per_cu);
-}
+hipError_t batch_occupancy(int* blocks_per_cu) { return batch_occupancy_t<256>(blocks_per_cu); }
 
 int batch_max_logm() { return BATCH_MAXLOGM; }
 

@@ -1,6 +1,8 @@
 // The batch kernels of one workgroup size: compiled once per size (MDFT_BATCH_T
-// = 256, 512, 1024) and launch shape (MDFT_BATCH_PERSISTENT_TU = 0, 1), since
-// each of the six holds every tile variant.
+// = 256, 512, 1024) and for 256 also as the persistent shapes
+// (MDFT_BATCH_PERSISTENT_TU = 1), since each holds many tile variants.  Row
+// tiles and whole images take 256 threads (a line of every batched length fits
+// those), so the larger sizes hold column tiles only.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -16,9 +18,9 @@ template <int T>
 __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(TILE_WAVES))) void k_batch_grid(
     const BatchJob* __restrict__ jobs, const uint2* __restrict__ items)
 {
-    __shared__ float lds[batch_lds<T>()];
+    __shared__ float lds[batch_lds<T, (T > 256)>()];
     // the host lays items out per XCD (block b runs on XCD b % 8)
-    run_item<T, true>(jobs, items[blockIdx.x], lds);
+    run_item<T, true, (T > 256)>(jobs, items[blockIdx.x], lds);
 }
 
 template <>
@@ -57,7 +59,7 @@ __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(TILE_WAVES)))
     const BatchJob* __restrict__ jobs, const uint2* __restrict__ items, uint32_t nitems, uint32_t* ctl,
     uint32_t spin_limit)
 {
-    __shared__ float lds[batch_lds<T>()];
+    __shared__ float lds[batch_lds<T, false>()];
     __shared__ uint32_t s_item;
     uint32_t* ticket = ctl;
     uint32_t* err = ctl + 1;
@@ -90,7 +92,7 @@ __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(TILE_WAVES)))
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         }
-        run_item<T, false>(jobs, item, lds);
+        run_item<T, false, false>(jobs, item, lds);
         if (bj.sig >= 0) {
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // release this wave's stores
             __syncthreads();

@@ -31,29 +31,39 @@
 
 namespace mdft {
 
-template <int S, int T>
+// The form of a shape a batch runs: two lines per thread where the shape has
+// that, along rows and in the column tiles of phase 2 (kernels of more than 256
+// threads, which hold columns only); one for the columns of phase 1 (small
+// whole images and single columns).
+__host__ __device__ constexpr int batch_shape(int s, int threads, bool cols)
+{
+    return has_x2(s) && (!cols || threads > 256) ? s | X2 : s;
+}
+
+template <int S, int T, bool COLS_ONLY>
 constexpr int lds_need()
 {
     if constexpr (tpl_of(S) > T) {
         return 0;
     } else {
-        constexpr int a = LineCfg<S, T>::template lds_floats<false>();
-        constexpr int b = LineCfg<S, T>::template lds_floats<true>();
+        constexpr int a = COLS_ONLY ? 0 : LineCfg<batch_shape(S, T, false), T>::template lds_floats<false>();
+        constexpr int b = LineCfg<batch_shape(S, T, true), T>::template lds_floats<true>();
         return a > b ? a : b;
     }
 }
 
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 
-template <int T>
+template <int T, bool C>
 constexpr int batch_lds()
 {
-    return cmax(cmax(cmax(cmax(lds_need<5, T>(), lds_need<6, T>()), cmax(lds_need<7, T>(), lds_need<8, T>())),
-                     cmax(cmax(cmax(lds_need<9, T>(), lds_need<10, T>()), cmax(lds_need<11, T>(), lds_need<12, T>())),
-                          lds_need<13, T>())),
-                cmax(cmax(cmax(lds_need<F3_BASE + 6, T>(), lds_need<F3_BASE + 7, T>()),
-                          cmax(lds_need<F3_BASE + 8, T>(), lds_need<F3_BASE + 9, T>())),
-                     cmax(lds_need<F3_BASE + 10, T>(), lds_need<F3_BASE + 11, T>())));
+    return cmax(cmax(cmax(cmax(lds_need<5, T, C>(), lds_need<6, T, C>()), cmax(lds_need<7, T, C>(), lds_need<8, T, C>())),
+                     cmax(cmax(cmax(lds_need<9, T, C>(), lds_need<10, T, C>()),
+                               cmax(lds_need<11, T, C>(), lds_need<12, T, C>())),
+                          lds_need<13, T, C>())),
+                cmax(cmax(cmax(lds_need<F3_BASE + 6, T, C>(), lds_need<F3_BASE + 7, T, C>()),
+                          cmax(lds_need<F3_BASE + 8, T, C>(), lds_need<F3_BASE + 9, T, C>())),
+                     cmax(lds_need<F3_BASE + 10, T, C>(), lds_need<F3_BASE + 11, T, C>())));
 }
 
 // One variant.  The thread and tile indices go through an empty asm of its own in every
@@ -67,23 +77,28 @@ __device__ __forceinline__ void run_variant(const AxisJob& job, int tile, float*
     line_tile<S, T, BLUE, COLS>(job, tile, lds, tid);
 }
 
-template <int S, int T>
+template <int S, int T, bool COLS>
+__device__ __forceinline__ void run_axis(const AxisJob& job, int blue, int tile, float* lds)
+{
+    if constexpr (S >= 2) {
+        if (blue) {
+            run_variant<batch_shape(S, T, COLS), T, true, COLS>(job, tile, lds);
+            return;
+        }
+    }
+    run_variant<batch_shape(S, T, COLS), T, false, COLS>(job, tile, lds);
+}
+
+template <int S, int T, bool COLS_ONLY>
 __device__ __forceinline__ void run_tile_body(const AxisJob& job, int blue, int cols, int tile, float* lds)
 {
     if constexpr (tpl_of(S) <= T) {
-        if constexpr (S >= 2) {
-            if (blue) {
-                if (cols)
-                    run_variant<S, T, true, true>(job, tile, lds);
-                else
-                    run_variant<S, T, true, false>(job, tile, lds);
-                return;
-            }
-        }
-        if (cols)
-            run_variant<S, T, false, true>(job, tile, lds);
+        if constexpr (COLS_ONLY)
+            run_axis<S, T, true>(job, blue, tile, lds);
+        else if (cols)
+            run_axis<S, T, true>(job, blue, tile, lds);
         else
-            run_variant<S, T, false, false>(job, tile, lds);
+            run_axis<S, T, false>(job, blue, tile, lds);
     }
 }
 
@@ -93,11 +108,11 @@ __device__ __noinline__ void run_tile_call(const BatchJob* jobs, uint32_t job, i
 // Grid kernels inline every variant (register allocation per region,
 // occupancy-constrained); the persistent kernels call them out of line, since
 // inlining into the ticket loop keeps too much alive across it.
-template <int S, int T, bool INL>
+template <int S, int T, bool INL, bool COLS_ONLY>
 __device__ __forceinline__ void run_tile(const BatchJob* jobs, uint32_t job, const BatchJob& bj, int tile, float* lds)
 {
     if constexpr (INL)
-        run_tile_body<S, T>(bj.job, bj.blue, bj.cols, tile, lds);
+        run_tile_body<S, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds);
     else
         run_tile_call<S, T>(jobs, job, tile, lds);
 }
@@ -121,39 +136,39 @@ __device__ __noinline__ void run_tile_call(const BatchJob* jobs, uint32_t job, i
 #pragma unroll
     for (size_t i = 0; i < sizeof(BatchJob) / 4; ++i) copy.w[i] = words[i];
     const BatchJob& bj = copy.job;
-    run_tile_body<S, T>(bj.job, bj.blue, bj.cols, __builtin_amdgcn_readfirstlane(tile), lds);
+    run_tile_body<S, T, false>(bj.job, bj.blue, bj.cols, __builtin_amdgcn_readfirstlane(tile), lds);
 }
 
-template <int T, bool INL>
+template <int T, bool INL, bool COLS_ONLY>
 __device__ __forceinline__ void run_job_tile(const BatchJob* jobs, uint32_t job, int tile, float* lds)
 {
     const BatchJob bj = jobs[job];
     switch (bj.shape) {
-    case 1: run_tile<1, T, INL>(jobs, job, bj, tile, lds); break;
-    case 2: run_tile<2, T, INL>(jobs, job, bj, tile, lds); break;
-    case 3: run_tile<3, T, INL>(jobs, job, bj, tile, lds); break;
-    case 4: run_tile<4, T, INL>(jobs, job, bj, tile, lds); break;
-    case 5: run_tile<5, T, INL>(jobs, job, bj, tile, lds); break;
-    case 6: run_tile<6, T, INL>(jobs, job, bj, tile, lds); break;
-    case 7: run_tile<7, T, INL>(jobs, job, bj, tile, lds); break;
-    case 8: run_tile<8, T, INL>(jobs, job, bj, tile, lds); break;
-    case 9: run_tile<9, T, INL>(jobs, job, bj, tile, lds); break;
-    case 10: run_tile<10, T, INL>(jobs, job, bj, tile, lds); break;
-    case 11: run_tile<11, T, INL>(jobs, job, bj, tile, lds); break;
-    case 12: run_tile<12, T, INL>(jobs, job, bj, tile, lds); break;
-    case 13: run_tile<13, T, INL>(jobs, job, bj, tile, lds); break;
-    case F3_BASE + 6: run_tile<F3_BASE + 6, T, INL>(jobs, job, bj, tile, lds); break;
-    case F3_BASE + 7: run_tile<F3_BASE + 7, T, INL>(jobs, job, bj, tile, lds); break;
-    case F3_BASE + 8: run_tile<F3_BASE + 8, T, INL>(jobs, job, bj, tile, lds); break;
-    case F3_BASE + 9: run_tile<F3_BASE + 9, T, INL>(jobs, job, bj, tile, lds); break;
-    case F3_BASE + 10: run_tile<F3_BASE + 10, T, INL>(jobs, job, bj, tile, lds); break;
-    case F3_BASE + 11: run_tile<F3_BASE + 11, T, INL>(jobs, job, bj, tile, lds); break;
+    case 1: run_tile<1, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case 2: run_tile<2, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case 3: run_tile<3, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case 4: run_tile<4, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case 5: run_tile<5, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case 6: run_tile<6, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case 7: run_tile<7, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case 8: run_tile<8, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case 9: run_tile<9, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case 10: run_tile<10, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case 11: run_tile<11, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case 12: run_tile<12, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case 13: run_tile<13, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case F3_BASE + 6: run_tile<F3_BASE + 6, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case F3_BASE + 7: run_tile<F3_BASE + 7, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case F3_BASE + 8: run_tile<F3_BASE + 8, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case F3_BASE + 9: run_tile<F3_BASE + 9, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case F3_BASE + 10: run_tile<F3_BASE + 10, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case F3_BASE + 11: run_tile<F3_BASE + 11, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
     default: break;
     }
 }
 
 // One item; every branch is on a wave-uniform value.
-template <int T, bool INL>
+template <int T, bool INL, bool COLS_ONLY>
 __device__ __forceinline__ void run_item(const BatchJob* __restrict__ jobs, uint2 item, float* lds)
 {
     const uint32_t x = __builtin_amdgcn_readfirstlane(item.x);
@@ -163,7 +178,7 @@ __device__ __forceinline__ void run_item(const BatchJob* __restrict__ jobs, uint
     uint32_t job = x;
     int tile = whole ? 0 : (int)y;
     for (int turn = 0;; ++turn) {
-        run_job_tile<T, INL>(jobs, job, tile, lds);
+        run_job_tile<T, INL, COLS_ONLY>(jobs, job, tile, lds);
         if (!whole || turn == 1) break;
         // the column tile reads what this workgroup's waves just stored
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");

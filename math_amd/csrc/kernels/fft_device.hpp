@@ -77,27 +77,43 @@ __device__ __forceinline__ float2 cscale(float2 a, float s) { return make_float2
 //    radix-12 pass (a 3 x 4 prime-factor butterfly).
 // The shape is a function of the line length and axis, so a line runs the
 // same schedule in every kernel.
+// S + X2: the same with two lines per thread.  The lines of a tile share the
+// chirp, the diagonal and the twiddles at a position, which one line per thread
+// loads anew for every line (42 of the 60 loads of a Bluestein line's thread);
+// a thread with two lines loads them once for both, reads two adjacent columns
+// with one 16-byte load, and a tile has twice the columns (runs of a row twice
+// as long) on the same LDS, the lines exchanging one after the other.
 constexpr int MAX_LOGM = 14;
+constexpr int X2 = 64;
+__host__ __device__ constexpr int base_of(int s) { return s & 63; }
+__host__ __device__ constexpr int lines_per_thread(int s) { return (s & X2) ? 2 : 1; }
 // waves per SIMD the tile kernels are compiled for (at most 128 VGPRs)
 constexpr int TILE_WAVES = 4;
 constexpr int F3_BASE = 32;
 constexpr int F3_MIN_K = 6;   // M = 192: the radix-12 pass follows at least two radix-4 passes
-constexpr int F3_MAX_K = 11;  // M = 6144: 512 threads per line
-__host__ __device__ constexpr bool is_f3(int s) { return s >= F3_BASE; }
-__host__ __device__ constexpr int f3_k(int s) { return s - F3_BASE; }
+constexpr int F3_MAX_K = 11;  // M = 6144: 24 points per thread, 256 threads per line
+__host__ __device__ constexpr bool is_f3(int s) { return base_of(s) >= F3_BASE; }
+__host__ __device__ constexpr int f3_k(int s) { return base_of(s) - F3_BASE; }
 // 8192 and 16384 points: 32 per thread
-__host__ __device__ constexpr bool is_wide(int s) { return s == 13 || s == 14; }
-__host__ __device__ constexpr int m_of(int s) { return is_f3(s) ? (3 << f3_k(s)) : (1 << s); }
-// points per thread
+__host__ __device__ constexpr bool is_wide(int s) { return base_of(s) == 13 || base_of(s) == 14; }
+// shapes with an X2 form: from 1024 points a 256-thread tile holds at most four lines
+__host__ __device__ constexpr bool has_x2(int s)
+{
+    return (base_of(s) >= 10 && base_of(s) <= 12) || (is_f3(s) && (f3_k(s) == 9 || f3_k(s) == 10));
+}
+__host__ __device__ constexpr int m_of(int s) { return is_f3(s) ? (3 << f3_k(s)) : (1 << base_of(s)); }
+// points of a line per thread
 __host__ __device__ constexpr int ept_of(int s)
 {
-    return is_f3(s) ? 12 : is_wide(s) ? 32 : s < 4 ? (1 << s) : 16;
+    return is_f3(s) ? (f3_k(s) == 11 ? 24 : 12) : is_wide(s) ? 32 : base_of(s) < 4 ? (1 << base_of(s)) : 16;
 }
 // threads per line
 __host__ __device__ constexpr int tpl_of(int s) { return m_of(s) / ept_of(s); }
 __host__ __device__ constexpr int npass_of(int s)
 {
-    return is_f3(s) ? (f3_k(s) - 2) / 2 + (f3_k(s) - 2) % 2 + 1 : is_wide(s) ? 3 : (s + 3) / 4;
+    return is_f3(s)     ? (f3_k(s) - 2) / 2 + (f3_k(s) - 2) % 2 + 1
+           : is_wide(s) ? 3
+                        : (base_of(s) + 3) / 4;
 }
 // radix of pass p (1 when p is past the last pass)
 __host__ __device__ constexpr int radix_of(int s, int p)
@@ -107,8 +123,8 @@ __host__ __device__ constexpr int radix_of(int s, int p)
         const int a = f3_k(s) - 2;
         return p < a / 2 ? 4 : (p == npass_of(s) - 1 ? 12 : 2);
     }
-    if (is_wide(s)) return p == 0 || (s == 14 && p == 1) ? 32 : 16;
-    return 1 << ((s - 4 * p) >= 4 ? 4 : (s - 4 * p));
+    if (is_wide(s)) return p == 0 || (base_of(s) == 14 && p == 1) ? 32 : 16;
+    return 1 << ((base_of(s) - 4 * p) >= 4 ? 4 : (base_of(s) - 4 * p));
 }
 // Stockham stride before pass p: the product of the earlier radices
 __host__ __device__ constexpr int ns_of(int s, int p)
@@ -157,7 +173,7 @@ __host__ __device__ constexpr int64_t tw_len(int s)
 __host__ __device__ constexpr int64_t tw_off(int s)
 {
     int64_t t = 0;
-    const int plast = is_f3(s) ? MAX_LOGM + 1 : s;
+    const int plast = is_f3(s) ? MAX_LOGM + 1 : base_of(s);
     for (int l = 1; l < plast; ++l) t += tw_len(l);
     if (is_f3(s))
         for (int k = F3_MIN_K; k < f3_k(s); ++k) t += tw_len(F3_BASE + k);
@@ -181,7 +197,7 @@ constexpr LdsMap kLdsMaps[] = {
 __host__ __device__ constexpr LdsMap lds_map(int shape, int threads, bool cols, int pass)
 {
     for (const LdsMap& e : kLdsMaps)
-        if (e.shape == shape && e.threads == threads && e.cols == (cols ? 1 : 0) && e.pass == pass) return e;
+        if (e.shape == base_of(shape) && e.threads == threads && e.cols == (cols ? 1 : 0) && e.pass == pass) return e;
     return LdsMap{shape, threads, cols ? 1 : 0, pass, -1, 0};  // missing: rejected by a static_assert
 }
 template <int S, int THREADS, bool COLS, int P>
@@ -197,12 +213,15 @@ struct LineCfg {
     static constexpr int M = m_of(S);
     static constexpr int EPT = ept_of(S);
     static constexpr int TPL = tpl_of(S);        // threads per line
-    static constexpr int LPW = THREADS / TPL;    // lines per tile
+    static constexpr int L = lines_per_thread(S);
+    static constexpr int SLOTS = THREADS / TPL;  // lines side by side in the workgroup
+    static constexpr int LPW = SLOTS * L;        // lines per tile
     static constexpr int NPASS = npass_of(S);
     // exchange the real parts, then the imaginary parts, through one plane
     static constexpr bool SPLIT = EPT > 16;
+    static_assert(!SPLIT || L == 1, "32 points per thread: one line");
     static_assert(TPL <= THREADS, "line does not fit the workgroup");
-    static_assert(LPW * TPL == THREADS, "workgroup must hold whole lines");
+    static_assert(SLOTS * TPL == THREADS, "workgroup must hold whole lines");
     // words of one line's slice: the largest padded position over the exchanges
     template <bool COLS, int P = 0>
     static constexpr int padm()
@@ -217,12 +236,12 @@ struct LineCfg {
     }
     // Line stride in LDS words.  Lanes of one wave cover q consecutive
     // positions of 32/q lines (rows: q = TPL; columns, lines fastest:
-    // q = 32/LPW); a stride of q times an odd number puts them on distinct
+    // q = 32/SLOTS); a stride of q times an odd number puts them on distinct
     // banks (the same rule gen_lds_maps.py assumes).
     template <bool COLS>
     static constexpr int lstride()
     {
-        const int q = COLS ? (LPW >= 32 ? 1 : 32 / LPW) : (TPL >= 32 ? 0 : TPL);
+        const int q = COLS ? (SLOTS >= 32 ? 1 : 32 / SLOTS) : (TPL >= 32 ? 0 : TPL);
         const int pm = padm<COLS>();
         if (q == 0) return pm;
         int s = pm;
@@ -232,7 +251,7 @@ struct LineCfg {
     template <bool COLS>
     static constexpr int lds_floats()
     {
-        return NPASS > 1 ? (SPLIT ? 1 : 2) * LPW * lstride<COLS>() : 0;
+        return NPASS > 1 ? (SPLIT ? 1 : 2) * SLOTS * lstride<COLS>() : 0;
     }
 };
 
@@ -556,6 +575,18 @@ __device__ __forceinline__ float2 load_global(const float2* p)
     return make_float2(x.x, x.y);
 }
 __device__ __forceinline__ void store_global(float2* p, float2 x) { *(MDFT_GLOBAL vec2*)p = vec2{x.x, x.y}; }
+// two adjacent elements (global accesses need no more than 4-byte alignment)
+typedef float vec4_8 __attribute__((ext_vector_type(4), aligned(8)));
+__device__ __forceinline__ void load_pair(const float2* p, float2& a, float2& b)
+{
+    const vec4 x = *(const MDFT_GLOBAL vec4_8*)p;
+    a = make_float2(x.x, x.y);
+    b = make_float2(x.z, x.w);
+}
+__device__ __forceinline__ void store_pair(float2* p, float2 a, float2 b)
+{
+    *(MDFT_GLOBAL vec4_8*)p = vec4{a.x, a.y, b.x, b.y};
+}
 // At a uniform address (p must not depend on the lane) plus a 32-bit element
 // index: the address is kept in scalar registers, so every slot's access takes
 // its offset from one vector register; left to itself the compiler adds each
@@ -685,6 +716,8 @@ struct FftPass {
     static constexpr int LST = C::template lstride<COLS>();
     static_assert(NB * R == C::EPT, "the radix divides the points per thread");
 
+    using Regs = float2 (&)[C::L][C::EPT];  // the thread's lines
+
     // Stockham positions of this pass's outputs, component c
     template <int c>
     __device__ __forceinline__ static void scatter(const float2 (&v)[C::EPT], int t, float* plane)
@@ -718,33 +751,36 @@ struct FftPass {
         }
     }
 
-    __device__ __forceinline__ static void exchange(float2 (&v)[C::EPT], int t, float* re, float* im)
+    __device__ __forceinline__ static void exchange(Regs v, int t, float* re, float* im)
     {
-        exchange_sync<WAVE>();  // the previous exchange's reads are done
-        if constexpr (C::SPLIT) {
-            scatter<0>(v, t, re);
-            exchange_sync<WAVE>();
-            gather<0>(v, t, re);
-            exchange_sync<WAVE>();
-            scatter<1>(v, t, re);
-            exchange_sync<WAVE>();
-            gather<1>(v, t, re);
-        } else {
-            scatter<0>(v, t, re);
-            scatter<1>(v, t, im);
-            exchange_sync<WAVE>();
-            gather<0>(v, t, re);
-            gather<1>(v, t, im);
+#pragma unroll
+        for (int l = 0; l < C::L; ++l) {
+            exchange_sync<WAVE>();  // the previous exchange's reads are done
+            if constexpr (C::SPLIT) {
+                scatter<0>(v[l], t, re);
+                exchange_sync<WAVE>();
+                gather<0>(v[l], t, re);
+                exchange_sync<WAVE>();
+                scatter<1>(v[l], t, re);
+                exchange_sync<WAVE>();
+                gather<1>(v[l], t, re);
+            } else {
+                scatter<0>(v[l], t, re);
+                scatter<1>(v[l], t, im);
+                exchange_sync<WAVE>();
+                gather<0>(v[l], t, re);
+                gather<1>(v[l], t, im);
+            }
         }
     }
 
     template <class Epi>
-    __device__ __forceinline__ static void run(float2 (&v)[C::EPT], int t, float* re, float* im, const float2* tw,
+    __device__ __forceinline__ static void run(Regs v, int t, float* re, float* im, const float2* tw,
                                                float4 (&w)[C::EPT / 2], const float2* pfs, float2 (&pf)[C::EPT],
                                                const Epi& epi)
     {
         static_assert(PF <= C::EPT && PFL <= C::EPT, "prefetch slots");
-        if constexpr (PF > 0 && C::NPASS == 1) {
+        if constexpr ((PF > 0 || PFL > 0) && C::NPASS == 1) {
 #pragma unroll
             for (int i = 0; i < (PFL > PF ? PFL : PF); ++i) pf[i] = load_at(pfs + i * C::TPL, uint32_t(t));
         }
@@ -763,31 +799,35 @@ struct FftPass {
                     if (b + NB * r < EL) tab[r] = load_at(pfs + (b + NB * r) * C::TPL, uint32_t(t));
             }
 #pragma unroll
-            for (int r = 0; r < R; ++r) u[r] = v[b + NB * r];
-            if constexpr (P > 0) {
-                constexpr int Q = tw_quads<R>();
-                float4 q[Q];
+            for (int l = 0; l < C::L; ++l) {
 #pragma unroll
-                for (int r2 = 0; r2 < Q; ++r2) q[r2] = w[b * Q + r2];
-                if constexpr (R == 16 || R == 32) {
-                    dft_twiddled<R>(u, q);
+                for (int r = 0; r < R; ++r) u[r] = v[l][b + NB * r];
+                if constexpr (P > 0) {
+                    // the same for the thread's lines
+                    constexpr int Q = tw_quads<R>();
+                    float4 q[Q];
+#pragma unroll
+                    for (int r2 = 0; r2 < Q; ++r2) q[r2] = w[b * Q + r2];
+                    if constexpr (R == 16 || R == 32) {
+                        dft_twiddled<R>(u, q);
+                    } else {
+                        float2 wt[R];
+                        expand_twiddles<R>(wt, q);
+#pragma unroll
+                        for (int r = 1; r < R; ++r) u[r] = cmul(u[r], wt[r]);
+                        dft_fwd<R>(u);
+                    }
                 } else {
-                    float2 wt[R];
-                    expand_twiddles<R>(wt, q);
-#pragma unroll
-                    for (int r = 1; r < R; ++r) u[r] = cmul(u[r], wt[r]);
-                    dft_fwd<R>(u);
+                    // ZIN: slot b + NB*r holds a zero for r > R/2 (b + NB*(R/2 + 1) >= EPT/2 + 1)
+                    dft_fwd<R, ZIN>(u);
                 }
-            } else {
-                // ZIN: slot b + NB*r holds a zero for r > R/2 (b + NB*(R/2 + 1) >= EPT/2 + 1)
-                dft_fwd<R, ZIN>(u);
-            }
-            static_assert(!ZIN || P == 0, "zero inputs only in the first pass");
+                static_assert(!ZIN || P == 0, "zero inputs only in the first pass");
 #pragma unroll
-            for (int r = 0; r < R; ++r) v[b + NB * r] = u[r];
+                for (int r = 0; r < R; ++r) v[l][b + NB * r] = u[r];
+            }
             if constexpr (LAST && C::SPLIT) {
 #pragma unroll
-                for (int r = 0; r < R; ++r) epi(b + NB * r, v[b + NB * r], tab[r]);
+                for (int r = 0; r < R; ++r) epi(b + NB * r, v[0][b + NB * r], tab[r]);
             }
             // one butterfly's operands at a time: without it the scheduler
             // starts the next one's loads early and spills
@@ -821,34 +861,36 @@ struct NoEpilogue {
 template <int S, int THREADS, bool COLS, bool ZIN = false, int PF = 0, int PFL = 0>
 struct FftTile {
     using C = LineCfg<S, THREADS>;
-    __device__ __forceinline__ static void run(float2 (&v)[C::EPT], int t, int ll, float* lds, const float2* tw)
+    using Regs = float2 (&)[C::L][C::EPT];
+    // no table: one line per thread
+    __device__ __forceinline__ static void run(float2 (&v)[C::EPT], int t, int slot, float* lds, const float2* tw)
     {
-        static_assert(PF == 0 && PFL == 0, "prefetch needs a destination");
+        static_assert(PF == 0 && PFL == 0 && C::L == 1, "prefetch needs a destination");
         float2 pf[C::EPT];
-        run_all<0>(v, t, ll, lds, tw, nullptr, pf, NoEpilogue{});
+        run_all<0>(reinterpret_cast<Regs>(v), t, slot, lds, tw, nullptr, pf, NoEpilogue{});
     }
-    __device__ __forceinline__ static void run(float2 (&v)[C::EPT], int t, int ll, float* lds, const float2* tw,
+    __device__ __forceinline__ static void run(Regs v, int t, int slot, float* lds, const float2* tw,
                                                const float2* pfs, float2 (&pf)[C::EPT])
     {
-        run_all<0>(v, t, ll, lds, tw, pfs, pf, NoEpilogue{});
+        run_all<0>(v, t, slot, lds, tw, pfs, pf, NoEpilogue{});
     }
     template <int EL, class Epi>
-    __device__ __forceinline__ static void run_epi(float2 (&v)[C::EPT], int t, int ll, float* lds, const float2* tw,
+    __device__ __forceinline__ static void run_epi(Regs v, int t, int slot, float* lds, const float2* tw,
                                                    const float2* pfs, const Epi& epi)
     {
         static_assert(C::SPLIT && PF == 0 && PFL == 0, "split exchange only");
         float2 pf[C::EPT];
-        run_all<EL>(v, t, ll, lds, tw, pfs, pf, epi);
+        run_all<EL>(v, t, slot, lds, tw, pfs, pf, epi);
     }
 
 private:
     template <int EL, class Epi>
-    __device__ __forceinline__ static void run_all(float2 (&v)[C::EPT], int t, int ll, float* lds, const float2* tw,
+    __device__ __forceinline__ static void run_all(Regs v, int t, int slot, float* lds, const float2* tw,
                                                    const float2* pfs, float2 (&pf)[C::EPT], const Epi& epi)
     {
         constexpr int LST = C::template lstride<COLS>();
-        float* re = lds + ll * LST;
-        float* im = C::SPLIT ? re : re + C::LPW * LST;
+        float* re = lds + slot * LST;
+        float* im = C::SPLIT ? re : re + C::SLOTS * LST;
         float4 w[C::EPT / 2];
         if constexpr (!C::SPLIT && C::NPASS > 1) TwLoad<S, THREADS, 1>::run(w, t, tw);
         FftPass<S, THREADS, COLS, 0, ZIN, PF, PFL, EL>::run(v, t, re, im, tw, w, pfs, pf, epi);
@@ -865,10 +907,15 @@ template <int S, int THREADS, bool BLUE, bool COLS, int IO = 0>
 __device__ __forceinline__ void line_tile(const AxisJob& job, int tile, float* lds, int tid, ImageIO io = ImageIO{})
 {
     using C = LineCfg<S, THREADS>;
-    const int ll = COLS ? (tid % C::LPW) : (tid / C::TPL);
-    const int t = COLS ? (tid / C::LPW) : (tid % C::TPL);
-    const int line = tile * C::LPW + ll;
-    const bool valid = line < job.count;
+    constexpr int L = C::L;
+    static_assert(IO == 0 || L == 1 || (COLS && (IO & IO_LUM) == 0), "image input: one line per thread");
+    const int slot = COLS ? (tid % C::SLOTS) : (tid / C::TPL);
+    const int t = COLS ? (tid / C::SLOTS) : (tid % C::TPL);
+    // the thread's lines: adjacent columns, or rows SLOTS apart
+    auto line_of = [&](int l) { return tile * C::LPW + (COLS ? slot * L + l : l * C::SLOTS + slot); };
+    auto valid = [&](int l) { return line_of(l) < job.count; };
+    // two columns of a tile without a missing column: 16-byte accesses
+    const bool pairs = COLS && L == 2 && (tile + 1) * C::LPW <= job.count;
     const int n = job.n;
     // Consecutive slots of a thread are TPL elements apart.  A column steps by
     // the image width: 64-bit addresses.  Rows are contiguous, and like the
@@ -877,9 +924,14 @@ __device__ __forceinline__ void line_tile(const AxisJob& job, int tile, float* l
     // elements, and one register serves every slot.
     const int64_t step = COLS ? int64_t(C::TPL) * job.es : int64_t(C::TPL);
     // (a line past the last one reads the tile's first line and stores nothing)
-    const int64_t base = COLS ? int64_t(valid ? line : tile * C::LPW) * job.ls + int64_t(t) * job.es
-                              : int64_t(tile) * C::LPW * job.ls;
-    const uint32_t off = COLS ? 0u : valid ? uint32_t(ll) * uint32_t(job.ls) + uint32_t(t) : uint32_t(t);
+    int64_t base[L];
+    uint32_t off[L];
+#pragma unroll
+    for (int l = 0; l < L; ++l) {
+        base[l] = COLS ? int64_t(valid(l) ? line_of(l) : tile * C::LPW) * job.ls + int64_t(t) * job.es
+                       : int64_t(tile) * C::LPW * job.ls;
+        off[l] = COLS ? 0u : valid(l) ? uint32_t(line_of(l) - tile * C::LPW) * uint32_t(job.ls) + uint32_t(t) : uint32_t(t);
+    }
     // direction enters as a sign mask: conjugation is one xor, and the
     // inverse's 1/n is a multiply by job.scale (exactly 1 for the forward)
     const uint32_t sgn = job.inverse ? 0x80000000u : 0u;
@@ -900,97 +952,128 @@ __device__ __forceinline__ void line_tile(const AxisJob& job, int tile, float* l
     // every live slot (dir_tables_len).  The line fills more than a quarter (a
     // third for 3 * 2^k) of the FFT, so the first slots need no check.
     constexpr int SURE = BLUE ? (is_f3(S) ? C::EPT / 3 : C::EPT / 4) : C::EPT;
-    float2 v[C::EPT];
+    float2 v[L][C::EPT];
     {
-        const float2* s = job.src + base;
         float2 c[LIVE];
+        if (pairs) {
+            const float2* s = job.src + base[0];
 #pragma unroll
-        for (int i = 0; i < LIVE; ++i) {
-            const bool in = i < SURE || t + i * C::TPL < n;
-            if constexpr ((IO & IO_LUM) != 0) {
-                const int64_t pos = in ? t + i * C::TPL : t;
-                v[i] = make_float2(image_luminance(io, int64_t(valid ? line : tile * C::LPW) * io.ils + pos * io.iel),
-                                   0.0f);
-            } else {
+            for (int i = 0; i < LIVE; ++i) {
+                const bool in = i < SURE || t + i * C::TPL < n;
                 // opaque: else the select becomes a branch around the load
-                if constexpr (COLS)
-                    v[i] = load_global(i < SURE ? s + i * step : s + opaque(in ? i * step : 0));
-                else
-                    v[i] = i < SURE ? load_at(s + i * step, off)
-                                    : load_at(s, opaque(in ? off + uint32_t(i * C::TPL) : off));
+                load_pair(i < SURE ? s + i * step : s + opaque(in ? i * step : 0), v[0][i], v[L - 1][i]);
             }
-            if constexpr (BLUE) c[i] = load_at(job.chirp + i * C::TPL, uint32_t(t));
+        } else {
+#pragma unroll
+            for (int i = 0; i < LIVE; ++i) {
+                const bool in = i < SURE || t + i * C::TPL < n;
+#pragma unroll
+                for (int l = 0; l < L; ++l) {
+                    const float2* s = job.src + base[l];
+                    if constexpr ((IO & IO_LUM) != 0) {
+                        const int64_t pos = in ? t + i * C::TPL : t;
+                        const int64_t line = valid(l) ? line_of(l) : tile * C::LPW;
+                        v[l][i] = make_float2(image_luminance(io, line * io.ils + pos * io.iel), 0.0f);
+                    } else if constexpr (COLS) {
+                        v[l][i] = load_global(i < SURE ? s + i * step : s + opaque(in ? i * step : 0));
+                    } else {
+                        v[l][i] = i < SURE ? load_at(s + i * step, off[l])
+                                           : load_at(s, opaque(in ? off[l] + uint32_t(i * C::TPL) : off[l]));
+                    }
+                }
+            }
+        }
+        if constexpr (BLUE) {
+#pragma unroll
+            for (int i = 0; i < LIVE; ++i) c[i] = load_at(job.chirp + i * C::TPL, uint32_t(t));
         }
 #pragma unroll
-        for (int i = 0; i < C::EPT; ++i) {
-            if (i >= LIVE) {
-                v[i] = make_float2(0.0f, 0.0f);
-            } else if constexpr (BLUE) {
-                // forward x*c, inverse x*conj(c) (direction tables)
-                const bool in = i < SURE || t + i * C::TPL < n;
-                const float2 x = cmul(v[i], c[i]);
-                v[i] = in ? x : make_float2(0.0f, 0.0f);
-            } else {
-                v[i] = cxor(v[i], sgn);  // conj for the inverse
+        for (int l = 0; l < L; ++l) {
+#pragma unroll
+            for (int i = 0; i < C::EPT; ++i) {
+                if (i >= LIVE) {
+                    v[l][i] = make_float2(0.0f, 0.0f);
+                } else if constexpr (BLUE) {
+                    // forward x*c, inverse x*conj(c) (direction tables)
+                    const bool in = i < SURE || t + i * C::TPL < n;
+                    const float2 x = cmul(v[l][i], c[i]);
+                    v[l][i] = in ? x : make_float2(0.0f, 0.0f);
+                } else {
+                    v[l][i] = cxor(v[l][i], sgn);  // conj for the inverse
+                }
             }
         }
     }
 
-    float2* o = job.dst + base;
     const float sc = job.scale;
-    // finished slot i into the output
-    auto put = [&](int i, float2 y) {
+    // finished slot i of the thread's lines into the output
+    auto put = [&](int i, const float2 (&y)[L]) {
         const uint32_t pos = uint32_t(t + i * C::TPL);
-        if (!valid || !in_line((int)pos)) return;
-        if constexpr ((IO & IO_MAG) != 0)
-            io.mag[int64_t(line) * io.mls + int64_t(pos) * io.mel] = cabs_scaled(y, io.mscale);
-        else if constexpr (COLS)
-            store_global(o + i * step, y);
-        else
-            store_at(o + i * step, off, y);
+        if (!in_line((int)pos)) return;
+        if constexpr (IO == 0 && L == 2) {
+            if (pairs) {
+                store_pair(job.dst + base[0] + i * step, y[0], y[L - 1]);
+                return;
+            }
+        }
+#pragma unroll
+        for (int l = 0; l < L; ++l) {
+            if (!valid(l)) continue;
+            if constexpr ((IO & IO_MAG) != 0)
+                io.mag[int64_t(line_of(l)) * io.mls + int64_t(pos) * io.mel] = cabs_scaled(y[l], io.mscale);
+            else if constexpr (COLS)
+                store_global(job.dst + base[l] + i * step, y[l]);
+            else
+                store_at(job.dst + base[l] + i * step, off[l], y[l]);
+        }
     };
 
     if constexpr (C::SPLIT) {
         if constexpr (BLUE) {
             // the products of the branch below, slot by slot in the last passes
             FftTile<S, THREADS, COLS, ZIN>::template run_epi<C::EPT>(
-                v, t, ll, lds, job.tw, job.dtab, [&](int, float2& x, float2 d) { x = cmul_conj(x, d); });
-            FftTile<S, THREADS, COLS>::template run_epi<LIVE>(v, t, ll, lds, job.tw, job.chirp_out,
+                v, t, slot, lds, job.tw, job.dtab, [&](int, float2& x, float2 d) { x = cmul_conj(x, d); });
+            FftTile<S, THREADS, COLS>::template run_epi<LIVE>(v, t, slot, lds, job.tw, job.chirp_out,
                                                                [&](int i, float2& x, float2 c) {
-                                                                   if (i < LIVE) put(i, cmul_conj(x, c));
+                                                                   if (i < LIVE) put(i, {cmul_conj(x, c)});
                                                                });
         } else {
             FftTile<S, THREADS, COLS>::template run_epi<0>(
-                v, t, ll, lds, job.tw, nullptr, [&](int i, float2& x, float2) { put(i, cscale(cxor(x, sgn), sc)); });
+                v, t, slot, lds, job.tw, nullptr,
+                [&](int i, float2& x, float2) { put(i, {cscale(cxor(x, sgn), sc)}); });
         }
     } else {
         // Bluestein: D arrives during the first FFT, its first half one pass
         // before the end and the rest at the start of the last pass (earlier
-        // loads of all of D spill at the 128-VGPR cap), and the live slots of
-        // the output chirp during the second
-        constexpr int PFD = (BLUE && C::NPASS <= 3) ? C::EPT / 2 : 0;
-        constexpr int PFDL = PFD > 0 ? C::EPT : 0;
+        // loads of all of D spill at the 128-VGPR cap; with two lines per thread
+        // it all comes in the last pass), and the live slots of the output
+        // chirp during the second
+        constexpr int PFD = (BLUE && C::NPASS <= 3 && L == 1) ? C::EPT / 2 : 0;
+        constexpr int PFDL = (BLUE && C::NPASS <= 3) ? C::EPT : 0;
         float2 pf[C::EPT];
-        FftTile<S, THREADS, COLS, ZIN, PFD, PFDL>::run(v, t, ll, lds, job.tw, job.dtab, pf);
+        FftTile<S, THREADS, COLS, ZIN, PFD, PFDL>::run(v, t, slot, lds, job.tw, job.dtab, pf);
 
         if constexpr (BLUE) {
             // forward conj(v*D), inverse conj(v)*D = conj(v*conj(D)); the outer
             // conjugation turns the next forward FFT into the inverse one
 #pragma unroll
             for (int i = 0; i < C::EPT; ++i) {
-                v[i] = cmul_conj(v[i], i < PFDL ? pf[i] : load_at(job.dtab + i * C::TPL, uint32_t(t)));
+                const float2 d = i < PFDL ? pf[i] : load_at(job.dtab + i * C::TPL, uint32_t(t));
+#pragma unroll
+                for (int l = 0; l < L; ++l) v[l][i] = cmul_conj(v[l][i], d);
             }
             // the output chirp block is followed by readable entries up to
             // position M/2 + M/16 (dir_tables_len), so every live slot can be loaded
-            FftTile<S, THREADS, COLS, false, LIVE>::run(v, t, ll, lds, job.tw, job.chirp_out, pf);
+            constexpr int PFO = L == 1 ? LIVE : 0;
+            FftTile<S, THREADS, COLS, false, PFO, LIVE>::run(v, t, slot, lds, job.tw, job.chirp_out, pf);
         }
 #pragma unroll
         for (int i = 0; i < LIVE; ++i) {
+            float2 y[L];
             // forward conj(v)*c = conj(v*conj(c)), inverse conj(v*c)/n = conj(v*(c/n))
-            if constexpr (BLUE)
-                put(i, cmul_conj(v[i], pf[i]));
-            else
-                put(i, cscale(cxor(v[i], sgn), sc));
+#pragma unroll
+            for (int l = 0; l < L; ++l) y[l] = BLUE ? cmul_conj(v[l][i], pf[i]) : cscale(cxor(v[l][i], sgn), sc);
+            put(i, y);
         }
     }
 }

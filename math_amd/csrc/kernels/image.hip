@@ -13,13 +13,6 @@
 
 namespace mdft {
 
-__host__ __device__ constexpr int image_threads(int shape, bool wide)
-{
-    const int tpl = tpl_of(shape);
-    const int base = wide ? 1024 : 256;
-    return tpl > base ? tpl : base;
-}
-
 template <int S, int T, bool BLUE, bool COLS, int IO>
 __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(TILE_WAVES))) void k_image_axis(AxisJob job, ImageIO io)
 {
@@ -55,14 +48,14 @@ template <int S>
 static hipError_t launch_image_t(const AxisJob& job, const ImageIO& io, bool blue, bool cols, int mode, bool wide,
                                  hipStream_t stream)
 {
-    constexpr int TN = image_threads(S, false), TW = image_threads(S, true);
+    constexpr int TN = narrow_threads(S), TW = wide_threads(S, true), SW = wide_shape(S);
     if (!cols) {
         if (mode == IO_LUM) return launch_image_tt<S, TN, false, IO_LUM>(job, io, blue, stream);
         if (mode == (IO_LUM | IO_MAG)) return launch_image_tt<S, TN, false, IO_LUM | IO_MAG>(job, io, blue, stream);
         return hipErrorInvalidValue;
     }
     if (mode == IO_MAG) {
-        if (wide && TW != TN) return launch_image_tt<S, TW, true, IO_MAG>(job, io, blue, stream);
+        if (wide) return launch_image_tt<SW, TW, true, IO_MAG>(job, io, blue, stream);
         return launch_image_tt<S, TN, true, IO_MAG>(job, io, blue, stream);
     }
     if (mode == (IO_LUM | IO_MAG)) return launch_image_tt<S, TN, true, IO_LUM | IO_MAG>(job, io, blue, stream);

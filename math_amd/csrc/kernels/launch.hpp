@@ -95,6 +95,13 @@ hipError_t gen_chirp(double2* chirp64, float2* chirp32, float2* dir, int n, int 
 hipError_t gen_dir_diagonal(float2* dir, const float2* dtab, int n, int m, hipStream_t stream);
 hipError_t gen_dtab(float2* dtab, const double2* chirp64, double* cos_scratch, int n, int m, hipStream_t stream);
 
+// Workgroup sizes of the single-image kernels.  Narrow: 256 threads, or one
+// line when a line needs more (16384 points: 512).  Wide tiles hold more lines:
+// the X2 form of a shape that has one (columns in 512 threads, so two tiles are
+// on a CU at a time; rows in 256), 1024 threads for other shapes.
+__host__ __device__ constexpr int narrow_threads(int shape) { return tpl_of(shape) > 256 ? tpl_of(shape) : 256; }
+__host__ __device__ constexpr int wide_shape(int shape) { return has_x2(shape) ? shape | X2 : shape; }
+__host__ __device__ constexpr int wide_threads(int shape, bool cols) { return !has_x2(shape) ? 1024 : cols ? 512 : 256; }
 // threads: 1024 wide tiles, 256 narrow, 128 or 64 small (clamped to one line per workgroup)
 hipError_t launch_axis(int shape, const AxisJob& job, bool blue, bool cols, int threads, hipStream_t stream);
 
@@ -109,11 +116,12 @@ hipError_t launch_image_magnitude(const ImageIO& io, const float2* src, int w, i
 // lengths 1024-4096 (wider contiguous runs per row), two workgroups per CU.
 constexpr int BATCH_COL_THREADS = 512;
 
-// batch kernels: threads is 256, 512 or 1024 (padded lengths up to 8192; 6144 from 512 threads)
+// batch kernels, padded lengths up to 8192: threads is 256 (any items), or 512 or 1024 (column tiles only);
+// the persistent shapes run in 256 threads
 hipError_t launch_batch_grid(int threads, const BatchJob* jobs, const uint2* items, uint32_t nitems,
                              hipStream_t stream);
-hipError_t launch_batch_persistent(int threads, const BatchJob* jobs, const uint2* items, uint32_t nitems,
-                                   uint32_t* ctl, uint32_t nctl, int grid, uint32_t spin_limit, hipStream_t stream);
+hipError_t launch_batch_persistent(const BatchJob* jobs, const uint2* items, uint32_t nitems, uint32_t* ctl,
+                                   uint32_t nctl, int grid, uint32_t spin_limit, hipStream_t stream);
 // their kernels of one workgroup size (batch_kernels.hip, compiled per size and launch shape)
 template <int T>
 hipError_t launch_batch_grid_t(const BatchJob* jobs, const uint2* items, uint32_t nitems, hipStream_t stream);
@@ -126,9 +134,9 @@ template <int T>
 hipError_t warm_batch_grid(uint32_t* word, hipStream_t stream);
 template <int T>
 hipError_t warm_batch_persistent(uint32_t* word, hipStream_t stream);
-// lines of a shape one tile of `threads` threads holds (0: the shape does not fit)
-int batch_lines_per_tile(int threads, int shape);
-hipError_t batch_occupancy(int threads, int* blocks_per_cu);
+// lines of a shape one tile holds: rows in 256 threads, columns in 256, 512 or 1024 (0: the shape does not fit)
+int batch_lines_per_tile(int threads, int shape, bool cols);
+hipError_t batch_occupancy(int* blocks_per_cu);
 int batch_max_logm();
 
 }  // namespace mdft
