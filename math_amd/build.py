@@ -36,6 +36,7 @@ SOURCES = [
     "kernels/tables.hip",
     "kernels/large.hip",
     "kernels/image.hip",
+    "kernels/smooth.hip",
     "host/runtime.cpp",
     "host/capi.cpp",
     "host/fft1d.cpp",

@@ -29,16 +29,25 @@ int batch_threads_for(const uint32_t* widths, const uint32_t* heights, size_t co
     for (size_t i = 0; i < count; ++i) {
         compute_m(widths[i]);  // validates the sides
         compute_m(heights[i]);
-        // the FFT lengths the tiles run (the padded length, or 3 * 2^k)
-        const int sr = line_shape(widths[i], false), sc = line_shape(heights[i], true);
-        if (m_of(sr) > (1 << limit) || m_of(sc) > (1 << limit))
-            throw Error(MDFT_ERR_SIZE, "batch transform " + std::to_string(i) + " (" + std::to_string(widths[i]) + "x" +
-                                           std::to_string(heights[i]) + ") exceeds the batch padded-length limit " +
-                                           std::to_string(1 << limit));
-        tpl = std::max({tpl, tpl_of(sr), tpl_of(sc)});
+        // the FFT lengths the tiles run (the padded length, or 3 * 2^k; a smooth length itself)
+        for (int shape : {line_shape(widths[i], false), line_shape(heights[i], true)}) {
+            if (shape == GEN_SHAPE) continue;
+            if (m_of(shape) > (1 << limit))
+                throw Error(MDFT_ERR_SIZE, "batch transform " + std::to_string(i) + " (" + std::to_string(widths[i]) +
+                                               "x" + std::to_string(heights[i]) +
+                                               ") exceeds the batch padded-length limit " +
+                                               std::to_string(1 << limit));
+            tpl = std::max(tpl, tpl_of(shape));
+        }
     }
-    // the smallest tile that holds a whole line of every length
+    // the smallest tile that holds a whole line of every length (256 threads up to the limit)
     return tpl <= 256 ? 256 : tpl <= 512 ? 512 : 1024;
+}
+
+// lines a tile of T threads holds of a plan's length
+static int lines_per_tile(int T, const LinePlan& lp, bool cols)
+{
+    return lp.gen ? T / lp.smooth.tpl : batch_lines_per_tile(T, lp.shape, cols);
 }
 
 void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int T, int TC, bool dependent,
@@ -61,6 +70,7 @@ void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int T, i
     struct Item {
         int phase;
         int m, shape, blue, kind;  // kind: 0 whole, 1 row tile, 2 column tile
+        int lpw;                   // lines of its tile
         uint32_t seq;
         uint2 v;
     };
@@ -74,13 +84,13 @@ void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int T, i
         auto cp = ctx.line_plan(h, true);
         out.keep.push_back(rp);
         out.keep.push_back(cp);
-        const int lpw_r = w > 1 ? batch_lines_per_tile(T, rp->shape, false) : 0;
+        const int lpw_r = w > 1 ? lines_per_tile(T, *rp, false) : 0;
         // a whole image runs both passes in one row-phase workgroup
-        const int lpw_cw = h > 1 ? batch_lines_per_tile(T, cp->shape, true) : 0;
+        const int lpw_cw = h > 1 ? lines_per_tile(T, *cp, true) : 0;
         const bool whole = (w > 1 && h > 1 && h <= lpw_r && w <= lpw_cw);
         // column tiles of images with a row pass run in the column phase (TC
         // threads); a single-column-pass image (w == 1) runs with the rows
-        const int lpw_c = h > 1 ? batch_lines_per_tile((w > 1 && !whole) ? TC : T, cp->shape, true) : 0;
+        const int lpw_c = h > 1 ? lines_per_tile((w > 1 && !whole) ? TC : T, *cp, true) : 0;
         const int ntr = w > 1 ? (h + lpw_r - 1) / lpw_r : 0;
         const int ntc = h > 1 ? (w + lpw_c - 1) / lpw_c : 0;
         const int sig = (dependent && w > 1 && h > 1 && !whole) ? (int)counter++ : -1;
@@ -117,15 +127,15 @@ void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int T, i
         }
         std::vector<uint2> ri, ci;
         if (whole) {
-            items.push_back({1, rp->m, rp->shape, rp->blue, 0, seq++, make_uint2(rj, BATCH_WHOLE | (uint32_t)cj)});
+            items.push_back({1, rp->m, rp->shape, rp->blue, 0, lpw_r, seq++, make_uint2(rj, BATCH_WHOLE | (uint32_t)cj)});
             ri.push_back(items.back().v);
         } else {
             for (int t = 0; t < ntr; ++t) {
-                items.push_back({1, rp->m, rp->shape, rp->blue, 1, seq++, make_uint2(rj, t)});
+                items.push_back({1, rp->m, rp->shape, rp->blue, 1, lpw_r, seq++, make_uint2(rj, t)});
                 ri.push_back(items.back().v);
             }
             for (int t = 0; t < ntc; ++t) {
-                items.push_back({w > 1 ? 2 : 1, cp->m, cp->shape, cp->blue, 2, seq++, make_uint2(cj, t)});
+                items.push_back({w > 1 ? 2 : 1, cp->m, cp->shape, cp->blue, 2, lpw_c, seq++, make_uint2(cj, t)});
                 ci.push_back(items.back().v);
             }
         }
@@ -152,8 +162,7 @@ void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int T, i
         std::vector<double> c1, c2;
         for (const Item& it : items) {
             // cost of a tile ~ points x passes (x2 for Bluestein's two FFTs)
-            const int lpw = batch_lines_per_tile(it.kind == 2 && it.phase == 2 ? TC : T, it.shape, it.kind == 2);
-            const double cost = double(lpw) * double(it.m) * (std::log2(double(it.m)) + 2) * (it.blue ? 2.0 : 1.0) *
+            const double cost = double(it.lpw) * double(it.m) * (std::log2(double(it.m)) + 2) * (it.blue ? 2.0 : 1.0) *
                                 (it.kind == 0 ? 2.0 : 1.0);
             (it.phase == 1 ? p1 : p2).push_back(it.v);
             (it.phase == 1 ? c1 : c2).push_back(cost);

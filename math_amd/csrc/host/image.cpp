@@ -115,7 +115,10 @@ int mdft_image_exec_device(mdft_image image, const void* src, uint32_t src_width
         io.mel = 1, io.mls = (int64_t)dst_pitch;
         const mdft::AxisJob j = ctx.make_job(row, nullptr, image->buf, 1, w, h, false);
         const int mode = mdft::IO_LUM | (h == 1 ? mdft::IO_MAG : 0);
-        launch(mdft::launch_image_axis(row.shape, j, io, row.blue, false, mode, false, s), "image row pass launch");
+        if (row.gen)
+            launch(mdft::launch_smooth_image(j, io, false, mode, 256, s), "image row pass launch");
+        else
+            launch(mdft::launch_image_axis(row.shape, j, io, row.blue, false, mode, false, s), "image row pass launch");
     }
     if (h > 1) {
         // columns: magnitude out; luminance in as well when there was no row pass
@@ -123,8 +126,14 @@ int mdft_image_exec_device(mdft_image image, const void* src, uint32_t src_width
         io.mel = (int64_t)dst_pitch, io.mls = 1;
         const mdft::AxisJob j = ctx.make_job(col, image->buf, nullptr, w, 1, w, false);
         const int mode = mdft::IO_MAG | (w == 1 ? mdft::IO_LUM : 0);
-        const bool wide = ctx.wide_tiles(col.shape, col.blue, true, w);
-        launch(mdft::launch_image_axis(col.shape, j, io, col.blue, true, mode, wide, s), "image column pass launch");
+        if (col.gen) {
+            launch(mdft::launch_smooth_image(j, io, true, mode, ctx.smooth_threads(col.smooth, true, w), s),
+                   "image column pass launch");
+        } else {
+            const bool wide = ctx.wide_tiles(col.shape, col.blue, true, w);
+            launch(mdft::launch_image_axis(col.shape, j, io, col.blue, true, mode, wide, s),
+                   "image column pass launch");
+        }
     }
     image->order.after(s);
     MDFT_API_END

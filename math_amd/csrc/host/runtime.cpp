@@ -67,6 +67,73 @@ uint64_t large_scratch_elems(long long m, long long count)
     return m > LineMaxTile ? (uint64_t)count * (uint64_t)m : 0;
 }
 
+namespace {
+
+// The fewest passes, then the fewest threads per line (the most points in each
+// thread's registers), then the smallest radices.
+void search_passes(int n, int left, int max_index, std::vector<int>& now, std::vector<int>& best, int& best_tpl)
+{
+    static const int radices[] = {16, 15, 12, 10, 9, 8, 7, 5, 4, 3, 2};
+    if (left == 1) {
+        int tpl = 1;
+        for (int r : now) {
+            const int nb = r >= 9 ? 1 : 16 / r, need = (n / r + nb - 1) / nb;
+            tpl = std::max(tpl, need);
+        }
+        if (tpl > 256) return;
+        if (best.empty() || now.size() < best.size() || (now.size() == best.size() && tpl < best_tpl)) {
+            best = now;
+            best_tpl = tpl;
+        }
+        return;
+    }
+    if (now.size() >= (size_t)GEN_MAX_PASS || (!best.empty() && now.size() >= best.size())) return;
+    for (int i = max_index; i < 11; ++i) {
+        if (left % radices[i]) continue;
+        now.push_back(radices[i]);
+        search_passes(n, left / radices[i], i, now, best, best_tpl);
+        now.pop_back();
+    }
+}
+
+}  // namespace
+
+bool smooth_plan(long long n, GenPlan* plan)
+{
+    if (n < 17 || n > GEN_MAX_N || is_pow2((uint64_t)n)) return false;
+    if (n % 3 == 0 && is_pow2((uint64_t)(n / 3)) && n >= (3LL << F3_MIN_K)) return false;
+    long long rest = n;
+    for (int f : {2, 3, 5, 7})
+        while (rest % f == 0) rest /= f;
+    if (rest != 1) return false;
+    std::vector<int> now, best;
+    int tpl = 0;
+    search_passes((int)n, (int)n, 0, now, best, tpl);
+    if (best.size() < 2) return false;
+    if (!plan) return true;
+    // an odd radix first (its scatter's stride meets every LDS bank), then ascending: the largest radix last has
+    // the fewest twiddle rows
+    std::sort(best.begin(), best.end());
+    auto odd = best.end();
+    for (auto it = best.begin(); it != best.end(); ++it)
+        if (*it % 2) odd = it;
+    if (odd != best.end()) std::rotate(best.begin(), odd, odd + 1);
+    *plan = GenPlan{};
+    plan->n = (int)n;
+    plan->npass = (int)best.size();
+    plan->tpl = tpl;
+    int ns = 1;
+    for (int p = 0; p < plan->npass; ++p) {
+        GenPass& g = plan->pass[p];
+        g.radix = best[p];
+        g.ns = ns;
+        g.nbf = (int)n / best[p];
+        g.magic = ns > 1 ? (uint32_t)(((uint64_t(1) << 32) + ns - 1) / ns) : 0u;
+        ns *= best[p];
+    }
+    return true;
+}
+
 int line_shape(long long n, bool cols)
 {
     const int m = compute_m(n);
@@ -74,6 +141,7 @@ int line_shape(long long n, bool cols)
     // n = 3 * 2^k itself: a direct FFT of that shape, no Bluestein
     if (n % 3 == 0 && is_pow2((uint64_t)(n / 3)) && n >= (3LL << F3_MIN_K) && n <= (3LL << F3_MAX_K))
         return F3_BASE + ilog2((uint64_t)(n / 3));
+    if (smooth_plan(n, nullptr)) return GEN_SHAPE;
     long long m3 = 3LL << F3_MIN_K;
     while (m3 < 2 * n - 1) m3 <<= 1;
     const int k3 = ilog2((uint64_t)(m3 / 3));
@@ -86,6 +154,7 @@ LinePlan::~LinePlan()
     if (chirp) (void)hipFree(chirp);
     if (dtab) (void)hipFree(dtab);
     if (dir) (void)hipFree(dir);
+    if (gen) (void)hipFree(gen);
     if (tw_lo) (void)hipFree(tw_lo);
     if (tw_hi) (void)hipFree(tw_hi);
 }
@@ -180,16 +249,14 @@ Context::Context(int device) : device_(device)
     hip_check(warm_axis(word, gen_stream_), "kernel load");
     hip_check(warm_image(word, gen_stream_), "kernel load");
     hip_check(warm_large(word, gen_stream_), "kernel load");
+    hip_check(warm_smooth(word, gen_stream_), "kernel load");
     hip_check(warm_batch(word, gen_stream_), "kernel load");
     hip_check(hipStreamSynchronize(gen_stream_), "kernel load");
     noalloc_setup(device);
-    // default tile shapes: wide tiles for columns of 1024 points and more, and for rows with an X2 form
+    // default tile shapes: wide tiles for columns of 1024 points and more
     for (int i = 0; i < NSHAPES; ++i) {
         const int shape = i <= MAX_LOGM ? i : F3_BASE + F3_MIN_K + (i - MAX_LOGM - 1);
-        for (int b = 0; b < 2; ++b) {
-            variant_[i][b][0] = has_x2(shape) ? 1 : 0;
-            variant_[i][b][1] = (m_of(shape) >= 1024) ? 1 : 0;
-        }
+        for (int b = 0; b < 2; ++b) variant_[i][b][1] = (m_of(shape) >= 1024) ? 1 : 0;
     }
 }
 
@@ -210,15 +277,23 @@ std::shared_ptr<const LinePlan> Context::line_plan(int n, bool cols)
     lp->n = n;
     lp->shape = shape;
     lp->padded = m;
-    lp->m = is_f3(lp->shape) ? m_of(lp->shape) : m;
-    lp->logm = is_f3(lp->shape) ? 0 : ilog2((uint64_t)m);
-    // powers of two and n = 3 * 2^k run a direct FFT of length n
+    const bool smooth = shape == GEN_SHAPE;
+    lp->m = smooth ? n : is_f3(lp->shape) ? m_of(lp->shape) : m;
+    lp->logm = smooth || is_f3(lp->shape) ? 0 : ilog2((uint64_t)m);
+    // powers of two, n = 3 * 2^k and other smooth lengths run a direct FFT of length n
     lp->blue = lp->m != n;
     if (lp->logm > LARGE_MAX_LOGM)
         throw Error(MDFT_ERR_SIZE, "Error size " + std::to_string(n) + ": padded length " + std::to_string(m) +
                                        " exceeds the longest supported line (2^" + std::to_string(LARGE_MAX_LOGM) +
                                        ")");
     DeviceGuard g(device_);
+    if (smooth) {
+        smooth_plan(n, &lp->smooth);
+        const size_t len = (size_t)smooth_block_len(lp->smooth);
+        hip_check(hipMalloc(&lp->gen, sizeof(float2) * len), "hipMalloc twiddles");
+        lp->bytes += sizeof(float2) * len;
+        hip_check(gen_smooth(lp->gen, lp->smooth, gen_stream_), "twiddle generation");
+    }
     if (lp->large()) {
         large_split(lp->logm, &lp->logm1, &lp->logm2, &lp->logm3);
         const int64_t nhi = int64_t(m) >> LARGE_LO_BITS;
@@ -364,7 +439,9 @@ AxisJob Context::make_job(const LinePlan& lp, const float2* src, float2* dst, in
     j.chirp = lp.dir ? lp.dir + (inverse ? n : 0) : nullptr;
     j.dtab = lp.dir ? lp.dir + 2 * n + (inverse ? m : 0) : nullptr;
     j.chirp_out = lp.dir ? lp.dir + 2 * n + 2 * m + (inverse ? n : 0) : nullptr;
-    j.tw = twiddles(lp.shape);
+    j.tw = lp.gen ? lp.gen : twiddles(lp.shape);
+    j.tpl = lp.smooth.tpl;
+    j.npass = lp.smooth.npass;
     return j;
 }
 
@@ -596,6 +673,10 @@ void Context::enqueue_axis(const LinePlan& lp, const float2* src, float2* dst, i
         return;
     }
     const AxisJob j = make_job(lp, src, dst, es, ls, count, inverse);
+    if (lp.gen) {
+        hip_check(launch_smooth(j, cols, smooth_threads(lp.smooth, cols, count), stream), "axis pass launch");
+        return;
+    }
     const int threads = tile_threads(lp.shape, lp.blue, cols, count);
     hip_check(launch_axis(lp.shape, j, lp.blue, cols, threads, stream), "axis pass launch");
 }
@@ -603,10 +684,10 @@ void Context::enqueue_axis(const LinePlan& lp, const float2* src, float2* dst, i
 bool Context::wide_tiles(int shape, bool blue, bool cols, int count) const
 {
     if (variant(shape, blue, cols) == 0) return false;
-    // keep at least one tile per CU (rows: the four that run at a time)
-    const int lines_wide = wide_threads(shape, cols) / tpl_of(shape) * lines_per_thread(wide_shape(shape));
+    // keep at least one tile per CU
+    const int lines_wide = wide_threads(shape, cols) / tpl_of(shape) * lines_per_thread(wide_shape(shape, cols));
     const int64_t tiles = (int64_t(count) + lines_wide - 1) / lines_wide;
-    return tiles >= int64_t(cols ? 1 : 4) * cu_count_;
+    return tiles >= int64_t(cu_count_);
 }
 
 int Context::tile_threads(int shape, bool blue, bool cols, int count) const
@@ -619,6 +700,16 @@ int Context::tile_threads(int shape, bool blue, bool cols, int count) const
     const int64_t want = int64_t(cols ? 1 : 4) * cu_count_;
     int t = tpl > 256 ? tpl : 256;
     while (t > 64 && t / 2 >= tpl && (int64_t(count) + t / tpl - 1) / (t / tpl) < want) t /= 2;
+    return t;
+}
+
+int Context::smooth_threads(const GenPlan& plan, bool cols, int count) const
+{
+    // as tile_threads: columns in the widest tiles that leave every CU one,
+    // rows in 256 threads, smaller ones where there are few lines
+    const int64_t want = int64_t(cols ? 1 : 4) * cu_count_;
+    int t = cols ? 512 : 256;
+    while (t > 64 && t / 2 >= plan.tpl && (int64_t(count) + t / plan.tpl - 1) / (t / plan.tpl) < want) t /= 2;
     return t;
 }
 

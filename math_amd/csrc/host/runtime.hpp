@@ -33,9 +33,13 @@ void hip_check(hipError_t e, const char* what);
 int compute_m(long long n);
 int ilog2(uint64_t v);
 bool is_pow2(uint64_t v);
+// Passes of a direct mixed-radix FFT of n points (smooth_device.hpp): false
+// unless n in [17, GEN_MAX_N] has no factor above 7 and splits into passes of at
+// most 256 threads, and neither n = 2^k nor 3 * 2^k >= 192 (compiled shapes).
+bool smooth_plan(long long n, GenPlan* plan);
 // FFT shape (fft_device.hpp) of a line of length n along an axis: log2(n)
-// for a power of two, 3 * 2^k for n = 3 * 2^k in [192, 6144] (both direct
-// FFTs of length n); for other lengths the Bluestein convolution length, the
+// for a power of two, 3 * 2^k for n = 3 * 2^k in [192, 6144], GEN_SHAPE for other
+// smooth lengths (all direct FFTs of length n); for other lengths the Bluestein convolution length, the
 // reference's compute_m(n) = 2^j, or 3 * 2^k >= 2n - 1 when that is shorter:
 // along columns for 3 * 2^k in [192, 6144], along rows in [3072, 6144] (the
 // shorter row tiles measured slower with the extra passes, the longer ones
@@ -69,6 +73,9 @@ struct LinePlan {
     float2* dtab = nullptr;   // m entries, Bluestein only
     // tile-resident Bluestein lengths: the direction tables (dir_tables_len)
     float2* dir = nullptr;
+    // smooth lengths: pass table and twiddle rows, and the plan they were made from
+    float2* gen = nullptr;
+    GenPlan smooth{};
     // lines longer than one tile: M = 2^logm1 * 2^logm2 (four-step), or
     // 2^logm1 * 2^logm2 * 2^logm3 (logm3 > 0: three factors), with a
     // two-level table of exp(-2*pi*i*j/M)
@@ -163,6 +170,8 @@ public:
     bool wide_tiles(int shape, bool blue, bool cols, int count) const;
     // workgroup size of a single-image pass of `count` lines (launch_axis)
     int tile_threads(int shape, bool blue, bool cols, int count) const;
+    // workgroup size of a pass over `count` lines of a smooth length (launch_smooth)
+    int smooth_threads(const GenPlan& plan, bool cols, int count) const;
     void set_variant(int shape, bool blue, bool cols, int v) { variant_[shape_index(shape)][blue][cols] = (uint8_t)v; }
 
 private:

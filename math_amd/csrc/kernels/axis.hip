@@ -45,7 +45,7 @@ template <int S, bool COLS>
 static hipError_t launch_axis_t(const AxisJob& job, bool blue, int threads, hipStream_t stream)
 {
     constexpr int TPL = tpl_of(S);
-    if (threads >= 1024) return launch_axis_tt<wide_shape(S), wide_threads(S, COLS), COLS>(job, blue, stream);
+    if (threads >= 1024) return launch_axis_tt<wide_shape(S, COLS), wide_threads(S, COLS), COLS>(job, blue, stream);
     if constexpr (TPL <= 64) {
         if (threads <= 64) return launch_axis_tt<S, 64, COLS>(job, blue, stream);
     }

@@ -28,16 +28,18 @@
 
 #include "fft_device.hpp"
 #include "launch.hpp"
+#include "smooth_device.hpp"
 
 namespace mdft {
 
 // The form of a shape a batch runs: two lines per thread where the shape has
-// that, along rows and in the column tiles of phase 2 (kernels of more than 256
-// threads, which hold columns only); one for the columns of phase 1 (small
-// whole images and single columns).
+// that in the column tiles of phase 2 (kernels of more than 256 threads, which
+// hold columns only); one along rows, where two measured no better (4096^2:
+// 140 us against 152), and for the columns of phase 1 (small whole images and
+// single columns).
 __host__ __device__ constexpr int batch_shape(int s, int threads, bool cols)
 {
-    return has_x2(s) && (!cols || threads > 256) ? s | X2 : s;
+    return has_x2(s) && cols && threads > 256 ? s | X2 : s;
 }
 
 template <int S, int T, bool COLS_ONLY>
@@ -57,13 +59,14 @@ constexpr int cmax(int a, int b) { return a > b ? a : b; }
 template <int T, bool C>
 constexpr int batch_lds()
 {
-    return cmax(cmax(cmax(cmax(lds_need<5, T, C>(), lds_need<6, T, C>()), cmax(lds_need<7, T, C>(), lds_need<8, T, C>())),
+    return cmax(gen_lds_floats(T),
+           cmax(cmax(cmax(cmax(lds_need<5, T, C>(), lds_need<6, T, C>()), cmax(lds_need<7, T, C>(), lds_need<8, T, C>())),
                      cmax(cmax(cmax(lds_need<9, T, C>(), lds_need<10, T, C>()),
                                cmax(lds_need<11, T, C>(), lds_need<12, T, C>())),
                           lds_need<13, T, C>())),
                 cmax(cmax(cmax(lds_need<F3_BASE + 6, T, C>(), lds_need<F3_BASE + 7, T, C>()),
                           cmax(lds_need<F3_BASE + 8, T, C>(), lds_need<F3_BASE + 9, T, C>())),
-                     cmax(lds_need<F3_BASE + 10, T, C>(), lds_need<F3_BASE + 11, T, C>())));
+                     cmax(lds_need<F3_BASE + 10, T, C>(), lds_need<F3_BASE + 11, T, C>()))));
 }
 
 // One variant.  The thread and tile indices go through an empty asm of its own in every
@@ -89,10 +92,26 @@ __device__ __forceinline__ void run_axis(const AxisJob& job, int blue, int tile,
     run_variant<batch_shape(S, T, COLS), T, false, COLS>(job, tile, lds);
 }
 
+// a smooth length (its own asm for the indices, like run_variant)
+template <int T, bool COLS>
+__device__ __forceinline__ void run_smooth(const AxisJob& job, int tile, float* lds)
+{
+    int tid = threadIdx.x;
+    asm volatile("; tile variant %2" : "+v"(tid), "+s"(tile) : "n"(GEN_SHAPE * 4 + (COLS ? 1 : 0)));
+    smooth_tile<T, COLS>(job, tile, lds, tid);
+}
+
 template <int S, int T, bool COLS_ONLY>
 __device__ __forceinline__ void run_tile_body(const AxisJob& job, int blue, int cols, int tile, float* lds)
 {
-    if constexpr (tpl_of(S) <= T) {
+    if constexpr (S == GEN_SHAPE) {
+        if constexpr (COLS_ONLY)
+            run_smooth<T, true>(job, tile, lds);
+        else if (cols)
+            run_smooth<T, true>(job, tile, lds);
+        else
+            run_smooth<T, false>(job, tile, lds);
+    } else if constexpr (tpl_of(S) <= T) {
         if constexpr (COLS_ONLY)
             run_axis<S, T, true>(job, blue, tile, lds);
         else if (cols)
@@ -163,6 +182,7 @@ __device__ __forceinline__ void run_job_tile(const BatchJob* jobs, uint32_t job,
     case F3_BASE + 9: run_tile<F3_BASE + 9, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
     case F3_BASE + 10: run_tile<F3_BASE + 10, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
     case F3_BASE + 11: run_tile<F3_BASE + 11, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case GEN_SHAPE: run_tile<GEN_SHAPE, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
     default: break;
     }
 }

@@ -77,7 +77,7 @@ __device__ __forceinline__ float2 cscale(float2 a, float s) { return make_float2
 //    radix-12 pass (a 3 x 4 prime-factor butterfly).
 // The shape is a function of the line length and axis, so a line runs the
 // same schedule in every kernel.
-// S + X2: the same with two lines per thread.  The lines of a tile share the
+// S + X2: the same with two lines per thread (column tiles).  The lines of a tile share the
 // chirp, the diagonal and the twiddles at a position, which one line per thread
 // loads anew for every line (42 of the 60 loads of a Bluestein line's thread);
 // a thread with two lines loads them once for both, reads two adjacent columns
@@ -92,7 +92,7 @@ constexpr int TILE_WAVES = 4;
 constexpr int F3_BASE = 32;
 constexpr int F3_MIN_K = 6;   // M = 192: the radix-12 pass follows at least two radix-4 passes
 constexpr int F3_MAX_K = 11;  // M = 6144: 24 points per thread, 256 threads per line
-__host__ __device__ constexpr bool is_f3(int s) { return base_of(s) >= F3_BASE; }
+__host__ __device__ constexpr bool is_f3(int s) { return base_of(s) >= F3_BASE && base_of(s) < 60; }
 __host__ __device__ constexpr int f3_k(int s) { return base_of(s) - F3_BASE; }
 // 8192 and 16384 points: 32 per thread
 __host__ __device__ constexpr bool is_wide(int s) { return base_of(s) == 13 || base_of(s) == 14; }
@@ -520,7 +520,24 @@ struct AxisJob {
     const float2* dtab;       // middle: D or conj(D), D = FFT_M(conj(c) embedded) / M
     const float2* chirp_out;  // store: conj(c) (forward) or c/n (inverse), k < n
     const float2* tw;      // twiddle block of the line's FFT shape
+    // smooth lengths (smooth_device.hpp): threads per line and passes
+    int tpl;
+    int npass;
 };
+
+// Pass of a smooth length: GEN_MAX_PASS of these head the length's block, then
+// for every pass after the first ns rows of four twiddles (tw_power).
+struct GenPass {
+    int radix;
+    int ns;          // Stockham stride: the product of the earlier radices
+    int nbf;         // butterflies, n / radix
+    uint32_t magic;  // ceil(2^32 / ns): j / ns = umulhi(j, magic) for j < 4096
+};
+constexpr int GEN_MAX_PASS = 8;
+constexpr int GEN_TABLE = GEN_MAX_PASS * (int)sizeof(GenPass) / (int)sizeof(float2);  // in float2
+// shape code of such lengths, and the longest
+constexpr int GEN_SHAPE = 60;
+constexpr int GEN_MAX_N = 4096;
 
 // ---------------------------------------------------------------------------
 // image input and output of the view path: the luminance of an RGBA pixel
@@ -692,7 +709,7 @@ __device__ __forceinline__ void expand_twiddles(float2 (&wt)[R], const float4* q
     wt[1] = make_float2(q[0].x, q[0].y);
     if constexpr (R > 2) {
         wt[2] = make_float2(q[0].z, q[0].w);
-        wt[3] = make_float2(q[1].x, q[1].y);
+        if constexpr (R > 3) wt[3] = make_float2(q[1].x, q[1].y);
     }
     if constexpr (R > 4) {
         wt[4] = make_float2(q[1].z, q[1].w);

@@ -97,13 +97,32 @@ hipError_t gen_dtab(float2* dtab, const double2* chirp64, double* cos_scratch, i
 
 // Workgroup sizes of the single-image kernels.  Narrow: 256 threads, or one
 // line when a line needs more (16384 points: 512).  Wide tiles hold more lines:
-// the X2 form of a shape that has one (columns in 512 threads, so two tiles are
-// on a CU at a time; rows in 256), 1024 threads for other shapes.
+// columns take 512 threads in the X2 form of a shape that has one and at 6144
+// points (two tiles on a CU at a time; 3000^2 184 us against 195 with 1024),
+// other shapes 1024 (8192 points: four columns, 2048 x 8192 128 us against 167).
 __host__ __device__ constexpr int narrow_threads(int shape) { return tpl_of(shape) > 256 ? tpl_of(shape) : 256; }
-__host__ __device__ constexpr int wide_shape(int shape) { return has_x2(shape) ? shape | X2 : shape; }
-__host__ __device__ constexpr int wide_threads(int shape, bool cols) { return !has_x2(shape) ? 1024 : cols ? 512 : 256; }
+__host__ __device__ constexpr int wide_shape(int shape, bool cols) { return cols && has_x2(shape) ? shape | X2 : shape; }
+__host__ __device__ constexpr int wide_threads(int shape, bool cols)
+{
+    return cols && (has_x2(shape) || ept_of(shape) == 24) ? 512 : 1024;
+}
 // threads: 1024 wide tiles, 256 narrow, 128 or 64 small (clamped to one line per workgroup)
 hipError_t launch_axis(int shape, const AxisJob& job, bool blue, bool cols, int threads, hipStream_t stream);
+
+// ---- lines of smooth length (smooth.hip) ----
+struct GenPlan {
+    int n, npass, tpl;
+    GenPass pass[GEN_MAX_PASS];
+};
+// threads: 64, 128, 256 or 512, at least job.tpl
+hipError_t launch_smooth(const AxisJob& job, bool cols, int threads, hipStream_t stream);
+// modes as launch_image_axis; 256 threads, or 512 for columns that store magnitudes
+hipError_t launch_smooth_image(const AxisJob& job, const ImageIO& io, bool cols, int mode, int threads,
+                               hipStream_t stream);
+// float2 entries of a length's block (pass table and twiddle rows), and its generation
+int64_t smooth_block_len(const GenPlan& plan);
+hipError_t gen_smooth(float2* out, const GenPlan& plan, hipStream_t stream);
+hipError_t warm_smooth(uint32_t* word, hipStream_t stream);
 
 // image path: an axis pass with fused luminance input and/or magnitude output
 // (mode = IO_LUM | IO_MAG bits), and the unfused conversions
