@@ -563,15 +563,50 @@ __host__ __device__ __forceinline__ float luminance_rgb(float r, float g, float 
     return __builtin_fmaf(0.0722f, b, __builtin_fmaf(0.7152f, g, 0.2126f * r));
 }
 
+// UNORM: c / 255, correctly rounded (one step of residual correction; equal to
+// the division for all 256 values), in 3 instructions where a division takes about ten
+__device__ __forceinline__ float unorm8(uint32_t c)
+{
+    const float r = 1.0f / 255.0f, x = (float)c, q = x * r;
+    return __builtin_fmaf(__builtin_fmaf(-q, 255.0f, x), r, q);
+}
+__device__ __forceinline__ float luminance_rgba8(uint32_t c)
+{
+    return luminance_rgb(unorm8(c & 0xffu), unorm8((c >> 8) & 0xffu), unorm8((c >> 16) & 0xffu));
+}
+
 __device__ __forceinline__ float image_luminance(const ImageIO& io, int64_t idx)
 {
-    if (io.fmt == PIXEL_RGBA8) {
-        const uchar4 c = static_cast<const uchar4*>(io.img)[idx];
-        // UNORM: c / 255
-        return luminance_rgb((float)c.x / 255.0f, (float)c.y / 255.0f, (float)c.z / 255.0f);
-    }
+    if (io.fmt == PIXEL_RGBA8) return luminance_rgba8(static_cast<const uint32_t*>(io.img)[idx]);
     const float4 c = static_cast<const float4*>(io.img)[idx];
     return luminance_rgb(c.x, c.y, c.z);
+}
+
+// out[i] = luminance of pixel index(i), i < N.  The format is uniform: one
+// branch around all the loads, which are in flight together (a branch per
+// pixel made every load a latency of its own).
+template <int N, class Index>
+__device__ __forceinline__ void load_luminance(const ImageIO& io, const Index& index, float (&out)[N])
+{
+    typedef float vec3 __attribute__((ext_vector_type(3)));
+    if (io.fmt == PIXEL_RGBA8) {
+        auto img = (const __attribute__((address_space(1))) uint32_t*)io.img;
+        uint32_t px[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) px[i] = img[index(i)];
+#pragma unroll
+        for (int i = 0; i < N; ++i) out[i] = luminance_rgba8(px[i]);
+    } else {
+        auto img = (const __attribute__((address_space(1))) float*)io.img;
+        vec3 px[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            auto p = img + 4 * index(i);
+            px[i] = vec3{p[0], p[1], p[2]};
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) out[i] = luminance_rgb(px[i].x, px[i].y, px[i].z);
+    }
 }
 
 __device__ __forceinline__ float cabs_scaled(float2 y, float s)
@@ -980,6 +1015,18 @@ __device__ __forceinline__ void line_tile(const AxisJob& job, int tile, float* l
                 // opaque: else the select becomes a branch around the load
                 load_pair(i < SURE ? s + i * step : s + opaque(in ? i * step : 0), v[0][i], v[L - 1][i]);
             }
+        } else if constexpr ((IO & IO_LUM) != 0) {
+            const int64_t line = valid(0) ? line_of(0) : tile * C::LPW;
+            float lum[LIVE];
+            load_luminance<LIVE>(
+                io,
+                [&](int i) {
+                    const int pos = i < SURE || t + i * C::TPL < n ? t + i * C::TPL : t;
+                    return line * io.ils + int64_t(opaque(pos)) * io.iel;
+                },
+                lum);
+#pragma unroll
+            for (int i = 0; i < LIVE; ++i) v[0][i] = make_float2(lum[i], 0.0f);
         } else {
 #pragma unroll
             for (int i = 0; i < LIVE; ++i) {
@@ -987,11 +1034,7 @@ __device__ __forceinline__ void line_tile(const AxisJob& job, int tile, float* l
 #pragma unroll
                 for (int l = 0; l < L; ++l) {
                     const float2* s = job.src + base[l];
-                    if constexpr ((IO & IO_LUM) != 0) {
-                        const int64_t pos = in ? t + i * C::TPL : t;
-                        const int64_t line = valid(l) ? line_of(l) : tile * C::LPW;
-                        v[l][i] = make_float2(image_luminance(io, line * io.ils + pos * io.iel), 0.0f);
-                    } else if constexpr (COLS) {
+                    if constexpr (COLS) {
                         v[l][i] = load_global(i < SURE ? s + i * step : s + opaque(in ? i * step : 0));
                     } else {
                         v[l][i] = i < SURE ? load_at(s + i * step, off[l])

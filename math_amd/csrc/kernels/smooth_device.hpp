@@ -200,15 +200,19 @@ struct GenPassRun {
             }
         }
         float2 u[NB][R];
-        if constexpr (FIRST) {
+        if constexpr (FIRST && (IO & IO_LUM) != 0) {
+            float lum[NB * R];
+            load_luminance<NB * R>(
+                *x.io,
+                [&](int i) { return x.iline * x.io->ils + int64_t(jj[i / R] + (i % R) * nbf) * x.io->iel; }, lum);
+#pragma unroll
+            for (int i = 0; i < NB * R; ++i) u[i / R][i % R] = make_float2(lum[i], 0.0f);
+        } else if constexpr (FIRST) {
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
-                    if constexpr ((IO & IO_LUM) != 0)
-                        u[b][r] = make_float2(
-                            image_luminance(*x.io, x.iline * x.io->ils + int64_t(jj[b] + r * nbf) * x.io->iel), 0.0f);
-                    else if constexpr (COLS)
+                    if constexpr (COLS)
                         u[b][r] = load_global(job.src + x.base + int64_t(jj[b]) * job.es + int64_t(r * nbf) * job.es);
                     else
                         u[b][r] = load_at(job.src + x.base + r * nbf, x.off + uint32_t(jj[b]));
