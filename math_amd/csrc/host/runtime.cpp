@@ -681,18 +681,27 @@ void Context::enqueue_axis(const LinePlan& lp, const float2* src, float2* dst, i
     hip_check(launch_axis(lp.shape, j, lp.blue, cols, threads, stream), "axis pass launch");
 }
 
+// the workgroup size of wide tiles, 0 when the table says narrow or wide tiles would leave CUs without one
+int Context::wide_tile_threads(int shape, bool blue, bool cols, int count) const
+{
+    if (variant(shape, blue, cols) == 0) return 0;
+    for (int t = wide_threads(shape, cols, blue); t >= 512; t /= 2) {
+        const int lines = std::max(1, t / tpl_of(shape)) * lines_per_thread(wide_shape(shape, cols));
+        if ((int64_t(count) + lines - 1) / lines >= int64_t(cu_count_)) return t;
+        if (!(cols && has_x2(shape))) break;  // one wide size
+    }
+    return 0;
+}
+
 bool Context::wide_tiles(int shape, bool blue, bool cols, int count) const
 {
-    if (variant(shape, blue, cols) == 0) return false;
-    // keep at least one tile per CU
-    const int lines_wide = wide_threads(shape, cols) / tpl_of(shape) * lines_per_thread(wide_shape(shape, cols));
-    const int64_t tiles = (int64_t(count) + lines_wide - 1) / lines_wide;
-    return tiles >= int64_t(cu_count_);
+    return wide_tile_threads(shape, blue, cols, count) > 0;
 }
 
 int Context::tile_threads(int shape, bool blue, bool cols, int count) const
 {
-    if (wide_tiles(shape, blue, cols, count)) return 1024;
+    const int wide = wide_tile_threads(shape, blue, cols, count);
+    if (wide) return wide;
     // passes with few lines: smaller tiles (one wave for lines of up to 1024
     // points) so every CU gets work; rows aim at four tiles per CU, columns at
     // one, since narrower column tiles read shorter runs of each row

@@ -168,6 +168,7 @@ public:
     int variant(int shape, bool blue, bool cols) const { return variant_[shape_index(shape)][blue][cols]; }
     // the table's choice, narrowed when wide tiles would leave CUs without work
     bool wide_tiles(int shape, bool blue, bool cols, int count) const;
+    int wide_tile_threads(int shape, bool blue, bool cols, int count) const;
     // workgroup size of a single-image pass of `count` lines (launch_axis)
     int tile_threads(int shape, bool blue, bool cols, int count) const;
     // workgroup size of a pass over `count` lines of a smooth length (launch_smooth)

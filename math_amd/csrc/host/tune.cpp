@@ -87,7 +87,7 @@ int mdft_tune_auto(double* seconds)
                     float best = 0;
                     int best_v = 0;
                     for (int v = 0; v < 2; ++v) {
-                        const int threads = v ? 1024 : 256;
+                        const int threads = v ? mdft::wide_threads(shape, cols != 0, blue != 0) : 256;
                         auto launch = [&]() {
                             mdft::hip_check(mdft::launch_axis(shape, j, blue != 0, cols != 0, threads, s),
                                             "tuning launch");

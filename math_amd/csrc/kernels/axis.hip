@@ -39,13 +39,20 @@ static hipError_t launch_axis_tt(const AxisJob& job, bool blue, hipStream_t stre
     return hipGetLastError();
 }
 
-// threads: 1024 = wide tiles (launch.hpp), 256 = narrow, 128 / 64 = small tiles
-// for passes with few lines (clamped up to one line per workgroup)
+// threads: 1024 or 512 = wide tiles (launch.hpp), 256 = narrow, 128 / 64 = small
+// tiles for passes with few lines (clamped up to one line per workgroup)
 template <int S, bool COLS>
 static hipError_t launch_axis_t(const AxisJob& job, bool blue, int threads, hipStream_t stream)
 {
     constexpr int TPL = tpl_of(S);
-    if (threads >= 1024) return launch_axis_tt<wide_shape(S, COLS), wide_threads(S, COLS), COLS>(job, blue, stream);
+    constexpr int W = wide_shape(S, COLS);
+    if constexpr (COLS && has_x2(S)) {
+        if (threads >= 1024) return launch_axis_tt<W, 1024, COLS>(job, blue, stream);
+        if (threads >= 512) return launch_axis_tt<W, 512, COLS>(job, blue, stream);
+    } else {
+        if (threads >= 512 && threads > narrow_threads(S))
+            return launch_axis_tt<S, wide_threads(S, COLS, false), COLS>(job, blue, stream);
+    }
     if constexpr (TPL <= 64) {
         if (threads <= 64) return launch_axis_tt<S, 64, COLS>(job, blue, stream);
     }
