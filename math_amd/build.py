@@ -31,6 +31,7 @@ SOURCES = [
     ("kernels/batch_kernels.hip", f"batch_{kind}_{t}", [f"-DMDFT_BATCH_T={t}", f"-DMDFT_BATCH_PERSISTENT_TU={p}"])
     for p, kind, t in ((0, "grid", 256), (1, "persistent", 256), (0, "grid", 512), (0, "grid", 1024))
 ] + [
+    "kernels/whole.hip",
     "kernels/axis.hip",
     "kernels/batch.hip",
     "kernels/tables.hip",

@@ -251,6 +251,7 @@ Context::Context(int device) : device_(device)
     hip_check(warm_large(word, gen_stream_), "kernel load");
     hip_check(warm_smooth(word, gen_stream_), "kernel load");
     hip_check(warm_batch(word, gen_stream_), "kernel load");
+    hip_check(warm_whole(word, gen_stream_), "kernel load");
     hip_check(hipStreamSynchronize(gen_stream_), "kernel load");
     noalloc_setup(device);
     // default tile shapes: wide tiles for columns of 1024 points and more
@@ -722,9 +723,34 @@ int Context::smooth_threads(const GenPlan& plan, bool cols, int count) const
     return t;
 }
 
+// Whether all rows, and all columns, of an image fit one tile of the single-launch kernel
+bool Context::one_tile(const LinePlan& row, const LinePlan& col, int w, int h)
+{
+    if (w < 2 || h < 2 || row.large() || col.large()) return false;
+    auto fits = [](const LinePlan& lp, int count) {
+        const int64_t tpl = lp.gen ? lp.smooth.tpl : tpl_of(lp.shape);
+        // tpl of 8192 points: 256 threads; longer lines do not fit
+        return tpl * count <= WHOLE_THREADS;
+    };
+    return fits(row, h) && fits(col, w);
+}
+
 void Context::enqueue_transform(const LinePlan& row, const LinePlan& col, int w, int h, bool inverse,
                                 const float2* src, float2* dst, float2* scratch, hipStream_t stream) const
 {
+    if (one_tile(row, col, w, h)) {
+        auto job = [&](const LinePlan& lp, const float2* from, int64_t es, int64_t ls, int count, bool cols) {
+            BatchJob j{};
+            j.job = make_job(lp, from, dst, es, ls, count, inverse);
+            j.shape = lp.shape;
+            j.blue = lp.blue;
+            j.cols = cols;
+            return j;
+        };
+        const BatchJob r = job(row, src, 1, w, h, false), c = job(col, dst, w, 1, w, true);
+        hip_check(launch_whole(r, c, stream), "whole image launch");
+        return;
+    }
     const float2* s = src;
     if (w > 1) {
         enqueue_axis(row, s, dst, 1, w, h, inverse, false, scratch, stream);

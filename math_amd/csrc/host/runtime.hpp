@@ -171,6 +171,7 @@ public:
     int wide_tile_threads(int shape, bool blue, bool cols, int count) const;
     // workgroup size of a single-image pass of `count` lines (launch_axis)
     int tile_threads(int shape, bool blue, bool cols, int count) const;
+    static bool one_tile(const LinePlan& row, const LinePlan& col, int w, int h);
     // workgroup size of a pass over `count` lines of a smooth length (launch_smooth)
     int smooth_threads(const GenPlan& plan, bool cols, int count) const;
     void set_variant(int shape, bool blue, bool cols, int v) { variant_[shape_index(shape)][blue][cols] = (uint8_t)v; }

@@ -187,6 +187,35 @@ __device__ __forceinline__ void run_job_tile(const BatchJob* jobs, uint32_t job,
     }
 }
 
+// the same for a job given by value (inlined)
+template <int T, bool COLS_ONLY>
+__device__ __forceinline__ void run_job(const BatchJob& bj, int tile, float* lds)
+{
+    switch (bj.shape) {
+    case 1: run_tile_body<1, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 2: run_tile_body<2, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 3: run_tile_body<3, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 4: run_tile_body<4, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 5: run_tile_body<5, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 6: run_tile_body<6, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 7: run_tile_body<7, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 8: run_tile_body<8, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 9: run_tile_body<9, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 10: run_tile_body<10, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 11: run_tile_body<11, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 12: run_tile_body<12, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 13: run_tile_body<13, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case F3_BASE + 6: run_tile_body<F3_BASE + 6, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case F3_BASE + 7: run_tile_body<F3_BASE + 7, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case F3_BASE + 8: run_tile_body<F3_BASE + 8, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case F3_BASE + 9: run_tile_body<F3_BASE + 9, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case F3_BASE + 10: run_tile_body<F3_BASE + 10, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case F3_BASE + 11: run_tile_body<F3_BASE + 11, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case GEN_SHAPE: run_tile_body<GEN_SHAPE, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    default: break;
+    }
+}
+
 // One item; every branch is on a wave-uniform value.
 template <int T, bool INL, bool COLS_ONLY>
 __device__ __forceinline__ void run_item(const BatchJob* __restrict__ jobs, uint2 item, float* lds)

@@ -157,6 +157,10 @@ template <int T>
 hipError_t warm_batch_grid(uint32_t* word, hipStream_t stream);
 template <int T>
 hipError_t warm_batch_persistent(uint32_t* word, hipStream_t stream);
+// a small image in one launch (whole.hip): its row and column tile in one workgroup
+constexpr int WHOLE_THREADS = 256;
+hipError_t launch_whole(const BatchJob& row, const BatchJob& col, hipStream_t stream);
+hipError_t warm_whole(uint32_t* word, hipStream_t stream);
 // lines of a shape one tile holds: rows in 256 threads, columns in 256, 512 or 1024 (0: the shape does not fit)
 int batch_lines_per_tile(int threads, int shape, bool cols);
 hipError_t batch_occupancy(int* blocks_per_cu);
