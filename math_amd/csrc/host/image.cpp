@@ -130,7 +130,7 @@ int mdft_image_exec_device(mdft_image image, const void* src, uint32_t src_width
             launch(mdft::launch_smooth_image(j, io, true, mode, ctx.smooth_threads(col.smooth, true, w), s),
                    "image column pass launch");
         } else {
-            const bool wide = ctx.wide_tiles(col.shape, col.blue, true, w);
+            const bool wide = ctx.axis_tile(col.shape, col.blue, true, w).threads >= 512;
             launch(mdft::launch_image_axis(col.shape, j, io, col.blue, true, mode, wide, s),
                    "image column pass launch");
         }

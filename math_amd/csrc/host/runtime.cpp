@@ -678,31 +678,43 @@ void Context::enqueue_axis(const LinePlan& lp, const float2* src, float2* dst, i
         hip_check(launch_smooth(j, cols, smooth_threads(lp.smooth, cols, count), stream), "axis pass launch");
         return;
     }
-    const int threads = tile_threads(lp.shape, lp.blue, cols, count);
-    hip_check(launch_axis(lp.shape, j, lp.blue, cols, threads, stream), "axis pass launch");
+    const AxisTile tile = axis_tile(lp.shape, lp.blue, cols, count);
+    hip_check(launch_axis(tile.x2 ? lp.shape | X2 : lp.shape, j, lp.blue, cols, tile.threads, stream),
+              "axis pass launch");
 }
 
-// the workgroup size of wide tiles, 0 when the table says narrow or wide tiles would leave CUs without one
-int Context::wide_tile_threads(int shape, bool blue, bool cols, int count) const
+// Where the lines between the tiles lie (256 CUs; us, cold buffers):
+//  * direct X2 columns: 1024 threads from 1.5 tiles per CU (4096^2 113, 139 with
+//    512), then 512 and 256 from one tile per CU (2048^2 31.4 with 512, 37.8
+//    narrow; 1024 x 2048 21.6 with 256, 23.8 narrow; 1024^2 14.3 with 256 and
+//    half the CUs idle, 12.6 narrow);
+//  * Bluestein X2 columns of 2048 points and more: 512 threads when both tiles
+//    that fit a CU are there (2001 x 1201 46, 55 narrow; 1030 x 1201, one tile per
+//    CU, 41, 37 narrow);
+//  * Bluestein X2 columns: 256 threads from 2.5 tiles per CU (1500 x 2047 40.9, 42
+//    with 512, 51.5 narrow; 4001 x 701 49.2, 52.1; 2049 x 701, two tiles per CU,
+//    31.6, 29.4 narrow);
+//  * other wide tiles from one per CU.
+Context::AxisTile Context::axis_tile(int shape, bool blue, bool cols, int count) const
 {
-    if (variant(shape, blue, cols) == 0) return 0;
-    for (int t = wide_threads(shape, cols, blue); t >= 512; t /= 2) {
-        const int lines = std::max(1, t / tpl_of(shape)) * lines_per_thread(wide_shape(shape, cols));
-        if ((int64_t(count) + lines - 1) / lines >= int64_t(cu_count_)) return t;
-        if (!(cols && has_x2(shape))) break;  // one wide size
+    if (variant(shape, blue, cols) != 0) {
+        const bool x2 = cols && has_x2(shape);
+        // tiles of t threads, in eighths of the CUs
+        auto per_cu8 = [&](int t) {
+            const int64_t lines = int64_t(t) / tpl_of(shape) * (x2 ? 2 : 1);
+            return lines < 1 ? int64_t(0) : 8 * ((int64_t(count) + lines - 1) / lines) / cu_count_;
+        };
+        if (x2 && blue) {
+            if (m_of(shape) >= 2048 && per_cu8(512) >= 15) return {512, true};
+            if (per_cu8(256) >= 20) return {256, true};
+        } else if (x2) {
+            if (per_cu8(1024) >= 12) return {1024, true};
+            if (per_cu8(512) >= 8) return {512, true};
+            if (per_cu8(256) >= 8) return {256, true};
+        } else if (per_cu8(wide_threads(shape, cols, blue)) >= 8) {
+            return {wide_threads(shape, cols, blue), false};
+        }
     }
-    return 0;
-}
-
-bool Context::wide_tiles(int shape, bool blue, bool cols, int count) const
-{
-    return wide_tile_threads(shape, blue, cols, count) > 0;
-}
-
-int Context::tile_threads(int shape, bool blue, bool cols, int count) const
-{
-    const int wide = wide_tile_threads(shape, blue, cols, count);
-    if (wide) return wide;
     // passes with few lines: smaller tiles (one wave for lines of up to 1024
     // points) so every CU gets work; rows aim at four tiles per CU, columns at
     // one, since narrower column tiles read shorter runs of each row
@@ -710,12 +722,12 @@ int Context::tile_threads(int shape, bool blue, bool cols, int count) const
     const int64_t want = int64_t(cols ? 1 : 4) * cu_count_;
     int t = tpl > 256 ? tpl : 256;
     while (t > 64 && t / 2 >= tpl && (int64_t(count) + t / tpl - 1) / (t / tpl) < want) t /= 2;
-    return t;
+    return {t, false};
 }
 
 int Context::smooth_threads(const GenPlan& plan, bool cols, int count) const
 {
-    // as tile_threads: columns in the widest tiles that leave every CU one,
+    // as axis_tile: columns in the widest tiles that leave every CU one,
     // rows in 256 threads, smaller ones where there are few lines
     const int64_t want = int64_t(cols ? 1 : 4) * cu_count_;
     int t = cols ? 512 : 256;

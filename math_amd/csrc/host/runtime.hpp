@@ -163,14 +163,15 @@ public:
     AxisJob make_job(const LinePlan& lp, const float2* src, float2* dst, int64_t es, int64_t ls, int count,
                      bool inverse) const;
 
-    // Tile-shape table of the single-image kernels: variant 0 = narrow
-    // (256-thread) tiles, 1 = wide (1024-thread) tiles, per (FFT shape, blue, cols).
+    // Tile table of the single-image kernels: variant 0 = narrow (256-thread)
+    // tiles, 1 = wide ones where enough of them remain, per (FFT shape, blue, cols).
     int variant(int shape, bool blue, bool cols) const { return variant_[shape_index(shape)][blue][cols]; }
-    // the table's choice, narrowed when wide tiles would leave CUs without work
-    bool wide_tiles(int shape, bool blue, bool cols, int count) const;
-    int wide_tile_threads(int shape, bool blue, bool cols, int count) const;
-    // workgroup size of a single-image pass of `count` lines (launch_axis)
-    int tile_threads(int shape, bool blue, bool cols, int count) const;
+    // tile of a single-image pass of `count` lines (launch_axis)
+    struct AxisTile {
+        int threads;
+        bool x2;
+    };
+    AxisTile axis_tile(int shape, bool blue, bool cols, int count) const;
     static bool one_tile(const LinePlan& row, const LinePlan& col, int w, int h);
     // workgroup size of a pass over `count` lines of a smooth length (launch_smooth)
     int smooth_threads(const GenPlan& plan, bool cols, int count) const;

@@ -89,7 +89,8 @@ int mdft_tune_auto(double* seconds)
                     for (int v = 0; v < 2; ++v) {
                         const int threads = v ? mdft::wide_threads(shape, cols != 0, blue != 0) : 256;
                         auto launch = [&]() {
-                            mdft::hip_check(mdft::launch_axis(shape, j, blue != 0, cols != 0, threads, s),
+                            mdft::hip_check(mdft::launch_axis(v && cols && mdft::has_x2(shape) ? shape | mdft::X2 : shape, j,
+                                                              blue != 0, cols != 0, threads, s),
                                             "tuning launch");
                         };
                         const float ms = time_launches(s, launch, 5);

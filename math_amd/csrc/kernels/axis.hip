@@ -42,14 +42,19 @@ static hipError_t launch_axis_tt(const AxisJob& job, bool blue, hipStream_t stre
 // threads: 1024 or 512 = wide tiles (launch.hpp), 256 = narrow, 128 / 64 = small
 // tiles for passes with few lines (clamped up to one line per workgroup)
 template <int S, bool COLS>
-static hipError_t launch_axis_t(const AxisJob& job, bool blue, int threads, hipStream_t stream)
+static hipError_t launch_axis_t(const AxisJob& job, bool blue, bool x2, int threads, hipStream_t stream)
 {
     constexpr int TPL = tpl_of(S);
-    constexpr int W = wide_shape(S, COLS);
-    if constexpr (COLS && has_x2(S)) {
-        if (threads >= 1024) return launch_axis_tt<W, 1024, COLS>(job, blue, stream);
-        if (threads >= 512) return launch_axis_tt<W, 512, COLS>(job, blue, stream);
-    } else {
+    if (x2) {
+        if constexpr (COLS && has_x2(S)) {
+            if (threads >= 1024) return launch_axis_tt<S | X2, 1024, COLS>(job, blue, stream);
+            if (threads >= 512) return launch_axis_tt<S | X2, 512, COLS>(job, blue, stream);
+            return launch_axis_tt<S | X2, 256, COLS>(job, blue, stream);
+        } else {
+            return hipErrorInvalidValue;
+        }
+    }
+    if constexpr (!(COLS && has_x2(S))) {
         if (threads >= 512 && threads > narrow_threads(S))
             return launch_axis_tt<S, wide_threads(S, COLS, false), COLS>(job, blue, stream);
     }
@@ -77,27 +82,28 @@ hipError_t warm_axis(uint32_t* word, hipStream_t stream)
 template <bool COLS>
 static hipError_t launch_axis_dir(int shape, const AxisJob& job, bool blue, int threads, hipStream_t stream)
 {
-    switch (shape) {
-    case 1: return launch_axis_t<1, COLS>(job, blue, threads, stream);
-    case 2: return launch_axis_t<2, COLS>(job, blue, threads, stream);
-    case 3: return launch_axis_t<3, COLS>(job, blue, threads, stream);
-    case 4: return launch_axis_t<4, COLS>(job, blue, threads, stream);
-    case 5: return launch_axis_t<5, COLS>(job, blue, threads, stream);
-    case 6: return launch_axis_t<6, COLS>(job, blue, threads, stream);
-    case 7: return launch_axis_t<7, COLS>(job, blue, threads, stream);
-    case 8: return launch_axis_t<8, COLS>(job, blue, threads, stream);
-    case 9: return launch_axis_t<9, COLS>(job, blue, threads, stream);
-    case 10: return launch_axis_t<10, COLS>(job, blue, threads, stream);
-    case 11: return launch_axis_t<11, COLS>(job, blue, threads, stream);
-    case 12: return launch_axis_t<12, COLS>(job, blue, threads, stream);
-    case 13: return launch_axis_t<13, COLS>(job, blue, threads, stream);
-    case 14: return launch_axis_t<14, COLS>(job, blue, threads, stream);
-    case F3_BASE + 6: return launch_axis_t<F3_BASE + 6, COLS>(job, blue, threads, stream);
-    case F3_BASE + 7: return launch_axis_t<F3_BASE + 7, COLS>(job, blue, threads, stream);
-    case F3_BASE + 8: return launch_axis_t<F3_BASE + 8, COLS>(job, blue, threads, stream);
-    case F3_BASE + 9: return launch_axis_t<F3_BASE + 9, COLS>(job, blue, threads, stream);
-    case F3_BASE + 10: return launch_axis_t<F3_BASE + 10, COLS>(job, blue, threads, stream);
-    case F3_BASE + 11: return launch_axis_t<F3_BASE + 11, COLS>(job, blue, threads, stream);
+    const bool x2 = (shape & X2) != 0;
+    switch (base_of(shape)) {
+    case 1: return launch_axis_t<1, COLS>(job, blue, x2, threads, stream);
+    case 2: return launch_axis_t<2, COLS>(job, blue, x2, threads, stream);
+    case 3: return launch_axis_t<3, COLS>(job, blue, x2, threads, stream);
+    case 4: return launch_axis_t<4, COLS>(job, blue, x2, threads, stream);
+    case 5: return launch_axis_t<5, COLS>(job, blue, x2, threads, stream);
+    case 6: return launch_axis_t<6, COLS>(job, blue, x2, threads, stream);
+    case 7: return launch_axis_t<7, COLS>(job, blue, x2, threads, stream);
+    case 8: return launch_axis_t<8, COLS>(job, blue, x2, threads, stream);
+    case 9: return launch_axis_t<9, COLS>(job, blue, x2, threads, stream);
+    case 10: return launch_axis_t<10, COLS>(job, blue, x2, threads, stream);
+    case 11: return launch_axis_t<11, COLS>(job, blue, x2, threads, stream);
+    case 12: return launch_axis_t<12, COLS>(job, blue, x2, threads, stream);
+    case 13: return launch_axis_t<13, COLS>(job, blue, x2, threads, stream);
+    case 14: return launch_axis_t<14, COLS>(job, blue, x2, threads, stream);
+    case F3_BASE + 6: return launch_axis_t<F3_BASE + 6, COLS>(job, blue, x2, threads, stream);
+    case F3_BASE + 7: return launch_axis_t<F3_BASE + 7, COLS>(job, blue, x2, threads, stream);
+    case F3_BASE + 8: return launch_axis_t<F3_BASE + 8, COLS>(job, blue, x2, threads, stream);
+    case F3_BASE + 9: return launch_axis_t<F3_BASE + 9, COLS>(job, blue, x2, threads, stream);
+    case F3_BASE + 10: return launch_axis_t<F3_BASE + 10, COLS>(job, blue, x2, threads, stream);
+    case F3_BASE + 11: return launch_axis_t<F3_BASE + 11, COLS>(job, blue, x2, threads, stream);
     default: return hipErrorInvalidValue;
     }
 }

@@ -48,7 +48,7 @@ template <int S>
 static hipError_t launch_image_t(const AxisJob& job, const ImageIO& io, bool blue, bool cols, int mode, bool wide,
                                  hipStream_t stream)
 {
-    constexpr int TN = narrow_threads(S), TW = wide_threads(S, true, true), SW = wide_shape(S, true);
+    constexpr int TN = narrow_threads(S), TW = wide_threads(S, true, true), SW = has_x2(S) ? S | X2 : S;
     if (!cols) {
         if (mode == IO_LUM) return launch_image_tt<S, TN, false, IO_LUM>(job, io, blue, stream);
         if (mode == (IO_LUM | IO_MAG)) return launch_image_tt<S, TN, false, IO_LUM | IO_MAG>(job, io, blue, stream);

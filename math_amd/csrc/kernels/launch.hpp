@@ -95,22 +95,19 @@ hipError_t gen_chirp(double2* chirp64, float2* chirp32, float2* dir, int n, int 
 hipError_t gen_dir_diagonal(float2* dir, const float2* dtab, int n, int m, hipStream_t stream);
 hipError_t gen_dtab(float2* dtab, const double2* chirp64, double* cos_scratch, int n, int m, hipStream_t stream);
 
-// Workgroup sizes of the single-image kernels.  Narrow: 256 threads, or one
-// line when a line needs more (16384 points: 512).  Wide tiles hold more lines;
-// columns use the X2 form of a shape that has one:
-//  * direct columns 1024 threads (eight columns of 4096: 64-byte runs of a row;
-//    4096^2 113 us, 139 with 512), 512 where that leaves CUs without a tile;
-//  * Bluestein columns 512, so the two tiles of a CU overlap their arithmetic
-//    and their memory traffic (4093 x 2047 106 us, 122 with 1024);
-//  * 6144 points 512 (3000^2 184 us against 195), 8192 points 1024 (2048 x 8192
-//    128 us against 167).
+// Tiles of the single-image kernels: a workgroup size, and for columns of a
+// shape with an X2 form whether it takes that (launch_axis: shape | X2).
+// Narrow: 256 threads, or one line when a line needs more (16384 points: 512).
 __host__ __device__ constexpr int narrow_threads(int shape) { return tpl_of(shape) > 256 ? tpl_of(shape) : 256; }
-__host__ __device__ constexpr int wide_shape(int shape, bool cols) { return cols && has_x2(shape) ? shape | X2 : shape; }
+// the widest tiles: X2 columns in 1024 threads when direct, 512 for Bluestein
+// (Context::axis_tile); else 6144-point columns in 512 threads (3000^2 184 us
+// against 195 in 1024) and 1024 (8192-point columns, 2048 x 8192: 128 us against 167)
 __host__ __device__ constexpr int wide_threads(int shape, bool cols, bool blue)
 {
     return cols && (ept_of(shape) == 24 || (blue && has_x2(shape))) ? 512 : 1024;
 }
-// threads: 1024 or 512 wide tiles, 256 narrow, 128 or 64 small (clamped to one line per workgroup)
+// threads: 1024, 512 (wide tiles, clamped to the shape's), 256, 128 or 64 (clamped to one line per workgroup);
+// shape + X2: columns in 1024, 512 or 256 threads
 hipError_t launch_axis(int shape, const AxisJob& job, bool blue, bool cols, int threads, hipStream_t stream);
 
 // ---- lines of smooth length (smooth.hip) ----
