@@ -74,7 +74,8 @@ __device__ __forceinline__ float2 cscale(float2 a, float s) { return make_float2
 //  * S = F3_BASE + k: M = 3 * 2^k (Bluestein convolutions, and lines of
 //    exactly 3 * 2^k points transformed directly), 12 points per
 //    thread: radix-4 passes, one radix-2 pass when k is odd, and a final
-//    radix-12 pass (a 3 x 4 prime-factor butterfly).
+//    radix-12 pass (a 3 x 4 prime-factor butterfly).  6144 points: 24 per thread
+//    in passes 8 x 8 x 8 x 12 (six passes of radix 4 and 2 took up to 15 % longer).
 // The shape is a function of the line length and axis, so a line runs the
 // same schedule in every kernel.
 // S + X2: the same with two lines per thread (column tiles).  The lines of a tile share the
@@ -111,7 +112,7 @@ __host__ __device__ constexpr int ept_of(int s)
 __host__ __device__ constexpr int tpl_of(int s) { return m_of(s) / ept_of(s); }
 __host__ __device__ constexpr int npass_of(int s)
 {
-    return is_f3(s)     ? (f3_k(s) - 2) / 2 + (f3_k(s) - 2) % 2 + 1
+    return is_f3(s)     ? (f3_k(s) == 11 ? 4 : (f3_k(s) - 2) / 2 + (f3_k(s) - 2) % 2 + 1)
            : is_wide(s) ? 3
                         : (base_of(s) + 3) / 4;
 }
@@ -121,6 +122,7 @@ __host__ __device__ constexpr int radix_of(int s, int p)
     if (p >= npass_of(s)) return 1;
     if (is_f3(s)) {
         const int a = f3_k(s) - 2;
+        if (a == 9) return p < 3 ? 8 : 12;
         return p < a / 2 ? 4 : (p == npass_of(s) - 1 ? 12 : 2);
     }
     if (is_wide(s)) return p == 0 || (base_of(s) == 14 && p == 1) ? 32 : 16;
@@ -142,10 +144,15 @@ __host__ __device__ constexpr int ns_of(int s, int p)
 //    w^16, w^8, w^4 * {1, W8}, w^2 * {1, W16, W16^2, W16^3}, w * {1, W32, .. W32^7};
 //  * other radices: w^1, w^2, w^3, w^4; the other powers are products of these
 //    (expand_twiddles).
-__host__ __device__ constexpr int tw_row(int radix) { return radix == 32 ? 16 : 4; }
+//  * 6144 points (full_rows): w^1 .. w^7 for radix 8, w^1 .. w^6, w^8, w^10 for
+//    radix 12, so a product of two stands for three of them at most: with rows
+//    of four the error against FP64 was 5 % above that of radix-4 passes.
+__host__ __device__ constexpr bool full_rows(int s) { return is_f3(s) && f3_k(s) == 11; }
+__host__ __device__ constexpr int tw_row(int radix, bool full = false) { return full ? 8 : radix == 32 ? 16 : 4; }
 // entry e of row k: exp(-2*pi*i*q/(Ns*R)) with q = power * k + rotation * Ns*R/32
-__host__ __device__ constexpr int tw_power(int radix, int e)
+__host__ __device__ constexpr int tw_power(int radix, int e, bool full = false)
 {
+    if (full) return radix == 8 ? (e < 7 ? e + 1 : 0) : e < 6 ? e + 1 : 2 * e - 4;
     return radix == 16 ? (1 << e) : radix == 32 ? (e == 0 ? 16 : e == 1 ? 8 : e < 4 ? 4 : e < 8 ? 2 : 1) : e + 1;
 }
 __host__ __device__ constexpr int tw_rotation(int radix, int e)
@@ -154,7 +161,7 @@ __host__ __device__ constexpr int tw_rotation(int radix, int e)
 }
 __host__ __device__ constexpr int64_t tw_pass_len(int s, int p)
 {
-    return p >= 1 && p < npass_of(s) ? int64_t(ns_of(s, p)) * tw_row(radix_of(s, p)) : 0;
+    return p >= 1 && p < npass_of(s) ? int64_t(ns_of(s, p)) * tw_row(radix_of(s, p), full_rows(s)) : 0;
 }
 __host__ __device__ constexpr int64_t tw_pass_off(int s, int p)
 {
@@ -185,7 +192,7 @@ __host__ __device__ constexpr int64_t tw_total() { return tw_off(F3_BASE + F3_MA
 // word p + c * (p >> sh) of the line's slice, with (c, sh) chosen per FFT
 // shape, workgroup size, axis and pass by gen_lds_maps.py (lds_maps.inc) so
 // that (a) offsets stay linear, f(t + i*TPL) = f(t) + f(i*TPL) for the next
-// pass's reads and f(base + r*NS) = f(base) + r*f(NS) for this pass's writes,
+// pass's reads and f(base + r*NS) = f(base) + f(r*NS) for this pass's writes,
 // making every LDS access a base register plus an immediate, and (b) no
 // write or read instruction has a bank conflict (32 banks, 32 lanes per cycle).
 struct LdsMap {
@@ -696,17 +703,17 @@ __device__ __forceinline__ void exchange_sync()
 // ahead (pass 1's with the tile's input), so the table latency overlaps the
 // LDS exchange instead of following it.
 // float4s of a row a radix-R butterfly reads
-template <int R>
+template <int R, bool FULL = false>
 __host__ __device__ constexpr int tw_quads()
 {
-    return R <= 2 ? 1 : R == 32 ? 8 : 2;
+    return R <= 2 ? 1 : tw_row(R, FULL) / 2;
 }
 
 template <int S, int THREADS, int P>
 struct TwLoad {
     using C = LineCfg<S, THREADS>;
     static constexpr int R = radix_of(S, P);
-    static constexpr int Q = tw_quads<R>();
+    static constexpr int Q = tw_quads<R, full_rows(S)>();
     static constexpr int NB = C::EPT / R;
     static constexpr int NS = ns_of(S, P);
     static_assert(NB * Q <= C::EPT / 2, "twiddle registers");
@@ -718,7 +725,7 @@ struct TwLoad {
             // the second float4 of a row is an immediate offset away
 #pragma unroll
             for (int r2 = 0; r2 < Q; ++r2)
-                w[b * Q + r2] = load4_at(tw + tw_pass_off(S, P), uint32_t(k) * uint32_t(8 * tw_row(R)) + 16u * r2);
+                w[b * Q + r2] = load4_at(tw + tw_pass_off(S, P), uint32_t(k) * uint32_t(8 * tw_row(R, full_rows(S))) + 16u * r2);
         }
     }
 };
@@ -738,9 +745,21 @@ __device__ __forceinline__ void expand_products(float2 (&wt)[R])
     }
 }
 
-template <int R>
+template <int R, bool FULL = false>
 __device__ __forceinline__ void expand_twiddles(float2 (&wt)[R], const float4* q)
 {
+    if constexpr (FULL) {
+        static_assert(R == 8 || R == 12, "radix");
+#pragma unroll
+        for (int e = 0; e < (R == 8 ? 7 : 8); ++e)
+            wt[tw_power(R, e, true)] = e % 2 ? make_float2(q[e / 2].z, q[e / 2].w) : make_float2(q[e / 2].x, q[e / 2].y);
+        if constexpr (R == 12) {
+            wt[7] = cmul(wt[4], wt[3]);
+            wt[9] = cmul(wt[8], wt[1]);
+            wt[11] = cmul(wt[8], wt[3]);
+        }
+        return;
+    }
     wt[1] = make_float2(q[0].x, q[0].y);
     if constexpr (R > 2) {
         wt[2] = make_float2(q[0].z, q[0].w);
@@ -778,12 +797,11 @@ struct FftPass {
         for (int b = 0; b < NB; ++b) {
             const int j = t + b * C::TPL;
             const int k = j & (NS - 1);
-            const int base = (j - k) * R + k;
-            // the layout keeps the R outputs' offsets linear: each step adds f(NS)
-            constexpr int step = lds_pos<S, THREADS, COLS, P>(NS);
-            const int q0 = lds_pos<S, THREADS, COLS, P>(base);
+            const int q0 = lds_pos<S, THREADS, COLS, P>((j - k) * R + k);
+            // the layout keeps the R outputs' offsets linear: f(base) + f(r*NS)
 #pragma unroll
-            for (int r = 0; r < R; ++r) plane[q0 + r * step] = c == 0 ? v[b + NB * r].x : v[b + NB * r].y;
+            for (int r = 0; r < R; ++r)
+                plane[q0 + lds_pos<S, THREADS, COLS, P>(r * NS)] = c == 0 ? v[b + NB * r].x : v[b + NB * r].y;
         }
     }
 
@@ -856,7 +874,7 @@ struct FftPass {
                 for (int r = 0; r < R; ++r) u[r] = v[l][b + NB * r];
                 if constexpr (P > 0) {
                     // the same for the thread's lines
-                    constexpr int Q = tw_quads<R>();
+                    constexpr int Q = tw_quads<R, full_rows(S)>();
                     float4 q[Q];
 #pragma unroll
                     for (int r2 = 0; r2 < Q; ++r2) q[r2] = w[b * Q + r2];
@@ -864,7 +882,7 @@ struct FftPass {
                         dft_twiddled<R>(u, q);
                     } else {
                         float2 wt[R];
-                        expand_twiddles<R>(wt, q);
+                        expand_twiddles<R, full_rows(S)>(wt, q);
 #pragma unroll
                         for (int r = 1; r < R; ++r) u[r] = cmul(u[r], wt[r]);
                         dft_fwd<R>(u);

@@ -39,6 +39,8 @@ def tpl_of(s):
 def radices(s):
     if is_f3(s):
         a = s - F3_BASE - 2
+        if a == 9:
+            return [8, 8, 8, 12]
         return [4] * (a // 2) + [2] * (a % 2) + [12]
     if s >= 13:
         return [32, 16, 16] if s == 13 else [32, 32, 16]

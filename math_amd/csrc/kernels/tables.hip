@@ -21,15 +21,15 @@ __device__ __forceinline__ double2 unit_root(int64_t q, int64_t den)
 }
 
 // row k of a pass: tw_row entries (tw_power, tw_rotation) of w = exp(-2*pi*i*k/(ns*radix))
-__global__ void k_gen_twiddle_block(float2* out, int ns, int radix)
+__global__ void k_gen_twiddle_block(float2* out, int ns, int radix, bool full)
 {
     const int64_t idx = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     const int64_t len = int64_t(ns) * radix;
-    const int row = tw_row(radix);
+    const int row = tw_row(radix, full);
     if (idx >= int64_t(ns) * row) return;
     const int64_t k = idx / row;
     const int e = (int)(idx % row);
-    const double2 w = unit_root((k * tw_power(radix, e) + tw_rotation(radix, e) * (len / 32)) % len, len);
+    const double2 w = unit_root((k * tw_power(radix, e, full) + tw_rotation(radix, e) * (len / 32)) % len, len);
     out[idx] = make_float2((float)w.x, (float)w.y);
 }
 
@@ -142,7 +142,8 @@ hipError_t gen_twiddles(float2* table, hipStream_t stream)
             const int64_t len = tw_pass_len(shape, p);
             float2* out = table + tw_off(shape) + tw_pass_off(shape, p);
             const int blocks = (int)((len + 255) / 256);
-            hipLaunchKernelGGL(k_gen_twiddle_block, dim3(blocks), dim3(256), 0, stream, out, ns, radix);
+            hipLaunchKernelGGL(k_gen_twiddle_block, dim3(blocks), dim3(256), 0, stream, out, ns, radix,
+                               full_rows(shape));
         }
     };
     for (int logm = 1; logm <= MAX_LOGM; ++logm) shape_rows(logm);
