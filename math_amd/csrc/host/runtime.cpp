@@ -98,19 +98,19 @@ void search_passes(int n, int left, int max_index, std::vector<int>& now, std::v
 
 }  // namespace
 
-bool smooth_plan(long long n, GenPlan* plan)
+// the plan of one length (smooth_plan), false where there is none
+static bool make_smooth_plan(int n, GenPlan* plan)
 {
-    if (n < 17 || n > GEN_MAX_N || is_pow2((uint64_t)n)) return false;
-    if (n % 3 == 0 && is_pow2((uint64_t)(n / 3)) && n >= (3LL << F3_MIN_K)) return false;
-    long long rest = n;
+    if (is_pow2((uint64_t)n)) return false;
+    if (n % 3 == 0 && is_pow2((uint64_t)(n / 3)) && n >= (3 << F3_MIN_K)) return false;
+    int rest = n;
     for (int f : {2, 3, 5, 7})
         while (rest % f == 0) rest /= f;
     if (rest != 1) return false;
     std::vector<int> now, best;
     int tpl = 0;
-    search_passes((int)n, (int)n, 0, now, best, tpl);
+    search_passes(n, n, 0, now, best, tpl);
     if (best.size() < 2) return false;
-    if (!plan) return true;
     // an odd radix first (its scatter's stride meets every LDS bank), then ascending: the largest radix last has
     // the fewest twiddle rows
     std::sort(best.begin(), best.end());
@@ -119,7 +119,7 @@ bool smooth_plan(long long n, GenPlan* plan)
         if (*it % 2) odd = it;
     if (odd != best.end()) std::rotate(best.begin(), odd, odd + 1);
     *plan = GenPlan{};
-    plan->n = (int)n;
+    plan->n = n;
     plan->npass = (int)best.size();
     plan->tpl = tpl;
     int ns = 1;
@@ -127,10 +127,32 @@ bool smooth_plan(long long n, GenPlan* plan)
         GenPass& g = plan->pass[p];
         g.radix = best[p];
         g.ns = ns;
-        g.nbf = (int)n / best[p];
+        g.nbf = n / best[p];
         g.magic = ns > 1 ? (uint32_t)(((uint64_t(1) << 32) + ns - 1) / ns) : 0u;
         ns *= best[p];
     }
+    return true;
+}
+
+bool smooth_plan(long long n, GenPlan* plan)
+{
+    // every length's plan once per process: line_shape asks for every image of every batch
+    struct Table {
+        std::vector<GenPlan> plans;
+        std::vector<int16_t> index;  // -1: none
+        Table() : index(GEN_MAX_N + 1, int16_t(-1))
+        {
+            for (int i = 17; i <= GEN_MAX_N; ++i) {
+                GenPlan p;
+                if (!make_smooth_plan(i, &p)) continue;
+                index[i] = (int16_t)plans.size();
+                plans.push_back(p);
+            }
+        }
+    };
+    static const Table table;
+    if (n < 17 || n > GEN_MAX_N || table.index[n] < 0) return false;
+    if (plan) *plan = table.plans[table.index[n]];
     return true;
 }
 
@@ -254,6 +276,7 @@ Context::Context(int device) : device_(device)
     hip_check(warm_whole(word, gen_stream_), "kernel load");
     hip_check(hipStreamSynchronize(gen_stream_), "kernel load");
     noalloc_setup(device);
+    (void)smooth_plan(17, nullptr);  // builds the table of smooth lengths
     // default tile shapes: wide tiles for columns of 1024 points and more
     for (int i = 0; i < NSHAPES; ++i) {
         const int shape = i <= MAX_LOGM ? i : F3_BASE + F3_MIN_K + (i - MAX_LOGM - 1);
