@@ -1084,23 +1084,31 @@ __device__ __forceinline__ void line_tile(const AxisJob& job, int tile, float* l
     }
 
     const float sc = job.scale;
+    // The output's addresses: with two lines per thread worked out anew from
+    // the thread index, since the input's would be kept (and spilled) through
+    // both FFTs, 48 bytes of scratch traffic a thread.
+    const int tid_o = L == 2 ? opaque(tid) : tid;
+    const int slot_o = COLS ? (tid_o % C::SLOTS) : (tid_o / C::TPL);
+    const int t_o = COLS ? (tid_o / C::SLOTS) : (tid_o % C::TPL);
     // finished slot i of the thread's lines into the output
     auto put = [&](int i, const float2 (&y)[L]) {
-        const uint32_t pos = uint32_t(t + i * C::TPL);
+        const uint32_t pos = uint32_t(t_o + i * C::TPL);
         if (!in_line((int)pos)) return;
+        const int first = tile * C::LPW + (COLS ? slot_o * L : slot_o);  // the thread's first line
         if constexpr (IO == 0 && L == 2) {
             if (pairs) {
-                store_pair(job.dst + base[0] + i * step, y[0], y[L - 1]);
+                store_pair(job.dst + int64_t(first) * job.ls + int64_t(t_o) * job.es + i * step, y[0], y[L - 1]);
                 return;
             }
         }
 #pragma unroll
         for (int l = 0; l < L; ++l) {
-            if (!valid(l)) continue;
+            const int line = first + (COLS ? l : l * C::SLOTS);
+            if (line >= job.count) continue;
             if constexpr ((IO & IO_MAG) != 0)
-                io.mag[int64_t(line_of(l)) * io.mls + int64_t(pos) * io.mel] = cabs_scaled(y[l], io.mscale);
+                io.mag[int64_t(line) * io.mls + int64_t(pos) * io.mel] = cabs_scaled(y[l], io.mscale);
             else if constexpr (COLS)
-                store_global(job.dst + base[l] + i * step, y[l]);
+                store_global(job.dst + int64_t(line) * job.ls + int64_t(t_o) * job.es + i * step, y[l]);
             else
                 store_at(job.dst + base[l] + i * step, off[l], y[l]);
         }
