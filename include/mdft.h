@@ -135,9 +135,11 @@ int mdft_exec_device_noalloc(uint32_t width, uint32_t height, int inverse, const
  * shape: 1..14 for 2^shape points, 38..43 for 3 * 2^(shape - 32) points
  * (lines of exactly 3 * 2^k points, and the Bluestein convolution length used
  * when 3 * 2^k >= 2n - 1 is shorter than the reference's compute_m(n): along
- * columns from 192 points, along rows from 3072); Bluestein (blue != 0) or power-of-two, along
- * rows (cols == 0) or columns: 0 = 256-thread tiles, 1 = 1024-thread tiles
- * (four times the lines per tile).  No counterpart in the reference, whose
+ * columns from 192 points, along rows from 3072); Bluestein (blue != 0) or direct, along
+ * rows (cols == 0) or columns: 0 = 256-thread tiles, 1 = wider ones
+ * (up to 1024 threads, for columns with two lines per thread where the length
+ * has that, when enough of them fill the device).  Other smooth lengths (17 to
+ * 4096 points) have no entry.  No counterpart in the reference, whose
  * tile size follows the device's shared-memory limit
  * (src/gpu/dft/fft.cpp:51-61, function.cpp:94-118); this build picks it per
  * shape by measurement. */

@@ -4,22 +4,24 @@
 // element stride es and line stride ls inside a row-major complex<float>
 // image (rows: es = 1, ls = w; columns: es = w, ls = 1).  A line of length n
 // is transformed through an FFT of length M: directly when n is a power of
-// two or 3 * 2^k in [192, 6144] (M = n), otherwise by Bluestein's chirp-z
+// two or 3 * 2^k in [192, 6144] (M = n; other smooth lengths run in
+// smooth_device.hpp), otherwise by Bluestein's chirp-z
 // method with M >= 2n - 1: the reference's padded length bit_ceil(2n - 2)
 // (src/gpu/dft/function.cpp:32-45), or 3 * 2^k when that is shorter, and the
 // chirp tables of function.cpp:49-92 generated in FP64 on the device.
 //
-// A workgroup owns LPW whole lines (a "tile").  Each thread holds EPT = 16
-// points of one line in VGPRs, at positions t + i*TPL (TPL = M/16 threads per
-// line).  The FFT is a radix-16 Stockham autosort (passes of 16 and one
-// remainder pass), DIT form: pass p gathers its operands from LDS at the
-// thread's fixed positions, multiplies by the per-pass twiddle row, runs a
-// radix-R butterfly in registers and scatters to the Stockham positions.  The
-// first pass needs no twiddles and reads straight from HBM; the last pass
-// leaves its results at the thread's own positions, so it writes straight to
-// HBM and Bluestein's two FFTs chain without an LDS exchange.  LDS holds one
-// exchange buffer, split into real and imaginary planes with one pad word per
-// 16 to keep the scatter conflict-free.
+// A workgroup owns LPW whole lines (a "tile").  Each thread holds EPT points
+// (16, 32, 12 or 24, see the shapes below) of one line or of two in VGPRs, at
+// positions t + i*TPL (TPL = M/EPT threads per line).  The FFT is a Stockham
+// autosort in passes of up to radix 32, DIT form: pass p gathers its operands
+// from LDS at the thread's fixed positions, runs a radix-R butterfly with the
+// pass's twiddle row fused into it in registers and scatters to the Stockham
+// positions.  The first pass needs no twiddles and reads straight from HBM; the
+// last pass leaves its results at the thread's own positions, so it writes
+// straight to HBM and Bluestein's two FFTs chain without an LDS exchange.  LDS
+// holds one exchange buffer of real and imaginary planes (one plane, used twice,
+// for 24 and 32 points per thread) in the layouts of lds_maps.inc, conflict-free
+// for every exchange.
 //
 // Only the forward FFT exists: an inverse transform is conj(FFT(conj(x))),
 // folded into the load, the D multiply and the store.
