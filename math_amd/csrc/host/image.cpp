@@ -118,7 +118,7 @@ int mdft_image_exec_device(mdft_image image, const void* src, uint32_t src_width
         if (row.gen)
             launch(mdft::launch_smooth_image(j, io, false, mode, 256, s), "image row pass launch");
         else
-            launch(mdft::launch_image_axis(row.shape, j, io, row.blue, false, mode, false, s), "image row pass launch");
+            launch(mdft::launch_image_axis(row.shape, j, io, row.blue, false, mode, 256, s), "image row pass launch");
     }
     if (h > 1) {
         // columns: magnitude out; luminance in as well when there was no row pass
@@ -130,8 +130,9 @@ int mdft_image_exec_device(mdft_image image, const void* src, uint32_t src_width
             launch(mdft::launch_smooth_image(j, io, true, mode, ctx.smooth_threads(col.smooth, true, w), s),
                    "image column pass launch");
         } else {
-            const bool wide = ctx.axis_tile(col.shape, col.blue, true, w).threads >= 512;
-            launch(mdft::launch_image_axis(col.shape, j, io, col.blue, true, mode, wide, s),
+            const Context::AxisTile tile = ctx.axis_tile(col.shape, col.blue, true, w);
+            launch(mdft::launch_image_axis(tile.x2 ? col.shape | mdft::X2 : col.shape, j, io, col.blue, true, mode,
+                                           tile.threads, s),
                    "image column pass launch");
         }
     }

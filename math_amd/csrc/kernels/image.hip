@@ -31,7 +31,8 @@ static hipError_t launch_image_tt(const AxisJob& job, const ImageIO& io, bool bl
     if (grid64 == 0) return hipSuccess;
     const unsigned grid = (unsigned)grid64;
     if (blue) {
-        if constexpr (S >= 2)
+        // Bluestein X2 columns take 512 threads at most (Context::axis_tile)
+        if constexpr (base_of(S) >= 2 && !((S & X2) && T == 1024))
             hipLaunchKernelGGL((k_image_axis<S, T, true, COLS, IO>), dim3(grid), dim3(T), 0, stream, job, io);
         else
             return hipErrorInvalidValue;
@@ -42,20 +43,44 @@ static hipError_t launch_image_tt(const AxisJob& job, const ImageIO& io, bool bl
 }
 
 // rows: IO_LUM, or IO_LUM|IO_MAG for a one-row image; columns: IO_MAG, or
-// IO_LUM|IO_MAG for a one-column image.  Wide tiles only for the column
-// pass that stores magnitudes (the shape of the ordinary column pass).
+// IO_LUM|IO_MAG for a one-column image.  The column pass that stores
+// magnitudes takes the tile of the ordinary column pass (launch_axis: wide and
+// X2 forms), the other passes narrow ones.  Magnitudes leave a thread with two
+// lines as two single words where complex results leave in one store, so direct
+// X2 columns below 3072 points gain from 512 threads only (2050 x 1024: 39.2 us
+// in 256 threads, 35.0 narrow; 6200 x 2048: 173 in 1024, 167 in 512), longer
+// ones as the ordinary pass (4096 x 4096: 154 in 1024, 171 in 512; 600 x 4096:
+// 39.2 in 256, 40.8 narrow), Bluestein ones as well (1540 x 2047: 57.1 in 256,
+// 62.9 narrow).
 template <int S>
-static hipError_t launch_image_t(const AxisJob& job, const ImageIO& io, bool blue, bool cols, int mode, bool wide,
-                                 hipStream_t stream)
+static hipError_t launch_image_t(const AxisJob& job, const ImageIO& io, bool blue, bool x2, bool cols, int mode,
+                                 int threads, hipStream_t stream)
 {
-    constexpr int TN = narrow_threads(S), TW = wide_threads(S, true, true), SW = has_x2(S) ? S | X2 : S;
+    constexpr int TN = narrow_threads(S);
+    if (x2) {
+        if constexpr (has_x2(S)) {
+            if (!cols || mode != IO_MAG) return hipErrorInvalidValue;
+            constexpr bool LONG = m_of(S) >= 3072;
+            if constexpr (LONG) {
+                if (threads >= 1024) return launch_image_tt<S | X2, 1024, true, IO_MAG>(job, io, blue, stream);
+            }
+            if (threads >= 512) return launch_image_tt<S | X2, 512, true, IO_MAG>(job, io, blue, stream);
+            if (LONG || blue) return launch_image_tt<S | X2, 256, true, IO_MAG>(job, io, blue, stream);
+            return launch_image_tt<S, TN, true, IO_MAG>(job, io, blue, stream);
+        } else {
+            return hipErrorInvalidValue;
+        }
+    }
     if (!cols) {
         if (mode == IO_LUM) return launch_image_tt<S, TN, false, IO_LUM>(job, io, blue, stream);
         if (mode == (IO_LUM | IO_MAG)) return launch_image_tt<S, TN, false, IO_LUM | IO_MAG>(job, io, blue, stream);
         return hipErrorInvalidValue;
     }
     if (mode == IO_MAG) {
-        if (wide) return launch_image_tt<SW, TW, true, IO_MAG>(job, io, blue, stream);
+        if constexpr (!has_x2(S)) {
+            if (threads >= 512 && threads > TN)
+                return launch_image_tt<S, wide_threads(S, true, false), true, IO_MAG>(job, io, blue, stream);
+        }
         return launch_image_tt<S, TN, true, IO_MAG>(job, io, blue, stream);
     }
     if (mode == (IO_LUM | IO_MAG)) return launch_image_tt<S, TN, true, IO_LUM | IO_MAG>(job, io, blue, stream);
@@ -63,29 +88,30 @@ static hipError_t launch_image_t(const AxisJob& job, const ImageIO& io, bool blu
 }
 
 hipError_t launch_image_axis(int shape, const AxisJob& job, const ImageIO& io, bool blue, bool cols, int mode,
-                             bool wide, hipStream_t stream)
+                             int threads, hipStream_t stream)
 {
-    switch (shape) {
-    case 1: return launch_image_t<1>(job, io, blue, cols, mode, wide, stream);
-    case 2: return launch_image_t<2>(job, io, blue, cols, mode, wide, stream);
-    case 3: return launch_image_t<3>(job, io, blue, cols, mode, wide, stream);
-    case 4: return launch_image_t<4>(job, io, blue, cols, mode, wide, stream);
-    case 5: return launch_image_t<5>(job, io, blue, cols, mode, wide, stream);
-    case 6: return launch_image_t<6>(job, io, blue, cols, mode, wide, stream);
-    case 7: return launch_image_t<7>(job, io, blue, cols, mode, wide, stream);
-    case 8: return launch_image_t<8>(job, io, blue, cols, mode, wide, stream);
-    case 9: return launch_image_t<9>(job, io, blue, cols, mode, wide, stream);
-    case 10: return launch_image_t<10>(job, io, blue, cols, mode, wide, stream);
-    case 11: return launch_image_t<11>(job, io, blue, cols, mode, wide, stream);
-    case 12: return launch_image_t<12>(job, io, blue, cols, mode, wide, stream);
-    case 13: return launch_image_t<13>(job, io, blue, cols, mode, wide, stream);
-    case 14: return launch_image_t<14>(job, io, blue, cols, mode, wide, stream);
-    case F3_BASE + 6: return launch_image_t<F3_BASE + 6>(job, io, blue, cols, mode, wide, stream);
-    case F3_BASE + 7: return launch_image_t<F3_BASE + 7>(job, io, blue, cols, mode, wide, stream);
-    case F3_BASE + 8: return launch_image_t<F3_BASE + 8>(job, io, blue, cols, mode, wide, stream);
-    case F3_BASE + 9: return launch_image_t<F3_BASE + 9>(job, io, blue, cols, mode, wide, stream);
-    case F3_BASE + 10: return launch_image_t<F3_BASE + 10>(job, io, blue, cols, mode, wide, stream);
-    case F3_BASE + 11: return launch_image_t<F3_BASE + 11>(job, io, blue, cols, mode, wide, stream);
+    const bool x2 = (shape & X2) != 0;
+    switch (base_of(shape)) {
+    case 1: return launch_image_t<1>(job, io, blue, x2, cols, mode, threads, stream);
+    case 2: return launch_image_t<2>(job, io, blue, x2, cols, mode, threads, stream);
+    case 3: return launch_image_t<3>(job, io, blue, x2, cols, mode, threads, stream);
+    case 4: return launch_image_t<4>(job, io, blue, x2, cols, mode, threads, stream);
+    case 5: return launch_image_t<5>(job, io, blue, x2, cols, mode, threads, stream);
+    case 6: return launch_image_t<6>(job, io, blue, x2, cols, mode, threads, stream);
+    case 7: return launch_image_t<7>(job, io, blue, x2, cols, mode, threads, stream);
+    case 8: return launch_image_t<8>(job, io, blue, x2, cols, mode, threads, stream);
+    case 9: return launch_image_t<9>(job, io, blue, x2, cols, mode, threads, stream);
+    case 10: return launch_image_t<10>(job, io, blue, x2, cols, mode, threads, stream);
+    case 11: return launch_image_t<11>(job, io, blue, x2, cols, mode, threads, stream);
+    case 12: return launch_image_t<12>(job, io, blue, x2, cols, mode, threads, stream);
+    case 13: return launch_image_t<13>(job, io, blue, x2, cols, mode, threads, stream);
+    case 14: return launch_image_t<14>(job, io, blue, x2, cols, mode, threads, stream);
+    case F3_BASE + 6: return launch_image_t<F3_BASE + 6>(job, io, blue, x2, cols, mode, threads, stream);
+    case F3_BASE + 7: return launch_image_t<F3_BASE + 7>(job, io, blue, x2, cols, mode, threads, stream);
+    case F3_BASE + 8: return launch_image_t<F3_BASE + 8>(job, io, blue, x2, cols, mode, threads, stream);
+    case F3_BASE + 9: return launch_image_t<F3_BASE + 9>(job, io, blue, x2, cols, mode, threads, stream);
+    case F3_BASE + 10: return launch_image_t<F3_BASE + 10>(job, io, blue, x2, cols, mode, threads, stream);
+    case F3_BASE + 11: return launch_image_t<F3_BASE + 11>(job, io, blue, x2, cols, mode, threads, stream);
     default: return hipErrorInvalidValue;
     }
 }

@@ -126,9 +126,9 @@ hipError_t gen_smooth(float2* out, const GenPlan& plan, hipStream_t stream);
 hipError_t warm_smooth(uint32_t* word, hipStream_t stream);
 
 // image path: an axis pass with fused luminance input and/or magnitude output
-// (mode = IO_LUM | IO_MAG bits), and the unfused conversions
+// (mode = IO_LUM | IO_MAG bits), and the unfused conversions; shape and threads as launch_axis
 hipError_t launch_image_axis(int shape, const AxisJob& job, const ImageIO& io, bool blue, bool cols, int mode,
-                             bool wide, hipStream_t stream);
+                             int threads, hipStream_t stream);
 hipError_t launch_image_luminance(const ImageIO& io, float2* dst, int w, int h, hipStream_t stream);
 hipError_t launch_image_magnitude(const ImageIO& io, const float2* src, int w, int h, hipStream_t stream);
 

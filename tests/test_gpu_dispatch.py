@@ -7,7 +7,7 @@ import statistics
 import numpy as np
 import pytest
 
-from tests.helpers import rand_c64
+from tests.helpers import rand_c64, tol_nl2
 
 pytestmark = pytest.mark.gpu
 
@@ -92,3 +92,55 @@ def test_short_rows_at_tile_edges(mdft, n, count):
         err = np.linalg.norm(got[1:-1].reshape(count, n) - ref) / np.linalg.norm(ref)
         assert err <= 2e-6 * max(1.0, np.log2(n)), (inv, err)
     f.close()
+
+
+# The view's columns run in the plan's tiles: 16384-point columns of an image too narrow for wide tiles (8, 70 and
+# 131 columns of one line each: 26, 37 and 41 us with 256 + 256 threads a line, 37, 46 and 51 in 1024-thread tiles
+# that leave most CUs idle).
+@pytest.mark.parametrize("w,h", [(8, 5681), (70, 6510), (131, 5715)])
+def test_narrow_image_columns_cost_what_the_plan_costs(mdft, w, h):
+    import torch
+
+    pixels = torch.zeros((h, w, 4), dtype=torch.uint8, device="cuda")
+    mag = torch.empty((h, w), dtype=torch.float32, device="cuda")
+    src = torch.zeros(w * h, dtype=torch.complex64, device="cuda")
+    dst = torch.empty_like(src)
+    image, plan = mdft.Image(w, h, mdft.PIXEL_RGBA8), mdft.Plan(w, h)
+    print(f"image columns {w}x{h}", flush=True)
+    r = time_ratio(captured(lambda st: image.exec_device(pixels.data_ptr(), w, h, w, 0, 0, mag.data_ptr(), w, st)),
+                   captured(lambda st: plan.exec_device(False, src.data_ptr(), dst.data_ptr(), st)))
+    image.close()
+    plan.close()
+    assert r <= 1.15, r
+
+
+# Columns with magnitudes in every tile the plan's rule picks on 256 CUs, the last tile short of a column or a pair:
+# (width, height, tile threads, two lines per thread)
+IMAGE_COLUMNS = [(3067, 4096, 1024, True), (2049, 2048, 512, True), (1025, 2048, 256, True), (515, 4096, 256, True),
+                 (3841, 1021, 512, True), (1923, 1201, 512, True), (1923, 2047, 512, True), (1283, 2047, 256, True),
+                 (2561, 701, 256, True), (5121, 509, 256, True), (1027, 8192, 1024, False), (515, 2999, 512, False),
+                 (513, 6007, 1024, False), (61, 6007, 512, False), (192, 71, 256, False), (60, 139, 128, False)]
+
+
+# and of a smooth height (1921 x 1080: 512 threads)
+@pytest.mark.parametrize("w,h", [c[:2] for c in IMAGE_COLUMNS] + [(1921, 1080), (31, 1080)])
+def test_image_columns_in_every_tile(mdft, w, h):
+    import torch
+
+    g = torch.Generator(device="cuda")
+    g.manual_seed(w + h)
+    x, y, sw, pitch, out = 2, 1, w + 4, w + 9, w + 3
+    px = torch.rand((h + 2, pitch, 4), dtype=torch.float32, device="cuda", generator=g)
+    dst = torch.full((h, out), -7.0, dtype=torch.float32, device="cuda")
+    image = mdft.Image(w, h, mdft.PIXEL_RGBA32F)
+    print(f"image columns {w}x{h}", flush=True)
+    image.exec_device(px.data_ptr(), sw, h + 2, pitch, x, y, dst.data_ptr(), out,
+                      torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    image.close()
+    assert bool((dst[:, w:] == -7.0).all())
+    lum = px[y:y + h, x:x + w, :3].cpu().to(torch.float64) @ torch.tensor([0.2126, 0.7152, 0.0722],
+                                                                          dtype=torch.float64)
+    ref = torch.fft.fft2(lum).abs() / (w * h)
+    err = torch.linalg.norm(dst[:, :w].cpu().to(torch.float64) - ref) / torch.linalg.norm(ref)
+    assert err <= tol_nl2(w, h), float(err)
