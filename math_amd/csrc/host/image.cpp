@@ -130,7 +130,7 @@ int mdft_image_exec_device(mdft_image image, const void* src, uint32_t src_width
             launch(mdft::launch_smooth_image(j, io, true, mode, ctx.smooth_threads(col.smooth, true, w), s),
                    "image column pass launch");
         } else {
-            const Context::AxisTile tile = ctx.axis_tile(col.shape, col.blue, true, w);
+            const mdft::AxisTile tile = ctx.axis_tile(col.shape, col.blue, true, w);
             launch(mdft::launch_image_axis(tile.x2 ? col.shape | mdft::X2 : col.shape, j, io, col.blue, true, mode,
                                            tile.threads, s),
                    "image column pass launch");

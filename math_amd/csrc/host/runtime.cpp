@@ -718,14 +718,14 @@ void Context::enqueue_axis(const LinePlan& lp, const float2* src, float2* dst, i
 //    with 512, 51.5 narrow; 4001 x 701 49.2, 52.1; 2049 x 701, two tiles per CU,
 //    31.6, 29.4 narrow);
 //  * other wide tiles from one per CU.
-Context::AxisTile Context::axis_tile(int shape, bool blue, bool cols, int count) const
+AxisTile axis_tile(int shape, bool blue, bool cols, int count, int variant, int cu_count)
 {
-    if (variant(shape, blue, cols) != 0) {
+    if (variant != 0) {
         const bool x2 = cols && has_x2(shape);
         // tiles of t threads, in eighths of the CUs
         auto per_cu8 = [&](int t) {
             const int64_t lines = int64_t(t) / tpl_of(shape) * (x2 ? 2 : 1);
-            return lines < 1 ? int64_t(0) : 8 * ((int64_t(count) + lines - 1) / lines) / cu_count_;
+            return lines < 1 ? int64_t(0) : 8 * ((int64_t(count) + lines - 1) / lines) / cu_count;
         };
         if (x2 && blue) {
             if (m_of(shape) >= 2048 && per_cu8(512) >= 15) return {512, true};
@@ -742,7 +742,7 @@ Context::AxisTile Context::axis_tile(int shape, bool blue, bool cols, int count)
     // points) so every CU gets work; rows aim at four tiles per CU, columns at
     // one, since narrower column tiles read shorter runs of each row
     const int tpl = tpl_of(shape);
-    const int64_t want = int64_t(cols ? 1 : 4) * cu_count_;
+    const int64_t want = int64_t(cols ? 1 : 4) * cu_count;
     int t = tpl > 256 ? tpl : 256;
     while (t > 64 && t / 2 >= tpl && (int64_t(count) + t / tpl - 1) / (t / tpl) < want) t /= 2;
     return {t, false};

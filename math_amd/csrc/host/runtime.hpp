@@ -50,6 +50,15 @@ int line_shape(long long n, bool cols);
 constexpr int NSHAPES = MAX_LOGM + 1 + (F3_MAX_K - F3_MIN_K + 1);
 inline int shape_index(int shape) { return is_f3(shape) ? MAX_LOGM + 1 + (f3_k(shape) - F3_MIN_K) : shape; }
 
+// Tile of a single-image pass (launch_axis): threads, and whether columns take
+// the two-lines-per-thread form, for `count` lines on cu_count CUs (variant: the
+// entry of the context's tile table).
+struct AxisTile {
+    int threads;
+    bool x2;
+};
+AxisTile axis_tile(int shape, bool blue, bool cols, int count, int variant, int cu_count);
+
 // Lines whose padded length is 2^three_factor_min_logm() or more split in
 // three factors (2^29 unless MDFT_LARGE_SPLIT3_LOGM in [15, 29] says otherwise,
 // read once per process: a testing knob that runs the three-factor steps on
@@ -166,12 +175,11 @@ public:
     // Tile table of the single-image kernels: variant 0 = narrow (256-thread)
     // tiles, 1 = wide ones where enough of them remain, per (FFT shape, blue, cols).
     int variant(int shape, bool blue, bool cols) const { return variant_[shape_index(shape)][blue][cols]; }
-    // tile of a single-image pass of `count` lines (launch_axis)
-    struct AxisTile {
-        int threads;
-        bool x2;
-    };
-    AxisTile axis_tile(int shape, bool blue, bool cols, int count) const;
+    // tile of a single-image pass of `count` lines under that table
+    AxisTile axis_tile(int shape, bool blue, bool cols, int count) const
+    {
+        return mdft::axis_tile(shape, blue, cols, count, variant(shape, blue, cols), cu_count_);
+    }
     static bool one_tile(const LinePlan& row, const LinePlan& col, int w, int h);
     // workgroup size of a pass over `count` lines of a smooth length (launch_smooth)
     int smooth_threads(const GenPlan& plan, bool cols, int count) const;

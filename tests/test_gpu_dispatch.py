@@ -114,12 +114,13 @@ def test_narrow_image_columns_cost_what_the_plan_costs(mdft, w, h):
     assert r <= 1.15, r
 
 
-# Columns with magnitudes in every tile the plan's rule picks on 256 CUs, the last tile short of a column or a pair:
+# Columns with magnitudes in every tile the plan's rule picks on 256 CUs (the image path runs those of less than 256
+# threads in 256), the last tile short of a column or a pair:
 # (width, height, tile threads, two lines per thread)
 IMAGE_COLUMNS = [(3067, 4096, 1024, True), (2049, 2048, 512, True), (1025, 2048, 256, True), (515, 4096, 256, True),
                  (3841, 1021, 512, True), (1923, 1201, 512, True), (1923, 2047, 512, True), (1283, 2047, 256, True),
                  (2561, 701, 256, True), (5121, 509, 256, True), (1027, 8192, 1024, False), (515, 2999, 512, False),
-                 (513, 6007, 1024, False), (61, 6007, 512, False), (192, 71, 256, False), (60, 139, 128, False)]
+                 (513, 6007, 1024, False), (61, 6007, 512, False), (192, 71, 64, False), (60, 139, 64, False)]
 
 
 # and of a smooth height (1921 x 1080: 512 threads)
@@ -144,3 +145,74 @@ def test_image_columns_in_every_tile(mdft, w, h):
     ref = torch.fft.fft2(lum).abs() / (w * h)
     err = torch.linalg.norm(dst[:, :w].cpu().to(torch.float64) - ref) / torch.linalg.norm(ref)
     assert err <= tol_nl2(w, h), float(err)
+
+
+# Plan columns in every wide tile: the tile a size takes is checked against the rule in test_tile_rule.py
+PLAN_COLUMNS = [(3067, 4096, 1024, True), (6131, 2048, 1024, True), (4099, 3072, 1024, True), (2049, 2048, 512, True),
+                (4099, 1024, 512, True), (1025, 2048, 256, True), (515, 4096, 256, True), (1027, 1536, 256, True),
+                (1923, 2047, 512, True), (3841, 1021, 512, True), (1923, 1201, 512, True), (1283, 2047, 256, True),
+                (2563, 1021, 256, True), (1283, 1201, 256, True), (2561, 701, 256, True), (5121, 509, 256, True),
+                (1027, 8192, 1024, False), (1029, 4093, 1024, False), (515, 2999, 512, False),
+                (517, 6144, 512, False), (513, 6007, 1024, False)]
+
+
+# A wide tile gives the bits of the narrow one (the tile table's entry 0), and FP64's values
+@pytest.mark.parametrize("w,h", [c[:2] for c in PLAN_COLUMNS])
+def test_plan_columns_in_every_wide_tile(mdft, w, h):
+    import torch
+
+    g = torch.Generator(device="cuda")
+    g.manual_seed(w * 3 + h)
+    src = torch.randn(w * h, dtype=torch.complex64, device="cuda", generator=g)
+    st = torch.cuda.current_stream().cuda_stream
+    direct = h & (h - 1) == 0 or (h % 3 == 0 and (h // 3) & (h // 3 - 1) == 0)
+    shapes = [s for s in list(range(1, 15)) + list(range(38, 44))]
+    keep = {s: mdft.tune_get(s, not direct, 1) for s in shapes}
+    p = mdft.Plan(w, h)
+    outs = []
+    print(f"plan columns {w}x{h}", flush=True)
+    try:
+        for variant in (0, 1):
+            for s in shapes:
+                mdft.tune_set(s, not direct, 1, variant)
+            for inv in (False, True):
+                dst = torch.full_like(src, float("nan"))
+                p.exec_device(inv, src.data_ptr(), dst.data_ptr(), st)
+                outs.append(dst)
+    finally:
+        for s in shapes:
+            mdft.tune_set(s, not direct, 1, keep[s])
+    torch.cuda.synchronize()
+    p.close()
+    for a, b in ((0, 2), (1, 3)):
+        assert torch.equal(torch.view_as_real(outs[a]), torch.view_as_real(outs[b]))
+    ref = torch.fft.fft2(src.cpu().reshape(h, w).to(torch.complex128))
+    err = torch.linalg.norm(outs[2].cpu().reshape(h, w) - ref) / torch.linalg.norm(ref)
+    assert err <= tol_nl2(w, h), float(err)
+
+
+@pytest.mark.parametrize("flags", [4, 6])
+def test_smooth_lengths_in_a_dependent_batch(mdft, flags):
+    import torch
+
+    sizes = [(100, 300), (640, 480), (45, 1920), (1, 90), (90, 1), (20, 18), (3000, 2), (37, 3600), (1021, 75)]
+    invs = [i % 2 == 0 for i in range(len(sizes))]
+    rng = np.random.default_rng(12)
+    xs = [rand_c64(rng, (h, w)) for w, h in sizes]
+    offs = np.cumsum([0] + [w * h for w, h in sizes])[:-1].tolist()
+    src = torch.from_numpy(np.concatenate([x.ravel() for x in xs])).cuda()
+    dst = torch.empty_like(src)
+    st = torch.cuda.current_stream().cuda_stream
+    print(f"smooth dependent batch flags={flags}", flush=True)
+    b = mdft.Batch(sizes, invs, offs, offs, flags)
+    b.exec_device(src.data_ptr(), dst.data_ptr(), st)
+    b.check()
+    torch.cuda.synchronize()
+    b.close()
+    for (w, h), inv, o in zip(sizes, invs, offs):
+        alone = torch.empty(w * h, dtype=torch.complex64, device="cuda")
+        p = mdft.Plan(w, h)
+        p.exec_device(inv, src.data_ptr() + 8 * o, alone.data_ptr(), st)
+        torch.cuda.synchronize()
+        p.close()
+        assert torch.equal(torch.view_as_real(dst[o:o + w * h]), torch.view_as_real(alone)), (w, h)

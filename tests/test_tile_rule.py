@@ -1,0 +1,51 @@
+"""The single-image tile rule on the CPU: the sizes of the GPU tests reach the
+tiles they are there for (a moved line fails here, where the GPU test would
+quietly compare a kernel with itself)."""
+import os
+import subprocess
+
+import pytest
+
+from tests import test_gpu_dispatch as G
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+GEN_SHAPE = 60  # smooth lengths: their own kernels
+
+
+@pytest.fixture(scope="module")
+def ask(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("tool") / "tile_tool")
+    lib = os.path.join(ROOT, "math_amd", "lib")
+    subprocess.run(["g++", "-std=c++17", "-O1", os.path.join(ROOT, "tests", "cpp", "tile_tool.cpp"), "-o", exe,
+                    "-L" + lib, "-lmdft", "-Wl,-rpath," + lib], check=True)
+
+    def run(query):
+        r = subprocess.run([exe], input=" ".join(str(int(q) if isinstance(q, bool) else q) for q in query) + "\n",
+                           capture_output=True, text=True, check=True)
+        return [int(v) for v in r.stdout.split()]
+
+    return run
+
+
+def column_tile(ask, w, h, variant):
+    shape = ask(("n", h, 1))[0]
+    direct = h & (h - 1) == 0 or (h % 3 == 0 and (h // 3) & (h // 3 - 1) == 0)
+    assert shape != GEN_SHAPE
+    threads, x2 = ask((shape, not direct, True, w, variant))
+    return shape, not direct, threads, bool(x2)
+
+
+@pytest.mark.parametrize("w,h,threads,x2", G.IMAGE_COLUMNS + G.PLAN_COLUMNS)
+def test_sizes_reach_their_tiles(ask, w, h, threads, x2):
+    assert column_tile(ask, w, h, 1)[2:] == (threads, x2)
+
+
+@pytest.mark.parametrize("w,h,threads,x2", G.PLAN_COLUMNS)
+def test_the_tables_narrow_entry_gives_another_tile(ask, w, h, threads, x2):
+    t, two = column_tile(ask, w, h, 0)[2:]
+    assert not two and t < threads or (x2 and not two)
+
+
+def test_image_cases_with_smooth_heights_are_named_apart(ask):
+    assert ask(("n", 1080, 1)) == [GEN_SHAPE]
+    assert ask(("n", 71, 1)) == [38] and ask(("n", 139, 1)) == [39]
