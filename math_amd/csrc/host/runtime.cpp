@@ -717,6 +717,10 @@ void Context::enqueue_axis(const LinePlan& lp, const float2* src, float2* dst, i
 //  * Bluestein X2 columns: 256 threads from 2.5 tiles per CU (1500 x 2047 40.9, 42
 //    with 512, 51.5 narrow; 4001 x 701 49.2, 52.1; 2049 x 701, two tiles per CU,
 //    31.6, 29.4 narrow);
+//  * 8192-point columns: 1024 threads (four lines, 32-byte runs where a narrow
+//    tile reads single elements) from half a tile per CU when direct (770 x 8192
+//    71.5, 112 narrow; 512 x 8192 41.6, 55.8; 256 x 8192 42.4, 38.6 narrow), from
+//    5/8 for Bluestein (700 x 4093 46.5, 50.3 narrow; 512 x 4093 45.6, 41.8 narrow);
 //  * other wide tiles from one per CU.
 AxisTile axis_tile(int shape, bool blue, bool cols, int count, int variant, int cu_count)
 {
@@ -734,8 +738,10 @@ AxisTile axis_tile(int shape, bool blue, bool cols, int count, int variant, int 
             if (per_cu8(1024) >= 12) return {1024, true};
             if (per_cu8(512) >= 8) return {512, true};
             if (per_cu8(256) >= 8) return {256, true};
-        } else if (per_cu8(wide_threads(shape, cols, blue)) >= 8) {
-            return {wide_threads(shape, cols, blue), false};
+        } else {
+            const int wide = wide_threads(shape, cols, blue);
+            const int need = cols && wide / tpl_of(shape) >= 4 ? (blue ? 5 : 4) : 8;
+            if (per_cu8(wide) >= need) return {wide, false};
         }
     }
     // passes with few lines: smaller tiles (one wave for lines of up to 1024

@@ -152,8 +152,8 @@ PLAN_COLUMNS = [(3067, 4096, 1024, True), (6131, 2048, 1024, True), (4099, 3072,
                 (4099, 1024, 512, True), (1025, 2048, 256, True), (515, 4096, 256, True), (1027, 1536, 256, True),
                 (1923, 2047, 512, True), (3841, 1021, 512, True), (1923, 1201, 512, True), (1283, 2047, 256, True),
                 (2563, 1021, 256, True), (1283, 1201, 256, True), (2561, 701, 256, True), (5121, 509, 256, True),
-                (1027, 8192, 1024, False), (1029, 4093, 1024, False), (515, 2999, 512, False),
-                (517, 6144, 512, False), (513, 6007, 1024, False)]
+                (1027, 8192, 1024, False), (1029, 4093, 1024, False), (770, 8192, 1024, False),
+                (770, 4093, 1024, False), (515, 2999, 512, False), (517, 6144, 512, False), (513, 6007, 1024, False)]
 
 
 # A wide tile gives the bits of the narrow one (the tile table's entry 0), and FP64's values

@@ -46,6 +46,12 @@ def test_the_tables_narrow_entry_gives_another_tile(ask, w, h, threads, x2):
     assert not two and t < threads or (x2 and not two)
 
 
+# 8192-point columns: wide tiles where they are fewer than the CUs but faster all the same, narrow ones below
+@pytest.mark.parametrize("w,h,threads", [(509, 8192, 1024), (508, 8192, 256), (637, 4093, 1024), (636, 4093, 256)])
+def test_8192_point_columns(ask, w, h, threads):
+    assert column_tile(ask, w, h, 1)[2:] == (threads, False)
+
+
 def test_image_cases_with_smooth_heights_are_named_apart(ask):
     assert ask(("n", 1080, 1)) == [GEN_SHAPE]
     assert ask(("n", 71, 1)) == [38] and ask(("n", 139, 1)) == [39]
