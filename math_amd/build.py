@@ -28,8 +28,11 @@ COMMON = [
 # a source, or (source, object name, defines) for one compiled several times;
 # the longest compilations first
 SOURCES = [
-    ("kernels/batch_kernels.hip", f"batch_{kind}_{t}", [f"-DMDFT_BATCH_T={t}", f"-DMDFT_BATCH_PERSISTENT_TU={p}"])
-    for p, kind, t in ((0, "grid", 256), (1, "persistent", 256), (0, "grid", 512), (0, "grid", 1024))
+    ("kernels/batch_kernels.hip", f"batch_{kind}_{t}{'_' + hold if hold != 'BATCH_ALL' else ''}",
+     [f"-DMDFT_BATCH_T={t}", f"-DMDFT_BATCH_HOLD={hold}", f"-DMDFT_BATCH_PERSISTENT_TU={p}"])
+    for p, kind, t, hold in ((0, "grid", 256, "BATCH_ALL"), (1, "persistent", 256, "BATCH_ALL"),
+                             (0, "grid", 512, "BATCH_COLS_X2"), (0, "grid", 1024, "BATCH_COLS_X2"),
+                             (0, "grid", 512, "BATCH_COLS"))
 ] + [
     "kernels/whole.hip",
     "kernels/axis.hip",

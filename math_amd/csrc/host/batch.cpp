@@ -75,10 +75,10 @@ void enqueue_batch(mdft_batch_s* b, hipStream_t stream)
                                                       b->spin_limit, stream),
                         "batch launch (phase 2)");
     } else {
-        mdft::hip_check(mdft::launch_batch_grid(T, b->jobs_dev, b->items_dev, b->nphase1, stream),
+        mdft::hip_check(mdft::launch_batch_grid(T, mdft::BATCH_ALL, b->jobs_dev, b->items_dev, b->nphase1, stream),
                         "batch launch (phase 1)");
-        mdft::hip_check(mdft::launch_batch_grid(b->threads_cols, b->jobs_dev, b->items_dev + b->nphase1,
-                                                b->nitems - b->nphase1, stream),
+        mdft::hip_check(mdft::launch_batch_grid(b->threads_cols, b->build.hold_cols, b->jobs_dev,
+                                                b->items_dev + b->nphase1, b->nitems - b->nphase1, stream),
                         "batch launch (phase 2)");
     }
 }
@@ -103,9 +103,10 @@ float time_column_phase(Context& ctx, const std::vector<mdft::BatchEntry>& entri
         err = hipMemcpy(items, bb.items.data() + bb.nphase1, sizeof(uint2) * n2, hipMemcpyHostToDevice);
     if (err == hipSuccess) err = hipEventCreate(&a);
     if (err == hipSuccess) err = hipEventCreate(&e);
-    if (err == hipSuccess) err = mdft::launch_batch_grid(TC, jobs, items, n2, s);
+    auto launch = [&]() { return mdft::launch_batch_grid(bb.threads_cols, bb.hold_cols, jobs, items, n2, s); };
+    if (err == hipSuccess) err = launch();
     if (err == hipSuccess) err = hipEventRecord(a, s);
-    for (int r = 0; r < 3 && err == hipSuccess; ++r) err = mdft::launch_batch_grid(TC, jobs, items, n2, s);
+    for (int r = 0; r < 3 && err == hipSuccess; ++r) err = launch();
     if (err == hipSuccess) err = hipEventRecord(e, s);
     if (err == hipSuccess) err = hipEventSynchronize(e);
     if (err == hipSuccess) err = hipEventElapsedTime(&ms, a, e);
@@ -191,6 +192,7 @@ int mdft_batch_create(mdft_batch* batch, const mdft_desc* descs, uint32_t count,
     }
     mdft::build_batch(ctx, entries.data(), count, T, b->threads_cols, (flags & MDFT_BATCH_DEPENDENT) != 0, b->build,
                       &b->job_image, &b->job_is_col);
+    b->threads_cols = b->build.threads_cols;
     b->nphase1 = b->build.nphase1;
     b->nitems = (uint32_t)b->build.items.size();
     b->nctl = mdft::BATCH_CTL_HEADER + b->build.ncounters;
@@ -295,13 +297,14 @@ int mdft_batch_exec_phase(mdft_batch b, int phase, const void* src, void* dst, v
     hipStream_t stream = static_cast<hipStream_t>(stream_p);
     if (phase == 1) {
         prepare_exec(b, src, dst, stream);
-        mdft::hip_check(mdft::launch_batch_grid(b->threads, b->jobs_dev, b->items_dev, b->nphase1, stream),
+        mdft::hip_check(mdft::launch_batch_grid(b->threads, mdft::BATCH_ALL, b->jobs_dev, b->items_dev, b->nphase1,
+                                                stream),
                         "batch launch (phase 1)");
     } else {
         if (src != b->cur_src || dst != b->cur_dst)
             throw Error(MDFT_ERR_STATE, "mdft_batch_exec_phase: phase 2 needs the pointers of the phase 1 call");
-        mdft::hip_check(mdft::launch_batch_grid(b->threads_cols, b->jobs_dev, b->items_dev + b->nphase1,
-                                                b->nitems - b->nphase1, stream),
+        mdft::hip_check(mdft::launch_batch_grid(b->threads_cols, b->build.hold_cols, b->jobs_dev,
+                                                b->items_dev + b->nphase1, b->nitems - b->nphase1, stream),
                         "batch launch (phase 2)");
     }
     b->last_stream = stream;

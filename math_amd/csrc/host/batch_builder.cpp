@@ -45,9 +45,57 @@ int batch_threads_for(const uint32_t* widths, const uint32_t* heights, size_t co
 }
 
 // lines a tile of T threads holds of a plan's length
-static int lines_per_tile(int T, const LinePlan& lp, bool cols)
+static int lines_per_tile(int T, BatchHold hold, const LinePlan& lp)
 {
-    return lp.gen ? T / lp.smooth.tpl : batch_lines_per_tile(T, lp.shape, cols);
+    return lp.gen ? T / lp.smooth.tpl : batch_lines_per_tile(T, hold, lp.shape);
+}
+
+// whole images run both passes in one row-phase workgroup
+static bool runs_whole(int w, int h, int T, const LinePlan& row, const LinePlan& col)
+{
+    return w > 1 && h > 1 && h <= lines_per_tile(T, BATCH_ALL, row) && w <= lines_per_tile(T, BATCH_ALL, col);
+}
+
+// cost of one line ~ points x passes
+static double line_cost(const LinePlan& lp) { return double(lp.m) * (std::log2(double(lp.m)) + 2); }
+
+// The kernel of the column phase: its tiles in the smallest form that still
+// fills the device, since a tile's chain of loads, passes and exchanges takes as
+// long as it has lines (us of the phase, 256 CUs):
+//  * 256 threads while those tiles cost no more than one of the dearest per CU
+//    (direct ones counted twice: they wait for memory, where the shorter runs
+//    cost): 128 x 509 7.8 (10.0 in 512 threads with one line per thread, 14.4 with
+//    two), 57 x 4093 20.3 (24.8, 25.4), 256 x 2238 15.6 (17.4, 18.2), but 256 x
+//    4096 13.4 (10.8, 12.0);
+//  * 512 threads and one line per thread below 1.5 tiles per CU of the two-line
+//    form: 1024 x 1201 18.1 (18.3 with two), 2560 x 1021 22.3 (26.4); with two
+//    above: 2048 x 1201 27.1 (30.5 with one), 2048 x 2047 30.6 (34.4); direct lines
+//    gain more, tiles of 1536 and 3072 points count twice and of 4096 three times:
+//    2048 x 1536 13.0 (14.5 with one), 1024 x 3072 16.5 (21.5), 512 x 4096 15.0 (15.6);
+//  * one line per thread as well where no line has the two-line form (2048 x 4093
+//    65.6, 70.4 in the kernel with two).
+static BatchHold column_kernel(int T, int TC, int cu_count, const BatchEntry* entries, size_t count,
+                               const std::vector<std::shared_ptr<const LinePlan>>& plans)
+{
+    if (TC <= T) return BATCH_ALL;
+    if (TC != BATCH_COL_THREADS) return BATCH_COLS_X2;
+    double narrow = 0, dearest = 0;
+    int64_t two = 0;
+    bool any_two = false;
+    for (size_t i = 0; i < count; ++i) {
+        const int w = (int)entries[i].width, h = (int)entries[i].height;
+        const LinePlan &row = *plans[2 * i], &col = *plans[2 * i + 1];
+        if (w <= 1 || h <= 1 || runs_whole(w, h, T, row, col)) continue;
+        const int n1 = lines_per_tile(T, BATCH_ALL, col), n2 = lines_per_tile(TC, BATCH_COLS_X2, col);
+        const double cost = n1 * line_cost(col);
+        narrow += (w + n1 - 1) / n1 * cost * (col.blue ? 1 : 2);
+        dearest = std::max(dearest, cost);
+        const bool x2 = has_x2(col.shape);
+        two += int64_t((w + n2 - 1) / n2) * (!x2 || col.blue ? 1 : col.m == 4096 ? 3 : is_f3(col.shape) ? 2 : 1);
+        any_two |= x2;
+    }
+    if (narrow <= dearest * cu_count) return BATCH_ALL;
+    return any_two && 2 * two >= 3 * int64_t(cu_count) ? BATCH_COLS_X2 : BATCH_COLS;
 }
 
 void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int T, int TC, bool dependent,
@@ -75,22 +123,26 @@ void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int T, i
         uint2 v;
     };
     std::vector<Item> items;
+    std::vector<std::shared_ptr<const LinePlan>> plans(2 * count);  // rows, columns of every entry
+    for (size_t i = 0; i < count; ++i) {
+        plans[2 * i] = ctx.line_plan((int)entries[i].width, false);
+        plans[2 * i + 1] = ctx.line_plan((int)entries[i].height, true);
+    }
+    out.hold_cols = column_kernel(T, TC, ctx.cu_count(), entries, count, plans);
+    if (out.hold_cols == BATCH_ALL) TC = out.threads_cols = T;
     std::vector<std::pair<std::vector<uint2>, std::vector<uint2>>> per_image;  // dependency ordering
     uint32_t counter = 0, seq = 0;
     for (uint32_t idx : order) {
         const BatchEntry& e = entries[idx];
         const int w = (int)e.width, h = (int)e.height;
-        auto rp = ctx.line_plan(w, false);
-        auto cp = ctx.line_plan(h, true);
-        out.keep.push_back(rp);
-        out.keep.push_back(cp);
-        const int lpw_r = w > 1 ? lines_per_tile(T, *rp, false) : 0;
-        // a whole image runs both passes in one row-phase workgroup
-        const int lpw_cw = h > 1 ? lines_per_tile(T, *cp, true) : 0;
-        const bool whole = (w > 1 && h > 1 && h <= lpw_r && w <= lpw_cw);
+        const LinePlan *rp = plans[2 * idx].get(), *cp = plans[2 * idx + 1].get();
+        const int lpw_r = w > 1 ? lines_per_tile(T, BATCH_ALL, *rp) : 0;
+        const bool whole = runs_whole(w, h, T, *rp, *cp);
         // column tiles of images with a row pass run in the column phase (TC
         // threads); a single-column-pass image (w == 1) runs with the rows
-        const int lpw_c = h > 1 ? lines_per_tile((w > 1 && !whole) ? TC : T, *cp, true) : 0;
+        const int lpw_c = h <= 1             ? 0
+                          : w > 1 && !whole ? lines_per_tile(TC, out.hold_cols, *cp)
+                                            : lines_per_tile(T, BATCH_ALL, *cp);
         const int ntr = w > 1 ? (h + lpw_r - 1) / lpw_r : 0;
         const int ntc = h > 1 ? (w + lpw_c - 1) / lpw_c : 0;
         const int sig = (dependent && w > 1 && h > 1 && !whole) ? (int)counter++ : -1;
@@ -141,6 +193,7 @@ void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int T, i
         }
         per_image.push_back({ri, ci});
     }
+    out.keep = std::move(plans);
 
     if (dependent) {
         // rows of image k+1 before columns of image k: a column tile only

@@ -13,6 +13,7 @@ namespace mdft {
 struct BatchBuild {
     int threads = 256;       // workgroup size of whole images and row tiles
     int threads_cols = 256;  // workgroup size of column tiles
+    BatchHold hold_cols = BATCH_ALL;  // and the kernel that runs them
     std::vector<BatchJob> jobs;
     std::vector<uint2> items;
     uint32_t nphase1 = 0;

@@ -240,9 +240,10 @@ void launch_micro_batch(mdft_server_s* s, Lane& L, const std::vector<mdft::Batch
         if (e.width == 1 && e.height == 1)
             mdft::hip_check(hipMemcpyAsync(e.dst, e.src, sizeof(float2), hipMemcpyDeviceToDevice, L.stream), "copy");
     const uint32_t n = (uint32_t)bb.items.size();
-    mdft::hip_check(mdft::launch_batch_grid(T, jobs_dev, items_dev, bb.nphase1, L.stream), "serve launch");
-    mdft::hip_check(mdft::launch_batch_grid(bb.threads_cols, jobs_dev, items_dev + bb.nphase1, n - bb.nphase1,
-                                            L.stream),
+    mdft::hip_check(mdft::launch_batch_grid(T, mdft::BATCH_ALL, jobs_dev, items_dev, bb.nphase1, L.stream),
+                    "serve launch");
+    mdft::hip_check(mdft::launch_batch_grid(bb.threads_cols, bb.hold_cols, jobs_dev, items_dev + bb.nphase1,
+                                            n - bb.nphase1, L.stream),
                     "serve launch");
     mdft::hip_check(hipEventRecord(L.done, L.stream), "event record");
 }

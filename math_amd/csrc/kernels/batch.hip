@@ -16,22 +16,25 @@ __global__ void k_fill_u32(uint32_t* p, uint32_t n, uint32_t value)
     if (i < n) p[i] = value;
 }
 
-hipError_t launch_batch_grid(int threads, const BatchJob* jobs, const uint2* items, uint32_t nitems,
+hipError_t launch_batch_grid(int threads, BatchHold hold, const BatchJob* jobs, const uint2* items, uint32_t nitems,
                              hipStream_t stream)
 {
     if (nitems == 0) return hipSuccess;
-    if (threads == 256) return launch_batch_grid_t<256>(jobs, items, nitems, stream);
-    if (threads == 512) return launch_batch_grid_t<512>(jobs, items, nitems, stream);
-    return launch_batch_grid_t<1024>(jobs, items, nitems, stream);
+    if (!batch_holds(threads, hold)) return hipErrorInvalidValue;
+    if (hold == BATCH_ALL) return launch_batch_grid_t<256, BATCH_ALL>(jobs, items, nitems, stream);
+    if (hold == BATCH_COLS) return launch_batch_grid_t<512, BATCH_COLS>(jobs, items, nitems, stream);
+    if (threads == 512) return launch_batch_grid_t<512, BATCH_COLS_X2>(jobs, items, nitems, stream);
+    return launch_batch_grid_t<1024, BATCH_COLS_X2>(jobs, items, nitems, stream);
 }
 
 hipError_t warm_batch(uint32_t* word, hipStream_t stream)
 {
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, stream, word, 1u, 0u);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = warm_batch_grid<256>(word, stream);
-    if (e == hipSuccess) e = warm_batch_grid<512>(word, stream);
-    if (e == hipSuccess) e = warm_batch_grid<1024>(word, stream);
+    if (e == hipSuccess) e = warm_batch_grid<256, BATCH_ALL>(word, stream);
+    if (e == hipSuccess) e = warm_batch_grid<512, BATCH_COLS>(word, stream);
+    if (e == hipSuccess) e = warm_batch_grid<512, BATCH_COLS_X2>(word, stream);
+    if (e == hipSuccess) e = warm_batch_grid<1024, BATCH_COLS_X2>(word, stream);
     if (e == hipSuccess) e = warm_batch_persistent<256>(word, stream);
     return e;
 }
@@ -45,13 +48,13 @@ hipError_t launch_batch_persistent(const BatchJob* jobs, const uint2* items, uin
     return launch_batch_persistent_t<256>(jobs, items, nitems, ctl, grid, spin_limit, stream);
 }
 
-int batch_lines_per_tile(int threads, int shape, bool cols)
+int batch_lines_per_tile(int threads, BatchHold hold, int shape)
 {
     if (shape < 1 || (!is_f3(shape) && shape > BATCH_MAXLOGM) ||
         (is_f3(shape) && (f3_k(shape) < F3_MIN_K || f3_k(shape) > F3_MAX_K)))
         return 0;
     const int tpl = tpl_of(shape);
-    return tpl <= threads ? threads / tpl * lines_per_thread(batch_shape(shape, threads, cols)) : 0;
+    return tpl <= threads ? threads / tpl * lines_per_thread(batch_shape(shape, hold)) : 0;
 }
 
 hipError_t batch_occupancy(int* blocks_per_cu) { return batch_occupancy_t<256>(blocks_per_cu); }

@@ -1,8 +1,8 @@
-// The batch kernels of one workgroup size: compiled once per size (MDFT_BATCH_T
-// = 256, 512, 1024) and for 256 also as the persistent shapes
-// (MDFT_BATCH_PERSISTENT_TU = 1), since each holds many tile variants.  Row
-// tiles and whole images take 256 threads (a line of every batched length fits
-// those), so the larger sizes hold column tiles only.
+// The batch kernels of one workgroup size and content: compiled once each
+// (MDFT_BATCH_T = 256, 512, 1024, MDFT_BATCH_HOLD = a BatchHold) and for 256 also
+// as the persistent shapes (MDFT_BATCH_PERSISTENT_TU = 1), since each holds many
+// tile variants.  Row tiles and whole images take 256 threads (a line of every
+// batched length fits those), so the larger sizes hold column tiles only.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -14,33 +14,37 @@ namespace mdft {
 
 // Four waves per SIMD (<= 128 VGPRs): 256-thread tiles (4 workgroups per
 // CU), 512-thread tiles (two) or 1024-thread tiles (one).
-template <int T>
+template <int T, BatchHold H>
 __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(TILE_WAVES))) void k_batch_grid(
     const BatchJob* __restrict__ jobs, const uint2* __restrict__ items)
 {
-    __shared__ float lds[batch_lds<T, (T > 256)>()];
+    __shared__ float lds[batch_lds<T, H>()];
     // the host lays items out per XCD (block b runs on XCD b % 8)
-    run_item<T, true, (T > 256)>(jobs, items[blockIdx.x], lds);
+    run_item<T, true, H>(jobs, items[blockIdx.x], lds);
 }
 
+static_assert(batch_holds(MDFT_BATCH_T, BatchHold(MDFT_BATCH_HOLD)), "a size and content launch_batch_grid knows");
+
 template <>
-hipError_t launch_batch_grid_t<MDFT_BATCH_T>(const BatchJob* jobs, const uint2* items, uint32_t nitems,
-                                             hipStream_t stream)
+hipError_t launch_batch_grid_t<MDFT_BATCH_T, BatchHold(MDFT_BATCH_HOLD)>(const BatchJob* jobs, const uint2* items,
+                                                                         uint32_t nitems, hipStream_t stream)
 {
-    hipLaunchKernelGGL(k_batch_grid<MDFT_BATCH_T>, dim3(nitems), dim3(MDFT_BATCH_T), 0, stream, jobs, items);
+    hipLaunchKernelGGL((k_batch_grid<MDFT_BATCH_T, BatchHold(MDFT_BATCH_HOLD)>), dim3(nitems), dim3(MDFT_BATCH_T), 0,
+                       stream, jobs, items);
     return hipGetLastError();
 }
 
-template <int T>
+template <int T, BatchHold H>
 __global__ void k_warm_batch_grid(uint32_t* word)
 {
     if (threadIdx.x == 0) word[0] = 0u;
 }
 
 template <>
-hipError_t warm_batch_grid<MDFT_BATCH_T>(uint32_t* word, hipStream_t stream)
+hipError_t warm_batch_grid<MDFT_BATCH_T, BatchHold(MDFT_BATCH_HOLD)>(uint32_t* word, hipStream_t stream)
 {
-    hipLaunchKernelGGL(k_warm_batch_grid<MDFT_BATCH_T>, dim3(1), dim3(64), 0, stream, word);
+    hipLaunchKernelGGL((k_warm_batch_grid<MDFT_BATCH_T, BatchHold(MDFT_BATCH_HOLD)>), dim3(1), dim3(64), 0, stream,
+                       word);
     return hipGetLastError();
 }
 
@@ -59,7 +63,7 @@ __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(TILE_WAVES)))
     const BatchJob* __restrict__ jobs, const uint2* __restrict__ items, uint32_t nitems, uint32_t* ctl,
     uint32_t spin_limit)
 {
-    __shared__ float lds[batch_lds<T, false>()];
+    __shared__ float lds[batch_lds<T, BATCH_ALL>()];
     __shared__ uint32_t s_item;
     uint32_t* ticket = ctl;
     uint32_t* err = ctl + 1;
@@ -92,7 +96,7 @@ __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(TILE_WAVES)))
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         }
-        run_item<T, false, false>(jobs, item, lds);
+        run_item<T, false, BATCH_ALL>(jobs, item, lds);
         if (bj.sig >= 0) {
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // release this wave's stores
             __syncthreads();

@@ -34,30 +34,29 @@
 namespace mdft {
 
 // The form of a shape a batch runs: two lines per thread where the shape has
-// that in the column tiles of phase 2 (kernels of more than 256 threads, which
-// hold columns only); one along rows, where two measured no better (4096^2:
-// 140 us against 152), and for the columns of phase 1 (small whole images and
-// single columns).
-__host__ __device__ constexpr int batch_shape(int s, int threads, bool cols)
+// that in the kernels of two-line columns; one along rows, where two measured no
+// better (4096^2: 140 us against 152), and for the columns of phase 1 (small
+// whole images and single columns).
+__host__ __device__ constexpr int batch_shape(int s, BatchHold hold)
 {
-    return has_x2(s) && cols && threads > 256 ? s | X2 : s;
+    return has_x2(s) && hold == BATCH_COLS_X2 ? s | X2 : s;
 }
 
-template <int S, int T, bool COLS_ONLY>
+template <int S, int T, BatchHold H>
 constexpr int lds_need()
 {
     if constexpr (tpl_of(S) > T) {
         return 0;
     } else {
-        constexpr int a = COLS_ONLY ? 0 : LineCfg<batch_shape(S, T, false), T>::template lds_floats<false>();
-        constexpr int b = LineCfg<batch_shape(S, T, true), T>::template lds_floats<true>();
+        constexpr int a = H != BATCH_ALL ? 0 : LineCfg<batch_shape(S, H), T>::template lds_floats<false>();
+        constexpr int b = LineCfg<batch_shape(S, H), T>::template lds_floats<true>();
         return a > b ? a : b;
     }
 }
 
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 
-template <int T, bool C>
+template <int T, BatchHold C>
 constexpr int batch_lds()
 {
     return cmax(gen_lds_floats(T),
@@ -81,16 +80,16 @@ __device__ __forceinline__ void run_variant(const AxisJob& job, int tile, float*
     line_tile<S, T, BLUE, COLS>(job, tile, lds, tid);
 }
 
-template <int S, int T, bool COLS>
+template <int S, int T, BatchHold H, bool COLS>
 __device__ __forceinline__ void run_axis(const AxisJob& job, int blue, int tile, float* lds)
 {
     if constexpr (S >= 2) {
         if (blue) {
-            run_variant<batch_shape(S, T, COLS), T, true, COLS>(job, tile, lds);
+            run_variant<batch_shape(S, H), T, true, COLS>(job, tile, lds);
             return;
         }
     }
-    run_variant<batch_shape(S, T, COLS), T, false, COLS>(job, tile, lds);
+    run_variant<batch_shape(S, H), T, false, COLS>(job, tile, lds);
 }
 
 // a smooth length (its own asm for the indices, like run_variant)
@@ -102,23 +101,23 @@ __device__ __forceinline__ void run_smooth(const AxisJob& job, int tile, float* 
     smooth_tile<T, COLS>(job, tile, lds, tid);
 }
 
-template <int S, int T, bool COLS_ONLY>
+template <int S, int T, BatchHold H>
 __device__ __forceinline__ void run_tile_body(const AxisJob& job, int blue, int cols, int tile, float* lds)
 {
     if constexpr (S == GEN_SHAPE) {
-        if constexpr (COLS_ONLY)
+        if constexpr (H != BATCH_ALL)
             run_smooth<T, true>(job, tile, lds);
         else if (cols)
             run_smooth<T, true>(job, tile, lds);
         else
             run_smooth<T, false>(job, tile, lds);
     } else if constexpr (tpl_of(S) <= T) {
-        if constexpr (COLS_ONLY)
-            run_axis<S, T, true>(job, blue, tile, lds);
+        if constexpr (H != BATCH_ALL)
+            run_axis<S, T, H, true>(job, blue, tile, lds);
         else if (cols)
-            run_axis<S, T, true>(job, blue, tile, lds);
+            run_axis<S, T, H, true>(job, blue, tile, lds);
         else
-            run_axis<S, T, false>(job, blue, tile, lds);
+            run_axis<S, T, H, false>(job, blue, tile, lds);
     }
 }
 
@@ -128,11 +127,11 @@ __device__ __noinline__ void run_tile_call(const BatchJob* jobs, uint32_t job, i
 // Grid kernels inline every variant (register allocation per region,
 // occupancy-constrained); the persistent kernels call them out of line, since
 // inlining into the ticket loop keeps too much alive across it.
-template <int S, int T, bool INL, bool COLS_ONLY>
+template <int S, int T, bool INL, BatchHold H>
 __device__ __forceinline__ void run_tile(const BatchJob* jobs, uint32_t job, const BatchJob& bj, int tile, float* lds)
 {
     if constexpr (INL)
-        run_tile_body<S, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds);
+        run_tile_body<S, T, H>(bj.job, bj.blue, bj.cols, tile, lds);
     else
         run_tile_call<S, T>(jobs, job, tile, lds);
 }
@@ -156,69 +155,69 @@ __device__ __noinline__ void run_tile_call(const BatchJob* jobs, uint32_t job, i
 #pragma unroll
     for (size_t i = 0; i < sizeof(BatchJob) / 4; ++i) copy.w[i] = words[i];
     const BatchJob& bj = copy.job;
-    run_tile_body<S, T, false>(bj.job, bj.blue, bj.cols, __builtin_amdgcn_readfirstlane(tile), lds);
+    run_tile_body<S, T, BATCH_ALL>(bj.job, bj.blue, bj.cols, __builtin_amdgcn_readfirstlane(tile), lds);
 }
 
-template <int T, bool INL, bool COLS_ONLY>
+template <int T, bool INL, BatchHold H>
 __device__ __forceinline__ void run_job_tile(const BatchJob* jobs, uint32_t job, int tile, float* lds)
 {
     const BatchJob bj = jobs[job];
     switch (bj.shape) {
-    case 1: run_tile<1, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
-    case 2: run_tile<2, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
-    case 3: run_tile<3, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
-    case 4: run_tile<4, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
-    case 5: run_tile<5, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
-    case 6: run_tile<6, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
-    case 7: run_tile<7, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
-    case 8: run_tile<8, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
-    case 9: run_tile<9, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
-    case 10: run_tile<10, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
-    case 11: run_tile<11, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
-    case 12: run_tile<12, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
-    case 13: run_tile<13, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
-    case F3_BASE + 6: run_tile<F3_BASE + 6, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
-    case F3_BASE + 7: run_tile<F3_BASE + 7, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
-    case F3_BASE + 8: run_tile<F3_BASE + 8, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
-    case F3_BASE + 9: run_tile<F3_BASE + 9, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
-    case F3_BASE + 10: run_tile<F3_BASE + 10, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
-    case F3_BASE + 11: run_tile<F3_BASE + 11, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
-    case GEN_SHAPE: run_tile<GEN_SHAPE, T, INL, COLS_ONLY>(jobs, job, bj, tile, lds); break;
+    case 1: run_tile<1, T, INL, H>(jobs, job, bj, tile, lds); break;
+    case 2: run_tile<2, T, INL, H>(jobs, job, bj, tile, lds); break;
+    case 3: run_tile<3, T, INL, H>(jobs, job, bj, tile, lds); break;
+    case 4: run_tile<4, T, INL, H>(jobs, job, bj, tile, lds); break;
+    case 5: run_tile<5, T, INL, H>(jobs, job, bj, tile, lds); break;
+    case 6: run_tile<6, T, INL, H>(jobs, job, bj, tile, lds); break;
+    case 7: run_tile<7, T, INL, H>(jobs, job, bj, tile, lds); break;
+    case 8: run_tile<8, T, INL, H>(jobs, job, bj, tile, lds); break;
+    case 9: run_tile<9, T, INL, H>(jobs, job, bj, tile, lds); break;
+    case 10: run_tile<10, T, INL, H>(jobs, job, bj, tile, lds); break;
+    case 11: run_tile<11, T, INL, H>(jobs, job, bj, tile, lds); break;
+    case 12: run_tile<12, T, INL, H>(jobs, job, bj, tile, lds); break;
+    case 13: run_tile<13, T, INL, H>(jobs, job, bj, tile, lds); break;
+    case F3_BASE + 6: run_tile<F3_BASE + 6, T, INL, H>(jobs, job, bj, tile, lds); break;
+    case F3_BASE + 7: run_tile<F3_BASE + 7, T, INL, H>(jobs, job, bj, tile, lds); break;
+    case F3_BASE + 8: run_tile<F3_BASE + 8, T, INL, H>(jobs, job, bj, tile, lds); break;
+    case F3_BASE + 9: run_tile<F3_BASE + 9, T, INL, H>(jobs, job, bj, tile, lds); break;
+    case F3_BASE + 10: run_tile<F3_BASE + 10, T, INL, H>(jobs, job, bj, tile, lds); break;
+    case F3_BASE + 11: run_tile<F3_BASE + 11, T, INL, H>(jobs, job, bj, tile, lds); break;
+    case GEN_SHAPE: run_tile<GEN_SHAPE, T, INL, H>(jobs, job, bj, tile, lds); break;
     default: break;
     }
 }
 
 // the same for a job given by value (inlined)
-template <int T, bool COLS_ONLY>
+template <int T, BatchHold H>
 __device__ __forceinline__ void run_job(const BatchJob& bj, int tile, float* lds)
 {
     switch (bj.shape) {
-    case 1: run_tile_body<1, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 2: run_tile_body<2, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 3: run_tile_body<3, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 4: run_tile_body<4, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 5: run_tile_body<5, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 6: run_tile_body<6, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 7: run_tile_body<7, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 8: run_tile_body<8, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 9: run_tile_body<9, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 10: run_tile_body<10, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 11: run_tile_body<11, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 12: run_tile_body<12, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 13: run_tile_body<13, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case F3_BASE + 6: run_tile_body<F3_BASE + 6, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case F3_BASE + 7: run_tile_body<F3_BASE + 7, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case F3_BASE + 8: run_tile_body<F3_BASE + 8, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case F3_BASE + 9: run_tile_body<F3_BASE + 9, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case F3_BASE + 10: run_tile_body<F3_BASE + 10, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case F3_BASE + 11: run_tile_body<F3_BASE + 11, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case GEN_SHAPE: run_tile_body<GEN_SHAPE, T, COLS_ONLY>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 1: run_tile_body<1, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 2: run_tile_body<2, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 3: run_tile_body<3, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 4: run_tile_body<4, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 5: run_tile_body<5, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 6: run_tile_body<6, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 7: run_tile_body<7, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 8: run_tile_body<8, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 9: run_tile_body<9, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 10: run_tile_body<10, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 11: run_tile_body<11, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 12: run_tile_body<12, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case 13: run_tile_body<13, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case F3_BASE + 6: run_tile_body<F3_BASE + 6, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case F3_BASE + 7: run_tile_body<F3_BASE + 7, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case F3_BASE + 8: run_tile_body<F3_BASE + 8, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case F3_BASE + 9: run_tile_body<F3_BASE + 9, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case F3_BASE + 10: run_tile_body<F3_BASE + 10, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case F3_BASE + 11: run_tile_body<F3_BASE + 11, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+    case GEN_SHAPE: run_tile_body<GEN_SHAPE, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
     default: break;
     }
 }
 
 // One item; every branch is on a wave-uniform value.
-template <int T, bool INL, bool COLS_ONLY>
+template <int T, bool INL, BatchHold H>
 __device__ __forceinline__ void run_item(const BatchJob* __restrict__ jobs, uint2 item, float* lds)
 {
     const uint32_t x = __builtin_amdgcn_readfirstlane(item.x);
@@ -228,7 +227,7 @@ __device__ __forceinline__ void run_item(const BatchJob* __restrict__ jobs, uint
     uint32_t job = x;
     int tile = whole ? 0 : (int)y;
     for (int turn = 0;; ++turn) {
-        run_job_tile<T, INL, COLS_ONLY>(jobs, job, tile, lds);
+        run_job_tile<T, INL, H>(jobs, job, tile, lds);
         if (!whole || turn == 1) break;
         // the column tile reads what this workgroup's waves just stored
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");

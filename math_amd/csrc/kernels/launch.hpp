@@ -136,21 +136,28 @@ hipError_t launch_image_magnitude(const ImageIO& io, const float2* src, int w, i
 // lengths 1024-4096 (wider contiguous runs per row), two workgroups per CU.
 constexpr int BATCH_COL_THREADS = 512;
 
-// batch kernels, padded lengths up to 8192: threads is 256 (any items), or 512 or 1024 (column tiles only);
-// the persistent shapes run in 256 threads
-hipError_t launch_batch_grid(int threads, const BatchJob* jobs, const uint2* items, uint32_t nitems,
+// What the kernels of a workgroup size hold: any items, one line per thread
+// (256 threads); or column tiles alone, two lines per thread where the shape has
+// that (512 and 1024 threads) or one (512).
+enum BatchHold { BATCH_ALL = 0, BATCH_COLS_X2 = 1, BATCH_COLS = 2 };
+__host__ __device__ constexpr bool batch_holds(int threads, BatchHold hold)
+{
+    return hold == BATCH_ALL ? threads == 256 : threads == 512 || (threads == 1024 && hold == BATCH_COLS_X2);
+}
+// batch kernels, padded lengths up to 8192 (an error where !batch_holds); the persistent shapes run in 256 threads
+hipError_t launch_batch_grid(int threads, BatchHold hold, const BatchJob* jobs, const uint2* items, uint32_t nitems,
                              hipStream_t stream);
 hipError_t launch_batch_persistent(const BatchJob* jobs, const uint2* items, uint32_t nitems, uint32_t* ctl,
                                    uint32_t nctl, int grid, uint32_t spin_limit, hipStream_t stream);
 // their kernels of one workgroup size (batch_kernels.hip, compiled per size and launch shape)
-template <int T>
+template <int T, BatchHold H>
 hipError_t launch_batch_grid_t(const BatchJob* jobs, const uint2* items, uint32_t nitems, hipStream_t stream);
 template <int T>
 hipError_t launch_batch_persistent_t(const BatchJob* jobs, const uint2* items, uint32_t nitems, uint32_t* ctl,
                                      int grid, uint32_t spin_limit, hipStream_t stream);
 template <int T>
 hipError_t batch_occupancy_t(int* blocks_per_cu);
-template <int T>
+template <int T, BatchHold H>
 hipError_t warm_batch_grid(uint32_t* word, hipStream_t stream);
 template <int T>
 hipError_t warm_batch_persistent(uint32_t* word, hipStream_t stream);
@@ -158,8 +165,8 @@ hipError_t warm_batch_persistent(uint32_t* word, hipStream_t stream);
 constexpr int WHOLE_THREADS = 256;
 hipError_t launch_whole(const BatchJob& row, const BatchJob& col, hipStream_t stream);
 hipError_t warm_whole(uint32_t* word, hipStream_t stream);
-// lines of a shape one tile holds: rows in 256 threads, columns in 256, 512 or 1024 (0: the shape does not fit)
-int batch_lines_per_tile(int threads, int shape, bool cols);
+// lines of a shape one tile holds (0: the shape does not fit)
+int batch_lines_per_tile(int threads, BatchHold hold, int shape);
 hipError_t batch_occupancy(int* blocks_per_cu);
 int batch_max_logm();
 

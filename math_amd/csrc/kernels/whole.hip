@@ -15,11 +15,11 @@ namespace mdft {
 __global__ __launch_bounds__(WHOLE_THREADS) __attribute__((amdgpu_waves_per_eu(TILE_WAVES))) void k_whole(BatchJob row,
                                                                                                           BatchJob col)
 {
-    __shared__ float lds[batch_lds<WHOLE_THREADS, false>()];
+    __shared__ float lds[batch_lds<WHOLE_THREADS, BATCH_ALL>()];
     // one copy of the tile code, two turns
     for (int turn = 0; turn < 2; ++turn) {
         const BatchJob bj = turn == 0 ? row : col;
-        run_job<WHOLE_THREADS, false>(bj, 0, lds);
+        run_job<WHOLE_THREADS, BATCH_ALL>(bj, 0, lds);
         if (turn == 1) break;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __syncthreads();

@@ -216,3 +216,78 @@ def test_smooth_lengths_in_a_dependent_batch(mdft, flags):
         torch.cuda.synchronize()
         p.close()
         assert torch.equal(torch.view_as_real(dst[o:o + w * h]), torch.view_as_real(alone)), (w, h)
+
+
+def run_batch(mdft, sizes, flags=0):
+    """(outputs of a batch on random images, outputs of plans on the same, info)"""
+    import torch
+
+    invs = [i % 2 == 1 for i in range(len(sizes))]
+    offs = np.cumsum([0] + [w * h for w, h in sizes])[:-1].tolist()
+    total = sum(w * h for w, h in sizes)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(total)
+    src = torch.randn(total, dtype=torch.complex64, device="cuda", generator=g)
+    dst, alone = torch.full_like(src, float("nan")), torch.full_like(src, float("nan"))
+    st = torch.cuda.current_stream().cuda_stream
+    b = mdft.Batch(sizes, invs, offs, offs, flags)
+    info = b.info()
+    b.exec_device(src.data_ptr(), dst.data_ptr(), st)
+    plans = {wh: mdft.Plan(*wh) for wh in set(sizes)}
+    for wh, inv, o in zip(sizes, invs, offs):
+        plans[wh].exec_device(inv, src.data_ptr() + 8 * o, alone.data_ptr() + 8 * o, st)
+    torch.cuda.synchronize()
+    b.close()
+    for p in plans.values():
+        p.close()
+    return torch.view_as_real(dst), torch.view_as_real(alone), info
+
+
+# The column phase of a batch by its number of tiles (256 CUs): 256 threads, 512 with one line per thread, with two:
+# (count, width, height, threads, column tiles)
+@pytest.mark.parametrize("count,w,h,threads,items", [
+    (1, 65, 701, 256, 33), (1, 2049, 701, 512, 513), (2, 4095, 701, 512, 1024), (1, 129, 509, 256, 33),
+    (1, 1025, 1201, 512, 513), (1, 2047, 1201, 512, 512), (1, 57, 4093, 256, 57), (1, 299, 4093, 512, 150),
+    (1, 255, 4096, 512, 128), (1, 513, 4096, 512, 129), (1, 511, 3072, 512, 256), (1, 801, 3072, 512, 201)])
+def test_batch_column_tiles(mdft, count, w, h, threads, items):
+    import torch
+
+    print(f"batch columns {count} x {w}x{h}", flush=True)
+    got, alone, info = run_batch(mdft, [(w, h)] * count)
+    assert torch.equal(got, alone)
+    assert (info["threads"][1], info["items"][1]) == (threads, items)
+
+
+# every FFT shape in one launch of each column kernel: one line per thread (a few images), two (eight times as many)
+def test_every_shape_in_every_column_kernel(mdft):
+    import torch
+
+    heights = [2, 3, 5, 9, 17, 33, 65, 129, 257, 509, 1021, 2047, 4093, 4, 8, 16, 32, 64, 128, 256, 512, 1024, 2048,
+               4096, 8192, 71, 139, 277, 701, 1201, 2999, 192, 384, 768, 1536, 3072, 6144, 18, 100, 1080, 2401, 3600]
+    items = []
+    for times in (1, 8):
+        print(f"every shape x {times}", flush=True)
+        got, alone, info = run_batch(mdft, [(35, h) for h in heights] * times)
+        assert torch.equal(got, alone)
+        assert info["threads"][1] == 512
+        items.append(info["items"][1])
+    assert items[1] < 8 * items[0]
+
+
+# A batch of one image costs about what its plan costs: few column tiles take the small forms (two lines per thread
+# in 512 threads: 1.5 to 1.9 times)
+@pytest.mark.parametrize("w,h", [(128, 509), (64, 1021), (256, 1201), (128, 2047)])
+def test_a_small_batch_costs_what_its_plans_cost(mdft, w, h):
+    import torch
+
+    src = torch.zeros(w * h, dtype=torch.complex64, device="cuda")
+    dst = torch.empty_like(src)
+    b, p = mdft.Batch([(w, h)], [False], [0], [0], 0), mdft.Plan(w, h)
+    b.exec_device(src.data_ptr(), dst.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    print(f"small batch {w}x{h}", flush=True)
+    r = time_ratio(captured(lambda st: b.exec_device(src.data_ptr(), dst.data_ptr(), st)),
+                   captured(lambda st: p.exec_device(False, src.data_ptr(), dst.data_ptr(), st)))
+    b.close()
+    p.close()
+    assert r <= 1.3, r
