@@ -2,8 +2,8 @@
 //
 // Each image contributes a row job and a column job, cut into tiles of whole
 // lines.  A small image whose rows and columns each fit one tile becomes a
-// single "whole" item done by one workgroup.  Without dependencies, items
-// are sorted by phase (whole images and row tiles first, column tiles
+// single "whole" item done by one workgroup.  Without dependencies, the jobs'
+// tile groups are sorted by phase (whole images and row tiles first, column tiles
 // second) and then by kernel variant (padded length, Bluestein or not, axis)
 // so neighbouring workgroups run the same code.  A line length gets the same
 // radix schedule in every batch, so a result is bitwise the same alone or in
@@ -19,8 +19,6 @@
 #include "../../../include/mdft.h"
 
 namespace mdft {
-
-void arrange_for_xcds(const std::vector<uint2>& items, const std::vector<double>& cost, std::vector<uint2>& out);
 
 int batch_threads_for(const uint32_t* widths, const uint32_t* heights, size_t count)
 {
@@ -54,6 +52,16 @@ static int lines_per_tile(int T, BatchHold hold, const LinePlan& lp)
 static bool runs_whole(int w, int h, int T, const LinePlan& row, const LinePlan& col)
 {
     return w > 1 && h > 1 && h <= lines_per_tile(T, BATCH_ALL, row) && w <= lines_per_tile(T, BATCH_ALL, col);
+}
+
+// the tiles of a group in order
+static uint32_t* write_tiles(const TileGroup& g, uint32_t* words)
+{
+    for (uint32_t t = 0; t < g.count; ++t) {
+        *words++ = g.job;
+        *words++ = g.first + t;
+    }
+    return words;
 }
 
 // cost of one line ~ points x passes
@@ -106,6 +114,7 @@ void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int T, i
     out.threads_cols = TC;
     if (job_image) job_image->clear();
     if (job_is_col) job_is_col->clear();
+    out.jobs.reserve(2 * count);
 
     std::vector<uint32_t> order(count);
     std::iota(order.begin(), order.end(), 0u);
@@ -115,14 +124,8 @@ void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int T, i
                   (double)compute_m(entries[i].height) * entries[i].width;
     std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t c) { return work[a] > work[c]; });
 
-    struct Item {
-        int phase;
-        int m, shape, blue, kind;  // kind: 0 whole, 1 row tile, 2 column tile
-        int lpw;                   // lines of its tile
-        uint32_t seq;
-        uint2 v;
-    };
-    std::vector<Item> items;
+    std::vector<TileGroup> groups;  // an image's one or two next to each other
+    groups.reserve(2 * count);
     std::vector<std::shared_ptr<const LinePlan>> plans(2 * count);  // rows, columns of every entry
     for (size_t i = 0; i < count; ++i) {
         plans[2 * i] = ctx.line_plan((int)entries[i].width, false);
@@ -130,8 +133,8 @@ void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int T, i
     }
     out.hold_cols = column_kernel(T, TC, ctx.cu_count(), entries, count, plans);
     if (out.hold_cols == BATCH_ALL) TC = out.threads_cols = T;
-    std::vector<std::pair<std::vector<uint2>, std::vector<uint2>>> per_image;  // dependency ordering
-    uint32_t counter = 0, seq = 0;
+    uint32_t counter = 0;
+    uint64_t nitems = 0;
     for (uint32_t idx : order) {
         const BatchEntry& e = entries[idx];
         const int w = (int)e.width, h = (int)e.height;
@@ -177,52 +180,41 @@ void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int T, i
             if (job_image) job_image->push_back(idx);
             if (job_is_col) job_is_col->push_back(1);
         }
-        std::vector<uint2> ri, ci;
+        auto add = [&](int phase, int kind, const LinePlan& lp, int lines, int job, uint32_t first, int tiles) {
+            const double cost = lines * line_cost(lp) * (lp.blue ? 2 : 1) * (kind == 0 ? 2 : 1);
+            groups.push_back({phase, lp.m, lp.shape, lp.blue, kind, (uint32_t)job, first, (uint32_t)tiles,
+                              std::max<int64_t>(1, std::llround(cost))});
+            nitems += (uint64_t)tiles;
+        };
         if (whole) {
-            items.push_back({1, rp->m, rp->shape, rp->blue, 0, lpw_r, seq++, make_uint2(rj, BATCH_WHOLE | (uint32_t)cj)});
-            ri.push_back(items.back().v);
+            add(1, 0, *rp, lpw_r, rj, BATCH_WHOLE | (uint32_t)cj, 1);
         } else {
-            for (int t = 0; t < ntr; ++t) {
-                items.push_back({1, rp->m, rp->shape, rp->blue, 1, lpw_r, seq++, make_uint2(rj, t)});
-                ri.push_back(items.back().v);
-            }
-            for (int t = 0; t < ntc; ++t) {
-                items.push_back({w > 1 ? 2 : 1, cp->m, cp->shape, cp->blue, 2, lpw_c, seq++, make_uint2(cj, t)});
-                ci.push_back(items.back().v);
-            }
+            if (ntr > 0) add(1, 1, *rp, lpw_r, rj, 0, ntr);
+            if (ntc > 0) add(w > 1 ? 2 : 1, 2, *cp, lpw_c, cj, 0, ntc);
         }
-        per_image.push_back({ri, ci});
     }
     out.keep = std::move(plans);
-
+    if (nitems > 0x7fffffff) throw Error(MDFT_ERR_SIZE, "batch of " + std::to_string(nitems) + " tiles");
+    out.items.resize((size_t)nitems);
+    uint32_t* words = reinterpret_cast<uint32_t*>(out.items.data());
     if (dependent) {
         // rows of image k+1 before columns of image k: a column tile only
         // waits on row tiles with smaller tickets
-        for (size_t k = 0; k < per_image.size(); ++k) {
-            out.items.insert(out.items.end(), per_image[k].first.begin(), per_image[k].first.end());
-            if (k > 0)
-                out.items.insert(out.items.end(), per_image[k - 1].second.begin(), per_image[k - 1].second.end());
+        const TileGroup* late = nullptr;  // columns of the image before
+        for (const TileGroup& g : groups) {
+            if (g.kind != 2) {
+                words = write_tiles(g, words);
+                if (late) words = write_tiles(*late, words);
+                late = nullptr;
+                continue;
+            }
+            if (late) words = write_tiles(*late, words);
+            late = &g;
         }
-        if (!per_image.empty())
-            out.items.insert(out.items.end(), per_image.back().second.begin(), per_image.back().second.end());
-        out.nphase1 = (uint32_t)out.items.size();
+        if (late) write_tiles(*late, words);
+        out.nphase1 = (uint32_t)nitems;
     } else {
-        std::stable_sort(items.begin(), items.end(), [](const Item& a, const Item& c) {
-            return std::make_tuple(a.phase, -a.m, a.shape, a.blue, a.kind, a.seq) <
-                   std::make_tuple(c.phase, -c.m, c.shape, c.blue, c.kind, c.seq);
-        });
-        std::vector<uint2> p1, p2;
-        std::vector<double> c1, c2;
-        for (const Item& it : items) {
-            // cost of a tile ~ points x passes (x2 for Bluestein's two FFTs)
-            const double cost = double(it.lpw) * double(it.m) * (std::log2(double(it.m)) + 2) * (it.blue ? 2.0 : 1.0) *
-                                (it.kind == 0 ? 2.0 : 1.0);
-            (it.phase == 1 ? p1 : p2).push_back(it.v);
-            (it.phase == 1 ? c1 : c2).push_back(cost);
-        }
-        out.nphase1 = (uint32_t)p1.size();
-        arrange_for_xcds(p1, c1, out.items);
-        arrange_for_xcds(p2, c2, out.items);
+        out.nphase1 = lay_out_tiles(groups, words);
     }
     out.ncounters = counter;
 }
@@ -231,58 +223,99 @@ void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int T, i
 // XCD b % 8, and each XCD has its own L2.  Give every job (its tiles, and
 // with them its chirp, diagonal and twiddle tables and, for column tiles,
 // the cache lines neighbouring tiles share) to one XCD, balancing the XCDs'
-// total cost (largest job first, jobs larger than an eighth of the launch
+// total cost (largest run first, jobs larger than a sixteenth of the launch
 // split), then lay the eight queues out so that queue x fills the blocks
-// b % 8 == x.  Within a queue the variant order of `items` is kept.
-void arrange_for_xcds(const std::vector<uint2>& items, const std::vector<double>& cost, std::vector<uint2>& out)
+// b % 8 == x.  Within a queue the order of the groups is kept.  Only the last
+// step touches single tiles: a burst of requests makes thousands, and its launch
+// waits for them (15 requests of 4781 tiles: 17 us for the whole build on the
+// scheduler's thread, 115 with every tile sorted, costed and copied by itself).
+static uint32_t* arrange_for_xcds(const TileGroup* groups, size_t ngroups, uint32_t* words)
 {
     constexpr int NXCD = 8;
-    const size_t n = items.size();
-    if (n == 0) return;
-    double total = 0;
-    for (double c : cost) total += c;
-    // runs of consecutive items of one job (items are grouped by variant, then job)
+    int64_t total = 0;
+    size_t n = 0;
+    for (size_t i = 0; i < ngroups; ++i) {
+        total += groups[i].cost * groups[i].count;
+        n += groups[i].count;
+    }
     struct Run {
-        size_t begin, end;
-        double cost;
+        uint32_t job, first, count;
+        int64_t cost;
     };
     std::vector<Run> runs;
-    const double cap = total / (2 * NXCD);
-    for (size_t i = 0; i < n;) {
-        size_t j = i;
-        double c = 0;
-        while (j < n && items[j].x == items[i].x && (j == i || c + cost[j] <= cap)) c += cost[j++];
-        runs.push_back({i, j, c});
-        i = j;
+    for (size_t i = 0; i < ngroups; ++i) {
+        const TileGroup& g = groups[i];
+        const int64_t most = std::max<int64_t>(1, total / (2 * NXCD * g.cost));
+        for (uint32_t t = 0; t < g.count;) {
+            const uint32_t k = (uint32_t)std::min<int64_t>(most, g.count - t);
+            runs.push_back({g.job, g.first + t, k, g.cost * k});
+            t += k;
+        }
     }
-    std::vector<size_t> by_cost(runs.size());
-    std::iota(by_cost.begin(), by_cost.end(), size_t(0));
-    std::stable_sort(by_cost.begin(), by_cost.end(), [&](size_t a, size_t b) { return runs[a].cost > runs[b].cost; });
-    std::vector<int> owner(runs.size());
-    double load[NXCD] = {};
-    for (size_t r : by_cost) {
+    std::vector<uint32_t> by_cost(runs.size());
+    std::iota(by_cost.begin(), by_cost.end(), 0u);
+    std::stable_sort(by_cost.begin(), by_cost.end(), [&](uint32_t a, uint32_t c) { return runs[a].cost > runs[c].cost; });
+    std::vector<uint8_t> owner(runs.size());
+    int64_t load[NXCD] = {};
+    for (uint32_t r : by_cost) {
         int best = 0;
         for (int x = 1; x < NXCD; ++x)
             if (load[x] < load[best]) best = x;
-        owner[r] = best;
+        owner[r] = (uint8_t)best;
         load[best] += runs[r].cost;
     }
-    std::vector<uint2> queue[NXCD];
-    for (size_t r = 0; r < runs.size(); ++r)
-        for (size_t i = runs[r].begin; i < runs[r].end; ++i) queue[owner[r]].push_back(items[i]);
-    // interleave; when a queue runs dry its slots take the longest remaining queue's items
-    size_t pos[NXCD] = {};
-    for (size_t b = 0; b < n; ++b) {
-        int x = int(b % NXCD);  // block index within this launch
-        if (pos[x] == queue[x].size()) {
-            int best = -1;
-            for (int y = 0; y < NXCD; ++y)
-                if (pos[y] < queue[y].size() && (best < 0 || queue[y].size() - pos[y] > queue[best].size() - pos[best]))
-                    best = y;
-            x = best;
-        }
-        out.push_back(queue[x][pos[x]++]);
+    struct Queue {
+        std::vector<Run> runs;
+        size_t at = 0, left = 0;  // the run being read, tiles not yet placed
+    } queue[NXCD];
+    for (size_t r = 0; r < runs.size(); ++r) {
+        queue[owner[r]].runs.push_back(runs[r]);
+        queue[owner[r]].left += runs[r].count;
     }
+    // while no queue is dry, queue x fills the blocks x, x + 8, ..
+    size_t rounds = queue[0].left;
+    for (const Queue& q : queue) rounds = std::min(rounds, q.left);
+    for (int x = 0; x < NXCD; ++x) {
+        Queue& q = queue[x];
+        uint32_t* w = words + 2 * x;
+        for (size_t left = rounds; left > 0;) {
+            Run& r = q.runs[q.at];
+            const uint32_t job = r.job, first = r.first, k = (uint32_t)std::min<size_t>(left, r.count);
+            for (uint32_t t = 0; t < k; ++t, w += 2 * NXCD) w[0] = job, w[1] = first + t;
+            r.first += k, r.count -= k, left -= k;
+            q.at += r.count == 0;
+        }
+        q.left -= rounds;
+    }
+    words += 2 * NXCD * rounds;
+    // then its slots take the longest remaining queue's items
+    for (size_t b = NXCD * rounds; b < n; ++b) {
+        int x = int(b % NXCD);  // block index within this launch
+        if (queue[x].left == 0)
+            for (int y = 0; y < NXCD; ++y)
+                if (queue[y].left > queue[x].left) x = y;
+        Queue& q = queue[x];
+        Run& r = q.runs[q.at];
+        *words++ = r.job;
+        *words++ = r.first++;
+        q.at += --r.count == 0;
+        --q.left;
+    }
+    return words;
+}
+
+uint32_t lay_out_tiles(std::vector<TileGroup>& groups, uint32_t* words)
+{
+    std::stable_sort(groups.begin(), groups.end(), [](const TileGroup& a, const TileGroup& c) {
+        return std::make_tuple(a.phase, -a.m, a.shape, a.blue, a.kind) <
+               std::make_tuple(c.phase, -c.m, c.shape, c.blue, c.kind);
+    });
+    size_t n1 = 0;
+    uint32_t tiles1 = 0;
+    for (; n1 < groups.size() && groups[n1].phase == 1; ++n1) tiles1 += groups[n1].count;
+    words = arrange_for_xcds(groups.data(), n1, words);
+    arrange_for_xcds(groups.data() + n1, groups.size() - n1, words);
+    return tiles1;
 }
 
 }  // namespace mdft

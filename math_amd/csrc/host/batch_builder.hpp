@@ -30,6 +30,17 @@ struct BatchEntry {
     float2* dst;
 };
 
+// The tiles of one job: items (job, first), (job, first + 1), ..
+struct TileGroup {
+    int phase;
+    int m, shape, blue, kind;  // kind: 0 a whole image, 1 row tiles, 2 column tiles
+    uint32_t job, first, count;
+    int64_t cost;  // of a tile: ~ points x passes (x2 for Bluestein's two FFTs, x2 for a whole image)
+};
+// Sorts groups by phase and kernel variant and writes the items of both phases
+// (two words each) as their launches take them; returns the items of phase 1.
+uint32_t lay_out_tiles(std::vector<TileGroup>& groups, uint32_t* words);
+
 // Workgroup size a set of sizes needs for whole images and row tiles: the
 // smallest of 256, 512 and 1024 threads that holds one line of the longest
 // padded length; throws MDFT_ERR_SIZE beyond the batch limit (8192).
