@@ -739,7 +739,7 @@ AxisTile axis_tile(int shape, bool blue, bool cols, int count, int variant, int 
             if (per_cu8(512) >= 8) return {512, true};
             if (per_cu8(256) >= 8) return {256, true};
         } else {
-            const int wide = wide_threads(shape, cols, blue);
+            const int wide = wide_threads(shape, cols);
             const int need = cols && wide / tpl_of(shape) >= 4 ? (blue ? 5 : 4) : 8;
             if (per_cu8(wide) >= need) return {wide, false};
         }

@@ -87,10 +87,12 @@ int mdft_tune_auto(double* seconds)
                     float best = 0;
                     int best_v = 0;
                     for (int v = 0; v < 2; ++v) {
-                        const int threads = v ? mdft::wide_threads(shape, cols != 0, blue != 0) : 256;
+                        // the tile a transform of this size gets under the entry
+                        const mdft::AxisTile tile =
+                            mdft::axis_tile(shape, blue != 0, cols != 0, count, v, ctx.cu_count());
                         auto launch = [&]() {
-                            mdft::hip_check(mdft::launch_axis(v && cols && mdft::has_x2(shape) ? shape | mdft::X2 : shape, j,
-                                                              blue != 0, cols != 0, threads, s),
+                            mdft::hip_check(mdft::launch_axis(tile.x2 ? shape | mdft::X2 : shape, j, blue != 0,
+                                                              cols != 0, tile.threads, s),
                                             "tuning launch");
                         };
                         const float ms = time_launches(s, launch, 5);
@@ -123,7 +125,7 @@ int mdft_tune_save(const char* path)
     Context& ctx = Context::get(Context::current_device());
     FILE* f = std::fopen(path, "w");
     if (!f) throw Error(MDFT_ERR_INVALID, std::string("tune: cannot write ") + path);
-    std::fprintf(f, "# mdft tile shapes: shape blue cols variant (0 = 256-thread tiles, 1 = 1024-thread tiles;\n"
+    std::fprintf(f, "# mdft tile shapes: shape blue cols variant (0 = 256-thread tiles, 1 = wider ones;\n"
                     "# shape 1..14: 2^shape points, 38..43: 3 * 2^(shape - 32) points)\n");
     for (int shape : all_shapes())
         for (int blue = 0; blue < 2; ++blue)

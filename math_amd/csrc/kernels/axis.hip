@@ -29,7 +29,7 @@ static hipError_t launch_axis_tt(const AxisJob& job, bool blue, hipStream_t stre
     if (grid64 == 0) return hipSuccess;
     const unsigned grid = (unsigned)grid64;
     if (blue) {
-        if constexpr (base_of(S) >= 2)
+        if constexpr (base_of(S) >= 2 && (!(S & X2) || x2_tile(S, T, true)))
             hipLaunchKernelGGL((k_axis<S, T, true, COLS>), dim3(grid), dim3(T), 0, stream, job);
         else
             return hipErrorInvalidValue;
@@ -56,7 +56,7 @@ static hipError_t launch_axis_t(const AxisJob& job, bool blue, bool x2, int thre
     }
     if constexpr (!(COLS && has_x2(S))) {
         if (threads >= 512 && threads > narrow_threads(S))
-            return launch_axis_tt<S, wide_threads(S, COLS, false), COLS>(job, blue, stream);
+            return launch_axis_tt<S, wide_threads(S, COLS), COLS>(job, blue, stream);
     }
     if constexpr (TPL <= 64) {
         if (threads <= 64) return launch_axis_tt<S, 64, COLS>(job, blue, stream);

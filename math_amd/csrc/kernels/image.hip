@@ -31,13 +31,15 @@ static hipError_t launch_image_tt(const AxisJob& job, const ImageIO& io, bool bl
     if (grid64 == 0) return hipSuccess;
     const unsigned grid = (unsigned)grid64;
     if (blue) {
-        // Bluestein X2 columns take 512 threads at most (Context::axis_tile)
-        if constexpr (base_of(S) >= 2 && !((S & X2) && T == 1024))
+        if constexpr (base_of(S) >= 2 && (!(S & X2) || x2_tile(S, T, true)))
             hipLaunchKernelGGL((k_image_axis<S, T, true, COLS, IO>), dim3(grid), dim3(T), 0, stream, job, io);
         else
             return hipErrorInvalidValue;
     } else {
-        hipLaunchKernelGGL((k_image_axis<S, T, false, COLS, IO>), dim3(grid), dim3(T), 0, stream, job, io);
+        if constexpr (!(S & X2) || T == 512 || m_of(S) >= 3072)
+            hipLaunchKernelGGL((k_image_axis<S, T, false, COLS, IO>), dim3(grid), dim3(T), 0, stream, job, io);
+        else
+            return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
@@ -79,7 +81,7 @@ static hipError_t launch_image_t(const AxisJob& job, const ImageIO& io, bool blu
     if (mode == IO_MAG) {
         if constexpr (!has_x2(S)) {
             if (threads >= 512 && threads > TN)
-                return launch_image_tt<S, wide_threads(S, true, false), true, IO_MAG>(job, io, blue, stream);
+                return launch_image_tt<S, wide_threads(S, true), true, IO_MAG>(job, io, blue, stream);
         }
         return launch_image_tt<S, TN, true, IO_MAG>(job, io, blue, stream);
     }

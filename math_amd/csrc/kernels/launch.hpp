@@ -99,12 +99,18 @@ hipError_t gen_dtab(float2* dtab, const double2* chirp64, double* cos_scratch, i
 // shape with an X2 form whether it takes that (launch_axis: shape | X2).
 // Narrow: 256 threads, or one line when a line needs more (16384 points: 512).
 __host__ __device__ constexpr int narrow_threads(int shape) { return tpl_of(shape) > 256 ? tpl_of(shape) : 256; }
-// the widest tiles: X2 columns in 1024 threads when direct, 512 for Bluestein
-// (Context::axis_tile); else 6144-point columns in 512 threads (3000^2 184 us
-// against 195 in 1024) and 1024 (8192-point columns, 2048 x 8192: 128 us against 167)
-__host__ __device__ constexpr int wide_threads(int shape, bool cols, bool blue)
+// the widest tiles with one line per thread: 6144-point columns in 512 threads
+// (3000^2 184 us against 195 in 1024), others in 1024 (8192-point columns, 2048 x
+// 8192: 128 us against 167)
+__host__ __device__ constexpr int wide_threads(int shape, bool cols)
 {
-    return cols && (ept_of(shape) == 24 || (blue && has_x2(shape))) ? 512 : 1024;
+    return cols && ept_of(shape) == 24 ? 512 : 1024;
+}
+// the X2 tiles there are, those axis_tile picks: direct ones in 256, 512 and 1024
+// threads, Bluestein in 256 and from 2048 points in 512
+__host__ __device__ constexpr bool x2_tile(int shape, int threads, bool blue)
+{
+    return !blue || threads == 256 || (threads == 512 && m_of(shape) >= 2048);
 }
 // threads: 1024, 512 (wide tiles, clamped to the shape's), 256, 128 or 64 (clamped to one line per workgroup);
 // shape + X2: columns in 1024, 512 or 256 threads

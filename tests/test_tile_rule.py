@@ -2,6 +2,7 @@
 tiles they are there for (a moved line fails here, where the GPU test would
 quietly compare a kernel with itself)."""
 import os
+import re
 import subprocess
 
 import pytest
@@ -55,3 +56,24 @@ def test_8192_point_columns(ask, w, h, threads):
 def test_image_cases_with_smooth_heights_are_named_apart(ask):
     assert ask(("n", 1080, 1)) == [GEN_SHAPE]
     assert ask(("n", 71, 1)) == [38] and ask(("n", 139, 1)) == [39]
+
+
+# Two-line tiles: the library holds the ones the rule picks over all counts, and no others (the autotuner times what
+# the rule picks, too)
+@pytest.mark.parametrize("kernel,args", [("k_axis", r"true"), ("k_image_axis", r"true, 2")])
+def test_two_line_tiles_are_the_ones_the_rule_picks(ask, kernel, args):
+    names = subprocess.run(["nm", "-C", os.path.join(ROOT, "math_amd", "lib", "libmdft.so")], capture_output=True,
+                           text=True, check=True).stdout
+    held = {tuple(m) for m in re.findall(rf"device_stub__{kernel}<(\d+), (\d+), (true|false), {args}>", names)
+            if int(m[0]) >= 64}
+    picked = set()
+    for shape in (10, 11, 12, 41, 42):
+        for blue in (False, True):
+            queries = [q for count in range(1, 20000, 61) for q in (shape, blue, True, count, 1)]
+            answers = ask(queries)
+            for threads, x2 in zip(answers[::2], answers[1::2]):
+                if x2:
+                    picked.add((str(shape + 64), str(threads), "true" if blue else "false"))
+    if kernel == "k_image_axis":  # direct columns below 3072 points: 512 threads only
+        picked -= {(str(s + 64), t, "false") for s in (10, 11, 41) for t in ("256", "1024")}
+    assert held == picked
