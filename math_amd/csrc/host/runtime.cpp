@@ -171,6 +171,28 @@ int line_shape(long long n, bool cols)
     return ilog2((uint64_t)m);
 }
 
+LineFit line_fit(long long n, bool cols)
+{
+    const int shape = line_shape(n, cols);
+    if (shape == GEN_SHAPE) {
+        GenPlan plan;
+        smooth_plan(n, &plan);
+        return {plan.tpl, 0};
+    }
+    return {tpl_of(shape), m_of(shape) == n ? 0 : m_of(shape)};
+}
+
+// Two Bluestein axes are two chains of two FFTs, which take one workgroup longer
+// than the second launch: 10 x 10 7.7 us of device time in one launch, 6.4 in
+// two, 31 x 31 8.5 and 7.4; with one direct axis (50 x 50 6.4, 6.7), or an axis
+// padded to 16 points or less, the one launch is as fast or nearly so and leaves
+// the caller an enqueue less (7 x 7 5.4, 5.0, but 6.6 and 8.9 us a call).
+bool one_launch(const LineFit& row, const LineFit& col, int w, int h)
+{
+    if (w < 2 || h < 2 || int64_t(row.tpl) * h > WHOLE_THREADS || int64_t(col.tpl) * w > WHOLE_THREADS) return false;
+    return row.conv < 32 || col.conv < 32;
+}
+
 LinePlan::~LinePlan()
 {
     if (chirp) (void)hipFree(chirp);
@@ -306,6 +328,7 @@ std::shared_ptr<const LinePlan> Context::line_plan(int n, bool cols)
     lp->logm = smooth || is_f3(lp->shape) ? 0 : ilog2((uint64_t)m);
     // powers of two, n = 3 * 2^k and other smooth lengths run a direct FFT of length n
     lp->blue = lp->m != n;
+    lp->fit = line_fit(n, cols);
     if (lp->logm > LARGE_MAX_LOGM)
         throw Error(MDFT_ERR_SIZE, "Error size " + std::to_string(n) + ": padded length " + std::to_string(m) +
                                        " exceeds the longest supported line (2^" + std::to_string(LARGE_MAX_LOGM) +
@@ -764,22 +787,10 @@ int Context::smooth_threads(const GenPlan& plan, bool cols, int count) const
     return t;
 }
 
-// Whether all rows, and all columns, of an image fit one tile of the single-launch kernel
-bool Context::one_tile(const LinePlan& row, const LinePlan& col, int w, int h)
-{
-    if (w < 2 || h < 2 || row.large() || col.large()) return false;
-    auto fits = [](const LinePlan& lp, int count) {
-        const int64_t tpl = lp.gen ? lp.smooth.tpl : tpl_of(lp.shape);
-        // tpl of 8192 points: 256 threads; longer lines do not fit
-        return tpl * count <= WHOLE_THREADS;
-    };
-    return fits(row, h) && fits(col, w);
-}
-
 void Context::enqueue_transform(const LinePlan& row, const LinePlan& col, int w, int h, bool inverse,
                                 const float2* src, float2* dst, float2* scratch, hipStream_t stream) const
 {
-    if (one_tile(row, col, w, h)) {
+    if (one_launch(row.fit, col.fit, w, h)) {
         auto job = [&](const LinePlan& lp, const float2* from, int64_t es, int64_t ls, int count, bool cols) {
             BatchJob j{};
             j.job = make_job(lp, from, dst, es, ls, count, inverse);

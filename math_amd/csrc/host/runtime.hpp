@@ -70,6 +70,16 @@ void large_split(int logm, int* l1, int* l2, int* l3);
 // elements above one tile, none otherwise
 uint64_t large_scratch_elems(long long m, long long count);
 
+// Threads a line of length n takes, and its convolution length (0: direct).
+struct LineFit {
+    int tpl = 1;
+    int conv = 0;
+};
+LineFit line_fit(long long n, bool cols);
+// Whether an image runs in the single-launch kernel: all its rows, and all its
+// columns, fit one tile of that, and it is the better one.
+bool one_launch(const LineFit& row, const LineFit& col, int w, int h);
+
 // Device tables of one line length n.
 struct LinePlan {
     int n = 0;
@@ -85,6 +95,7 @@ struct LinePlan {
     // smooth lengths: pass table and twiddle rows, and the plan they were made from
     float2* gen = nullptr;
     GenPlan smooth{};
+    LineFit fit;
     // lines longer than one tile: M = 2^logm1 * 2^logm2 (four-step), or
     // 2^logm1 * 2^logm2 * 2^logm3 (logm3 > 0: three factors), with a
     // two-level table of exp(-2*pi*i*j/M)
@@ -180,7 +191,6 @@ public:
     {
         return mdft::axis_tile(shape, blue, cols, count, variant(shape, blue, cols), cu_count_);
     }
-    static bool one_tile(const LinePlan& row, const LinePlan& col, int w, int h);
     // workgroup size of a pass over `count` lines of a smooth length (launch_smooth)
     int smooth_threads(const GenPlan& plan, bool cols, int count) const;
     void set_variant(int shape, bool blue, bool cols, int v) { variant_[shape_index(shape)][blue][cols] = (uint8_t)v; }

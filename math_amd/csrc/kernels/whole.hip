@@ -1,8 +1,10 @@
 // A small image in one launch: one workgroup runs the row tile, makes its
 // stores visible to its own waves, then runs the column tile (the whole items
 // of a batch).  For images whose rows and whose columns fit one 256-thread tile
-// the second launch costs as much as the work: 64 x 64 takes 9.5 us in two
-// launches, 5.5 in one; 50 x 50 10.3 and 6.2; 16 x 16 6.2 and 3.7.  With 1024
+// the second launch costs about what it saves on the device, and its enqueue on
+// the host (device time, and time per call among others): 64 x 64 takes 5.5 and
+// 6.3 us in one launch, 5.4 and 8.8 in two; 50 x 50 6.4 and 7.3, 6.7 and 8.9;
+// 16 x 16 3.5 and 5.9, 3.8 and 8.9.  Which images take it: one_launch.  With 1024
 // threads larger images fit, but one CU is then slower than two launches over
 // many (100 x 37 13.2 us against 9.2, 61 x 67 18.4 against 9.9).
 #include <hip/hip_runtime.h>

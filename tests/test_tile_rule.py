@@ -77,3 +77,12 @@ def test_two_line_tiles_are_the_ones_the_rule_picks(ask, kernel, args):
     if kernel == "k_image_axis":  # direct columns below 3072 points: 512 threads only
         picked -= {(str(s + 64), t, "false") for s in (10, 11, 41) for t in ("256", "1024")}
     assert held == picked
+
+
+# one launch: all rows and all columns in 256 threads, and not two Bluestein axes of 32 points or more
+@pytest.mark.parametrize("w,h,one", [(2, 2, 1), (16, 16, 1), (64, 64, 1), (65, 64, 0), (64, 65, 0), (50, 50, 1),
+                                     (100, 37, 0), (9, 9, 1), (6, 10, 1), (10, 10, 0), (14, 11, 0), (22, 11, 0),
+                                     (31, 31, 0), (61, 29, 0), (61, 13, 0), (20, 11, 1), (64, 11, 1), (11, 64, 1),
+                                     (1, 5, 0), (5, 1, 0), (4096, 2, 0), (256, 16, 1), (257, 16, 0)])
+def test_images_of_one_launch(ask, w, h, one):
+    assert ask(("one", w, h)) == [one]
