@@ -16,8 +16,7 @@ using mdft::LinePlan;
 struct mdft_batch_s {
     int device = 0;
     uint32_t flags = 0;
-    int threads = 256;       // whole images and row tiles
-    int threads_cols = 256;  // column tiles
+    int threads_cols = mdft::BATCH_THREADS;  // column tiles
     std::vector<mdft_desc> descs;
     mdft::BatchBuild build;
     std::vector<uint32_t> job_image;
@@ -61,7 +60,6 @@ void count_phase_bytes(mdft_batch_s* b)
 
 void enqueue_batch(mdft_batch_s* b, hipStream_t stream)
 {
-    const int T = b->threads;
     if (b->flags & MDFT_BATCH_DEPENDENT) {
         mdft::hip_check(mdft::launch_batch_persistent(b->jobs_dev, b->items_dev, b->nitems, b->ctl_dev, b->nctl,
                                                       b->grid, b->spin_limit, stream),
@@ -75,7 +73,8 @@ void enqueue_batch(mdft_batch_s* b, hipStream_t stream)
                                                       b->spin_limit, stream),
                         "batch launch (phase 2)");
     } else {
-        mdft::hip_check(mdft::launch_batch_grid(T, mdft::BATCH_ALL, b->jobs_dev, b->items_dev, b->nphase1, stream),
+        mdft::hip_check(mdft::launch_batch_grid(mdft::BATCH_THREADS, mdft::BATCH_ALL, b->jobs_dev, b->items_dev,
+                                                b->nphase1, stream),
                         "batch launch (phase 1)");
         mdft::hip_check(mdft::launch_batch_grid(b->threads_cols, b->build.hold_cols, b->jobs_dev,
                                                 b->items_dev + b->nphase1, b->nitems - b->nphase1, stream),
@@ -85,10 +84,10 @@ void enqueue_batch(mdft_batch_s* b, hipStream_t stream)
 
 // Time the column phase of one batch layout (column tiles of TC threads) on
 // zeroed scratch images: build, upload, one warm-up and three timed launches.
-float time_column_phase(Context& ctx, const std::vector<mdft::BatchEntry>& entries, int T, int TC, hipStream_t s)
+float time_column_phase(Context& ctx, const std::vector<mdft::BatchEntry>& entries, int TC, hipStream_t s)
 {
     mdft::BatchBuild bb;
-    mdft::build_batch(ctx, entries.data(), entries.size(), T, TC, false, bb);
+    mdft::build_batch(ctx, entries.data(), entries.size(), TC, false, bb);
     const uint32_t n2 = (uint32_t)bb.items.size() - bb.nphase1;
     if (n2 == 0) return 0.0f;
     BatchJob* jobs = nullptr;
@@ -121,14 +120,14 @@ float time_column_phase(Context& ctx, const std::vector<mdft::BatchEntry>& entri
 
 // Column-tile size of a grid-shape batch picked by measurement: 256 (when the
 // row tiles are 256-thread), 512 or 1024 threads.
-int tune_column_threads(Context& ctx, const mdft_desc* descs, uint32_t count, int T)
+int tune_column_threads(Context& ctx, const mdft_desc* descs, uint32_t count)
 {
     uint64_t total = 0;
     for (uint32_t i = 0; i < count; ++i) total += (uint64_t)descs[i].width * descs[i].height;
     float2* scratch = nullptr;
     mdft::hip_check(hipMalloc(&scratch, sizeof(float2) * std::max<uint64_t>(total, 1)), "hipMalloc tuning images");
     hipStream_t s = nullptr;
-    int best = mdft::BATCH_COL_THREADS > T ? mdft::BATCH_COL_THREADS : T;
+    int best = mdft::BATCH_COL_THREADS;
     try {
         mdft::hip_check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "hipStreamCreate");
         mdft::hip_check(hipMemsetAsync(scratch, 0, sizeof(float2) * std::max<uint64_t>(total, 1), s), "clear");
@@ -140,8 +139,7 @@ int tune_column_threads(Context& ctx, const mdft_desc* descs, uint32_t count, in
         }
         float best_ms = -1.0f;
         for (int tc : {256, 512, 1024}) {
-            if (tc < T) continue;
-            const float ms = time_column_phase(ctx, entries, T, tc, s);
+            const float ms = time_column_phase(ctx, entries, tc, s);
             if (best_ms < 0 || ms < best_ms) {
                 best_ms = ms;
                 best = tc;
@@ -172,25 +170,24 @@ int mdft_batch_create(mdft_batch* batch, const mdft_desc* descs, uint32_t count,
         ws[i] = descs[i].width;
         hs[i] = descs[i].height;
     }
-    const int T = mdft::batch_threads_for(ws.data(), hs.data(), count);  // validates sizes
+    mdft::check_batch_sizes(ws.data(), hs.data(), count);
 
     Context& ctx = Context::get(Context::current_device());
     mdft::DeviceGuard g(ctx.device());
     auto b = std::make_unique<mdft_batch_s>();
     b->device = ctx.device();
     b->flags = flags;
-    b->threads = T;
     // grid launches run column tiles in wide tiles; the persistent shapes use one size
     const bool grid_shape = !(flags & (MDFT_BATCH_PERSISTENT | MDFT_BATCH_DEPENDENT));
-    b->threads_cols = grid_shape ? (mdft::BATCH_COL_THREADS > T ? mdft::BATCH_COL_THREADS : T) : T;
-    if (grid_shape && (flags & MDFT_BATCH_TUNE)) b->threads_cols = tune_column_threads(ctx, descs, count, T);
+    b->threads_cols = grid_shape ? mdft::BATCH_COL_THREADS : mdft::BATCH_THREADS;
+    if (grid_shape && (flags & MDFT_BATCH_TUNE)) b->threads_cols = tune_column_threads(ctx, descs, count);
     b->descs.assign(descs, descs + count);
     std::vector<mdft::BatchEntry> entries(count);
     for (uint32_t i = 0; i < count; ++i) {
         entries[i] = {descs[i].width, descs[i].height, descs[i].inverse != 0, nullptr, nullptr};
         if (descs[i].width == 1 && descs[i].height == 1) b->copies.push_back(i);
     }
-    mdft::build_batch(ctx, entries.data(), count, T, b->threads_cols, (flags & MDFT_BATCH_DEPENDENT) != 0, b->build,
+    mdft::build_batch(ctx, entries.data(), count, b->threads_cols, (flags & MDFT_BATCH_DEPENDENT) != 0, b->build,
                       &b->job_image, &b->job_is_col);
     b->threads_cols = b->build.threads_cols;
     b->nphase1 = b->build.nphase1;
@@ -297,8 +294,8 @@ int mdft_batch_exec_phase(mdft_batch b, int phase, const void* src, void* dst, v
     hipStream_t stream = static_cast<hipStream_t>(stream_p);
     if (phase == 1) {
         prepare_exec(b, src, dst, stream);
-        mdft::hip_check(mdft::launch_batch_grid(b->threads, mdft::BATCH_ALL, b->jobs_dev, b->items_dev, b->nphase1,
-                                                stream),
+        mdft::hip_check(mdft::launch_batch_grid(mdft::BATCH_THREADS, mdft::BATCH_ALL, b->jobs_dev, b->items_dev,
+                                                b->nphase1, stream),
                         "batch launch (phase 1)");
     } else {
         if (src != b->cur_src || dst != b->cur_dst)
@@ -320,7 +317,7 @@ int mdft_batch_info(mdft_batch b, uint32_t* items1, uint32_t* items2, uint64_t* 
     if (items2) *items2 = b->nitems - b->nphase1;
     if (bytes1) *bytes1 = b->phase_bytes[0];
     if (bytes2) *bytes2 = b->phase_bytes[1];
-    if (threads1) *threads1 = (uint32_t)b->threads;
+    if (threads1) *threads1 = (uint32_t)mdft::BATCH_THREADS;
     if (threads2) *threads2 = (uint32_t)b->threads_cols;
     MDFT_API_END
 }

@@ -20,38 +20,33 @@
 
 namespace mdft {
 
-int batch_threads_for(const uint32_t* widths, const uint32_t* heights, size_t count)
+void check_batch_sizes(const uint32_t* widths, const uint32_t* heights, size_t count)
 {
     const int limit = batch_max_logm();
-    int tpl = 1;
     for (size_t i = 0; i < count; ++i) {
         compute_m(widths[i]);  // validates the sides
         compute_m(heights[i]);
         // the FFT lengths the tiles run (the padded length, or 3 * 2^k; a smooth length itself)
-        for (int shape : {line_shape(widths[i], false), line_shape(heights[i], true)}) {
-            if (shape == GEN_SHAPE) continue;
-            if (m_of(shape) > (1 << limit))
+        for (int shape : {line_shape(widths[i], false), line_shape(heights[i], true)})
+            if (shape != GEN_SHAPE && m_of(shape) > (1 << limit))
                 throw Error(MDFT_ERR_SIZE, "batch transform " + std::to_string(i) + " (" + std::to_string(widths[i]) +
                                                "x" + std::to_string(heights[i]) +
                                                ") exceeds the batch padded-length limit " +
                                                std::to_string(1 << limit));
-            tpl = std::max(tpl, tpl_of(shape));
-        }
     }
-    // the smallest tile that holds a whole line of every length (256 threads up to the limit)
-    return tpl <= 256 ? 256 : tpl <= 512 ? 512 : 1024;
 }
 
-// lines a tile of T threads holds of a plan's length
-static int lines_per_tile(int T, BatchHold hold, const LinePlan& lp)
+// lines a tile holds of a plan's length
+static int lines_per_tile(int threads, BatchHold hold, const LinePlan& lp)
 {
-    return lp.gen ? T / lp.smooth.tpl : batch_lines_per_tile(T, hold, lp.shape);
+    return lp.gen ? threads / lp.smooth.tpl : batch_lines_per_tile(threads, hold, lp.shape);
 }
+static int lines_per_tile(const LinePlan& lp) { return lines_per_tile(BATCH_THREADS, BATCH_ALL, lp); }
 
 // whole images run both passes in one row-phase workgroup
-static bool runs_whole(int w, int h, int T, const LinePlan& row, const LinePlan& col)
+static bool runs_whole(int w, int h, const LinePlan& row, const LinePlan& col)
 {
-    return w > 1 && h > 1 && h <= lines_per_tile(T, BATCH_ALL, row) && w <= lines_per_tile(T, BATCH_ALL, col);
+    return w > 1 && h > 1 && h <= lines_per_tile(row) && w <= lines_per_tile(col);
 }
 
 // the tiles of a group in order
@@ -82,10 +77,10 @@ static double line_cost(const LinePlan& lp) { return double(lp.m) * (std::log2(d
 //    2048 x 1536 13.0 (14.5 with one), 1024 x 3072 16.5 (21.5), 512 x 4096 15.0 (15.6);
 //  * one line per thread as well where no line has the two-line form (2048 x 4093
 //    65.6, 70.4 in the kernel with two).
-static BatchHold column_kernel(int T, int TC, int cu_count, const BatchEntry* entries, size_t count,
+static BatchHold column_kernel(int TC, int cu_count, const BatchEntry* entries, size_t count,
                                const std::vector<std::shared_ptr<const LinePlan>>& plans)
 {
-    if (TC <= T) return BATCH_ALL;
+    if (TC <= BATCH_THREADS) return BATCH_ALL;
     if (TC != BATCH_COL_THREADS) return BATCH_COLS_X2;
     double narrow = 0, dearest = 0;
     int64_t two = 0;
@@ -93,8 +88,8 @@ static BatchHold column_kernel(int T, int TC, int cu_count, const BatchEntry* en
     for (size_t i = 0; i < count; ++i) {
         const int w = (int)entries[i].width, h = (int)entries[i].height;
         const LinePlan &row = *plans[2 * i], &col = *plans[2 * i + 1];
-        if (w <= 1 || h <= 1 || runs_whole(w, h, T, row, col)) continue;
-        const int n1 = lines_per_tile(T, BATCH_ALL, col), n2 = lines_per_tile(TC, BATCH_COLS_X2, col);
+        if (w <= 1 || h <= 1 || runs_whole(w, h, row, col)) continue;
+        const int n1 = lines_per_tile(col), n2 = lines_per_tile(TC, BATCH_COLS_X2, col);
         const double cost = n1 * line_cost(col);
         narrow += (w + n1 - 1) / n1 * cost * (col.blue ? 1 : 2);
         dearest = std::max(dearest, cost);
@@ -106,11 +101,10 @@ static BatchHold column_kernel(int T, int TC, int cu_count, const BatchEntry* en
     return any_two && 2 * two >= 3 * int64_t(cu_count) ? BATCH_COLS_X2 : BATCH_COLS;
 }
 
-void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int T, int TC, bool dependent,
-                 BatchBuild& out, std::vector<uint32_t>* job_image, std::vector<uint8_t>* job_is_col)
+void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int TC, bool dependent, BatchBuild& out,
+                 std::vector<uint32_t>* job_image, std::vector<uint8_t>* job_is_col)
 {
     out = BatchBuild{};
-    out.threads = T;
     out.threads_cols = TC;
     if (job_image) job_image->clear();
     if (job_is_col) job_is_col->clear();
@@ -131,21 +125,21 @@ void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int T, i
         plans[2 * i] = ctx.line_plan((int)entries[i].width, false);
         plans[2 * i + 1] = ctx.line_plan((int)entries[i].height, true);
     }
-    out.hold_cols = column_kernel(T, TC, ctx.cu_count(), entries, count, plans);
-    if (out.hold_cols == BATCH_ALL) TC = out.threads_cols = T;
+    out.hold_cols = column_kernel(TC, ctx.cu_count(), entries, count, plans);
+    if (out.hold_cols == BATCH_ALL) TC = out.threads_cols = BATCH_THREADS;
     uint32_t counter = 0;
     uint64_t nitems = 0;
     for (uint32_t idx : order) {
         const BatchEntry& e = entries[idx];
         const int w = (int)e.width, h = (int)e.height;
         const LinePlan *rp = plans[2 * idx].get(), *cp = plans[2 * idx + 1].get();
-        const int lpw_r = w > 1 ? lines_per_tile(T, BATCH_ALL, *rp) : 0;
-        const bool whole = runs_whole(w, h, T, *rp, *cp);
+        const int lpw_r = w > 1 ? lines_per_tile(*rp) : 0;
+        const bool whole = runs_whole(w, h, *rp, *cp);
         // column tiles of images with a row pass run in the column phase (TC
         // threads); a single-column-pass image (w == 1) runs with the rows
         const int lpw_c = h <= 1             ? 0
                           : w > 1 && !whole ? lines_per_tile(TC, out.hold_cols, *cp)
-                                            : lines_per_tile(T, BATCH_ALL, *cp);
+                                            : lines_per_tile(*cp);
         const int ntr = w > 1 ? (h + lpw_r - 1) / lpw_r : 0;
         const int ntc = h > 1 ? (w + lpw_c - 1) / lpw_c : 0;
         const int sig = (dependent && w > 1 && h > 1 && !whole) ? (int)counter++ : -1;

@@ -11,8 +11,7 @@
 namespace mdft {
 
 struct BatchBuild {
-    int threads = 256;       // workgroup size of whole images and row tiles
-    int threads_cols = 256;  // workgroup size of column tiles
+    int threads_cols = BATCH_THREADS;  // workgroup size of column tiles
     BatchHold hold_cols = BATCH_ALL;  // and the kernel that runs them
     std::vector<BatchJob> jobs;
     std::vector<uint2> items;
@@ -41,18 +40,16 @@ struct TileGroup {
 // (two words each) as their launches take them; returns the items of phase 1.
 uint32_t lay_out_tiles(std::vector<TileGroup>& groups, uint32_t* words);
 
-// Workgroup size a set of sizes needs for whole images and row tiles: the
-// smallest of 256, 512 and 1024 threads that holds one line of the longest
-// padded length; throws MDFT_ERR_SIZE beyond the batch limit (8192).
-int batch_threads_for(const uint32_t* widths, const uint32_t* heights, size_t count);
+// Throws MDFT_ERR_SIZE where a side or its padded length is beyond the batch limit (8192).
+void check_batch_sizes(const uint32_t* widths, const uint32_t* heights, size_t count);
 
 // Builds jobs and items.  dependent: one-launch ordering with per-image
 // counters; otherwise two phases sorted by kernel variant.  job_image[i]
 // receives the index of the entry each job belongs to and job_is_col[i]
 // whether it is the column job.
-// threads: tiles of whole images and rows; threads_cols: column tiles.
-void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int threads, int threads_cols,
-                 bool dependent, BatchBuild& out, std::vector<uint32_t>* job_image = nullptr,
+// threads_cols: column tiles, 512 for what column_kernel picks.
+void build_batch(Context& ctx, const BatchEntry* entries, size_t count, int threads_cols, bool dependent,
+                 BatchBuild& out, std::vector<uint32_t>* job_image = nullptr,
                  std::vector<uint8_t>* job_is_col = nullptr);
 
 }  // namespace mdft

@@ -213,14 +213,8 @@ void grow(Lane& L, size_t njobs, size_t nitems)
 void launch_micro_batch(mdft_server_s* s, Lane& L, const std::vector<mdft::BatchEntry>& entries)
 {
     Context& ctx = Context::get(s->device);
-    std::vector<uint32_t> ws(entries.size()), hs(entries.size());
-    for (size_t i = 0; i < entries.size(); ++i) {
-        ws[i] = entries[i].width;
-        hs[i] = entries[i].height;
-    }
-    const int T = mdft::batch_threads_for(ws.data(), hs.data(), entries.size());
     mdft::BatchBuild bb;
-    mdft::build_batch(ctx, entries.data(), entries.size(), T, std::max(T, mdft::BATCH_COL_THREADS), false, bb);
+    mdft::build_batch(ctx, entries.data(), entries.size(), mdft::BATCH_COL_THREADS, false, bb);
     grow(L, bb.jobs.size(), bb.items.size());
     // jobs at the start of the table, items after the lane's job capacity: one upload
     BatchJob* jobs_host = reinterpret_cast<BatchJob*>(L.table_host);
@@ -240,7 +234,8 @@ void launch_micro_batch(mdft_server_s* s, Lane& L, const std::vector<mdft::Batch
         if (e.width == 1 && e.height == 1)
             mdft::hip_check(hipMemcpyAsync(e.dst, e.src, sizeof(float2), hipMemcpyDeviceToDevice, L.stream), "copy");
     const uint32_t n = (uint32_t)bb.items.size();
-    mdft::hip_check(mdft::launch_batch_grid(T, mdft::BATCH_ALL, jobs_dev, items_dev, bb.nphase1, L.stream),
+    mdft::hip_check(mdft::launch_batch_grid(mdft::BATCH_THREADS, mdft::BATCH_ALL, jobs_dev, items_dev, bb.nphase1,
+                                            L.stream),
                     "serve launch");
     mdft::hip_check(mdft::launch_batch_grid(bb.threads_cols, bb.hold_cols, jobs_dev, items_dev + bb.nphase1,
                                             n - bb.nphase1, L.stream),
@@ -436,7 +431,7 @@ static void server_submit(mdft_server s, uint32_t width, uint32_t height, int in
 {
     if (!s) throw Error(MDFT_ERR_NO_BUFFERS, "No DFT buffers");
     if (!src || !ticket) throw Error(MDFT_ERR_INVALID, "mdft_server_submit: src and ticket must not be NULL");
-    mdft::batch_threads_for(&width, &height, 1);  // size checks
+    mdft::check_batch_sizes(&width, &height, 1);
     Request r;
     r.w = width;
     r.h = height;

@@ -158,31 +158,20 @@ __device__ __noinline__ void run_tile_call(const BatchJob* jobs, uint32_t job, i
     run_tile_body<S, T, BATCH_ALL>(bj.job, bj.blue, bj.cols, __builtin_amdgcn_readfirstlane(tile), lds);
 }
 
+// every shape a batch runs
+#define MDFT_BATCH_SHAPES(X)                                                                           \
+    X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(F3_BASE + 6) X(F3_BASE + 7) \
+    X(F3_BASE + 8) X(F3_BASE + 9) X(F3_BASE + 10) X(F3_BASE + 11) X(GEN_SHAPE)
+
 template <int T, bool INL, BatchHold H>
 __device__ __forceinline__ void run_job_tile(const BatchJob* jobs, uint32_t job, int tile, float* lds)
 {
     const BatchJob bj = jobs[job];
     switch (bj.shape) {
-    case 1: run_tile<1, T, INL, H>(jobs, job, bj, tile, lds); break;
-    case 2: run_tile<2, T, INL, H>(jobs, job, bj, tile, lds); break;
-    case 3: run_tile<3, T, INL, H>(jobs, job, bj, tile, lds); break;
-    case 4: run_tile<4, T, INL, H>(jobs, job, bj, tile, lds); break;
-    case 5: run_tile<5, T, INL, H>(jobs, job, bj, tile, lds); break;
-    case 6: run_tile<6, T, INL, H>(jobs, job, bj, tile, lds); break;
-    case 7: run_tile<7, T, INL, H>(jobs, job, bj, tile, lds); break;
-    case 8: run_tile<8, T, INL, H>(jobs, job, bj, tile, lds); break;
-    case 9: run_tile<9, T, INL, H>(jobs, job, bj, tile, lds); break;
-    case 10: run_tile<10, T, INL, H>(jobs, job, bj, tile, lds); break;
-    case 11: run_tile<11, T, INL, H>(jobs, job, bj, tile, lds); break;
-    case 12: run_tile<12, T, INL, H>(jobs, job, bj, tile, lds); break;
-    case 13: run_tile<13, T, INL, H>(jobs, job, bj, tile, lds); break;
-    case F3_BASE + 6: run_tile<F3_BASE + 6, T, INL, H>(jobs, job, bj, tile, lds); break;
-    case F3_BASE + 7: run_tile<F3_BASE + 7, T, INL, H>(jobs, job, bj, tile, lds); break;
-    case F3_BASE + 8: run_tile<F3_BASE + 8, T, INL, H>(jobs, job, bj, tile, lds); break;
-    case F3_BASE + 9: run_tile<F3_BASE + 9, T, INL, H>(jobs, job, bj, tile, lds); break;
-    case F3_BASE + 10: run_tile<F3_BASE + 10, T, INL, H>(jobs, job, bj, tile, lds); break;
-    case F3_BASE + 11: run_tile<F3_BASE + 11, T, INL, H>(jobs, job, bj, tile, lds); break;
-    case GEN_SHAPE: run_tile<GEN_SHAPE, T, INL, H>(jobs, job, bj, tile, lds); break;
+#define MDFT_CASE(S) \
+    case S: run_tile<S, T, INL, H>(jobs, job, bj, tile, lds); break;
+        MDFT_BATCH_SHAPES(MDFT_CASE)
+#undef MDFT_CASE
     default: break;
     }
 }
@@ -192,26 +181,10 @@ template <int T, BatchHold H>
 __device__ __forceinline__ void run_job(const BatchJob& bj, int tile, float* lds)
 {
     switch (bj.shape) {
-    case 1: run_tile_body<1, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 2: run_tile_body<2, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 3: run_tile_body<3, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 4: run_tile_body<4, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 5: run_tile_body<5, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 6: run_tile_body<6, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 7: run_tile_body<7, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 8: run_tile_body<8, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 9: run_tile_body<9, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 10: run_tile_body<10, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 11: run_tile_body<11, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 12: run_tile_body<12, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case 13: run_tile_body<13, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case F3_BASE + 6: run_tile_body<F3_BASE + 6, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case F3_BASE + 7: run_tile_body<F3_BASE + 7, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case F3_BASE + 8: run_tile_body<F3_BASE + 8, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case F3_BASE + 9: run_tile_body<F3_BASE + 9, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case F3_BASE + 10: run_tile_body<F3_BASE + 10, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case F3_BASE + 11: run_tile_body<F3_BASE + 11, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
-    case GEN_SHAPE: run_tile_body<GEN_SHAPE, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+#define MDFT_CASE(S) \
+    case S: run_tile_body<S, T, H>(bj.job, bj.blue, bj.cols, tile, lds); break;
+        MDFT_BATCH_SHAPES(MDFT_CASE)
+#undef MDFT_CASE
     default: break;
     }
 }

@@ -786,7 +786,6 @@ struct FftPass {
     static constexpr int NB = C::EPT / R;
     static constexpr int NS = ns_of(S, P);
     static constexpr bool LAST = (P == C::NPASS - 1);
-    static constexpr int LST = C::template lstride<COLS>();
     static_assert(NB * R == C::EPT, "the radix divides the points per thread");
 
     using Regs = float2 (&)[C::L][C::EPT];  // the thread's lines

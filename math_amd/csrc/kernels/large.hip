@@ -189,8 +189,6 @@ __global__ __launch_bounds__(T) void k_large_step(LargeJob job)
         // the step's twiddle w_M^(tq*pos), tq*pos < M: n1*k2 (A), k2*j1 (B), M1*n2*k3 (A1),
         // kr*j1 (fused C), M1*k3*jr2 (X1)
         apply_twiddles<C>(v, job, tq, t);
-    } else if (job.store_mode == LARGE_STORE_DIAG) {
-        times_d();
     } else if (job.store_mode == LARGE_STORE_CONJ) {
 #pragma unroll
         for (int i = 0; i < C::EPT; ++i) v[i] = cscale(cxor(v[i], sgn), job.scale);

@@ -37,8 +37,8 @@ enum LargeLoad { LARGE_LOAD_PLAIN = 0, LARGE_LOAD_CONJ = 1, LARGE_LOAD_CHIRP = 2
 // LARGE_STORE_DIAG_FFT: conj(v * D) (natural index k2 + kmul*k1), a second FFT
 // of the same length, then the twiddle of LARGE_STORE_TWIDDLE (the middle of a
 // long Bluestein line in one step)
-enum LargeStore { LARGE_STORE_PLAIN = 0, LARGE_STORE_TWIDDLE = 1, LARGE_STORE_DIAG = 2, LARGE_STORE_CHIRP = 3,
-                  LARGE_STORE_CONJ = 4, LARGE_STORE_DIAG_FFT = 5 };
+enum LargeStore { LARGE_STORE_PLAIN = 0, LARGE_STORE_TWIDDLE = 1, LARGE_STORE_CHIRP = 2, LARGE_STORE_CONJ = 3,
+                  LARGE_STORE_DIAG_FFT = 4 };
 
 // One step of a long-line FFT: count sub-lines; sub-line L reads from
 // src + (L / sub_in) * ls_in + r * ls2_in with r = L % sub_in and element
@@ -59,7 +59,7 @@ struct LargeJob {
     int64_t count, lines;
     int load_mode, store_mode, inverse, pad;
     int64_t n, m1, m2;
-    int64_t kmul;  // natural index of the store modes DIAG, DIAG_FFT, CHIRP: q + kmul * pos
+    int64_t kmul;  // natural index of the store modes DIAG_FFT and CHIRP: q + kmul * pos
     // log2 of sub_in, sub2_in, sub_out, sub2_out, tmod, tdiv (all powers of two; -1: no second
     // split), filled in by launch_large_step
     float scale;
@@ -138,8 +138,10 @@ hipError_t launch_image_axis(int shape, const AxisJob& job, const ImageIO& io, b
 hipError_t launch_image_luminance(const ImageIO& io, float2* dst, int w, int h, hipStream_t stream);
 hipError_t launch_image_magnitude(const ImageIO& io, const float2* src, int w, int h, hipStream_t stream);
 
-// Workgroup size of batch column tiles: 2-16 columns per tile for padded
-// lengths 1024-4096 (wider contiguous runs per row), two workgroups per CU.
+// Workgroup size of a batch's whole images and row tiles (every batched line
+// fits), and of its column tiles where there are enough: 2-16 columns per tile
+// for padded lengths 1024-4096 (wider contiguous runs per row), two per CU.
+constexpr int BATCH_THREADS = 256;
 constexpr int BATCH_COL_THREADS = 512;
 
 // What the kernels of a workgroup size hold: any items, one line per thread
@@ -148,9 +150,9 @@ constexpr int BATCH_COL_THREADS = 512;
 enum BatchHold { BATCH_ALL = 0, BATCH_COLS_X2 = 1, BATCH_COLS = 2 };
 __host__ __device__ constexpr bool batch_holds(int threads, BatchHold hold)
 {
-    return hold == BATCH_ALL ? threads == 256 : threads == 512 || (threads == 1024 && hold == BATCH_COLS_X2);
+    return hold == BATCH_ALL ? threads == BATCH_THREADS : threads == 512 || (threads == 1024 && hold == BATCH_COLS_X2);
 }
-// batch kernels, padded lengths up to 8192 (an error where !batch_holds); the persistent shapes run in 256 threads
+// batch kernels, padded lengths up to 8192 (an error where !batch_holds); the persistent shapes run in BATCH_THREADS
 hipError_t launch_batch_grid(int threads, BatchHold hold, const BatchJob* jobs, const uint2* items, uint32_t nitems,
                              hipStream_t stream);
 hipError_t launch_batch_persistent(const BatchJob* jobs, const uint2* items, uint32_t nitems, uint32_t* ctl,
@@ -168,7 +170,7 @@ hipError_t warm_batch_grid(uint32_t* word, hipStream_t stream);
 template <int T>
 hipError_t warm_batch_persistent(uint32_t* word, hipStream_t stream);
 // a small image in one launch (whole.hip): its row and column tile in one workgroup
-constexpr int WHOLE_THREADS = 256;
+constexpr int WHOLE_THREADS = BATCH_THREADS;
 hipError_t launch_whole(const BatchJob& row, const BatchJob& col, hipStream_t stream);
 hipError_t warm_whole(uint32_t* word, hipStream_t stream);
 // lines of a shape one tile holds (0: the shape does not fit)
