@@ -125,6 +125,8 @@ struct Lane {
     char* table_dev = nullptr;
     char* table_host = nullptr;
     size_t cap_jobs = 0, cap_items = 0;
+    const BatchJob* jobs_dev() const { return reinterpret_cast<const BatchJob*>(table_dev); }
+    const uint2* items_dev() const { return reinterpret_cast<const uint2*>(table_dev + sizeof(BatchJob) * cap_jobs); }
 };
 
 }  // namespace
@@ -210,7 +212,7 @@ void grow(Lane& L, size_t njobs, size_t nitems)
 }
 
 // Launch one micro-batch on lane L (scheduler thread, lock not held).
-void launch_micro_batch(mdft_server_s* s, Lane& L, const std::vector<mdft::BatchEntry>& entries)
+mdft::BatchBuild launch_micro_batch(mdft_server_s* s, Lane& L, const std::vector<mdft::BatchEntry>& entries)
 {
     Context& ctx = Context::get(s->device);
     mdft::BatchBuild bb;
@@ -221,8 +223,8 @@ void launch_micro_batch(mdft_server_s* s, Lane& L, const std::vector<mdft::Batch
     uint2* items_host = reinterpret_cast<uint2*>(L.table_host + sizeof(BatchJob) * L.cap_jobs);
     std::copy(bb.jobs.begin(), bb.jobs.end(), jobs_host);
     std::copy(bb.items.begin(), bb.items.end(), items_host);
-    const BatchJob* jobs_dev = reinterpret_cast<const BatchJob*>(L.table_dev);
-    const uint2* items_dev = reinterpret_cast<const uint2*>(L.table_dev + sizeof(BatchJob) * L.cap_jobs);
+    const BatchJob* jobs_dev = L.jobs_dev();
+    const uint2* items_dev = L.items_dev();
     if (!bb.items.empty()) {
         // the used part: [0, jobs) and [cap_jobs, cap_jobs + items) as one span
         const size_t span = sizeof(BatchJob) * L.cap_jobs + sizeof(uint2) * bb.items.size();
@@ -241,12 +243,14 @@ void launch_micro_batch(mdft_server_s* s, Lane& L, const std::vector<mdft::Batch
                                             n - bb.nphase1, L.stream),
                     "serve launch");
     mdft::hip_check(hipEventRecord(L.done, L.stream), "event record");
+    return bb;
 }
 
-// One tiny micro-batch before traffic (a whole 16x16 image in phase 1's
-// 256-thread tiles, the 1000-point columns of a 2x1000 image in phase 2's
-// 512-thread tiles): the first launches of the batch kernels in a process
-// load their code and stalled the first requests of a stream by 17 ms.
+// One tiny micro-batch before traffic (a whole 16x16 image and a 2x1000 one),
+// whose column tile then runs in the larger column kernels as well, which few
+// columns do not reach by themselves: the first launches of the batch kernels
+// in a process load their code and stalled the first requests of a stream by
+// 17 ms.
 void warm_up(mdft_server_s* s)
 {
     const size_t need = sizeof(float2) * (16 * 16 + 2 * 1000);
@@ -254,7 +258,13 @@ void warm_up(mdft_server_s* s)
     float2* a = reinterpret_cast<float2*>(s->arena_mem);  // in place on arena contents, results unused
     const std::vector<mdft::BatchEntry> entries = {{16, 16, false, a, a}, {2, 1000, false, a + 256, a + 256}};
     Lane& L = s->lanes[0];
-    launch_micro_batch(s, L, entries);
+    const mdft::BatchBuild bb = launch_micro_batch(s, L, entries);
+    // an item holds in any kernel whose tiles are no narrower: tile 0 of two columns
+    const uint2* columns = L.items_dev() + bb.nphase1;
+    const uint32_t n = (uint32_t)bb.items.size() - bb.nphase1;
+    for (mdft::BatchHold hold : {mdft::BATCH_COLS, mdft::BATCH_COLS_X2})
+        mdft::hip_check(mdft::launch_batch_grid(mdft::BATCH_COL_THREADS, hold, L.jobs_dev(), columns, n, L.stream),
+                        "server warm-up");
     mdft::hip_check(hipStreamSynchronize(L.stream), "server warm-up");
 }
 
